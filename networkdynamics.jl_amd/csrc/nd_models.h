@@ -158,6 +158,23 @@ __device__ __forceinline__ S g_dst(S vs, S vd, const P* __restrict__ pe) {
     else return nan_of<S>();
 }
 
+// N sine edges at once (g_dst of each, the same operations): y[i] from vs[i], vd[i] and the
+// parameters pe[i], their sines evaluated together
+template <int EM, int N, int NP>
+__device__ __forceinline__ void g_dst_n(const double (&vs)[N], const double (&vd)[N], const double (&pe)[N][NP],
+                                        double (&y)[N]) {
+    static_assert(EM == ND_EM_KURAMOTO || EM == ND_EM_STATIC_LINE, "sine edges");
+    double x[N], s[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        if constexpr (EM == ND_EM_STATIC_LINE) x[i] = vs[i] - vd[i] - pe[i][1];
+        else x[i] = vs[i] - vd[i];
+    }
+    nd_sin_n<N>(x, s);
+#pragma unroll
+    for (int i = 0; i < N; ++i) y[i] = pe[i][0] * s[i];
+}
+
 template <typename S = double, typename P = double>
 __device__ __forceinline__ S g_dst_rt(int em, S vs, S vd, const P* __restrict__ pe) {
     switch (em) {

@@ -51,7 +51,12 @@ struct VDesc {            // one vertex batch as the kernels see it (0-based off
     const int32_t* lrp;   // hub-free destination lists: count+1 offsets into lslots
     const int2* lslots;
     const uint8_t* lseb;  // edge batch of each lslots entry (several edge batches only)
-    const int32_t* lnbr;  // with cached parameters instead of lslots: neighbour output index | (is_src << 31)
+    // with cached parameters instead of lslots: neighbour output index | (is_src << 31), and
+    // where lown is null the owner lane of the entry in bits 25..30
+    const int32_t* lnbr;
+    const uint8_t* lown;  // owner lane of every entry of the hub-free lists (its vertex's place in the wave)
+    const int4* wave;     // per wave of the low path: {first vertex, vertices, first entry, end of its entries}
+    int32_t nwave;
     const double* kfull;  // edge parameters per destination-list entry (rowptr order), or null
     const double* klow;   // the same for the hub-free lists (lrp order), or null
     // one-thread-per-vertex path (models with external inputs or time dependence, edge
@@ -245,6 +250,33 @@ __device__ __forceinline__ double slot_eval(int2 s, double nbr, const double* k,
     }
 }
 
+// N entries at once; sine edges evaluate their sines together
+template <int EM, int WRAP, int N, int NP>
+__device__ __forceinline__ void slot_eval_n(const int2 (&s)[N], const double (&nbr)[N], const double (&k)[N][NP],
+                                            const double (&own)[N], double (&v)[N]) {
+    if constexpr (EM == ND_EM_KURAMOTO && WRAP != ND_WRAP_SYMMETRIC) {
+        // K sin(nbr - own) on the dst side, -(K sin(own - nbr)) on the src side: the sine is odd
+        // bit for bit, so both are the same
+        double y[N];
+        g_dst_n<EM, N>(own, nbr, k, y);
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] = -y[i];
+    } else if constexpr (EM == ND_EM_KURAMOTO || EM == ND_EM_STATIC_LINE) {
+        double a[N], b[N], y[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            a[i] = (s[i].y & 1) ? own[i] : nbr[i];
+            b[i] = (s[i].y & 1) ? nbr[i] : own[i];
+        }
+        g_dst_n<EM, N>(a, b, k, y);
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] = ((s[i].y & 1) && WRAP != ND_WRAP_SYMMETRIC) ? -y[i] : y[i];
+    } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] = slot_eval<EM, WRAP>(s[i], nbr[i], k[i], own[i]);
+    }
+}
+
 constexpr int kUnroll = 4;   // entries whose loads are issued together per thread
 
 // Partial sum of the entries beg+t, beg+t+G, beg+t+2G, ... of one segment, in that
@@ -292,6 +324,7 @@ __device__ __forceinline__ double segment_sum(int32_t beg, int32_t end, int32_t 
 
 // Streamed reads of the low path (entry lists, parameter copy, own states and
 // parameters): nontemporal, so that they displace fewer neighbour outputs from L2
+constexpr int kOwnerShift = 25;    // of the owner lane in a packed entry
 constexpr bool kStreamNT = true;
 template <typename T>
 __device__ __forceinline__ T ld_stream(const T* p) {
@@ -300,18 +333,89 @@ __device__ __forceinline__ T ld_stream(const T* p) {
 }
 
 // LDS of the fused vertex kernels (each kernel that uses them gets its own copy): the
-// low path's per-wave entry windows (values, owners) and own outputs, the hub blocks'
-// wave partials (blocks of at most 256 threads)
+// low path's per-wave entry windows and own outputs, the hub blocks' wave partials (blocks
+// of at most 256 threads)
 __shared__ double rhs_val[4 * 256];
 __shared__ double rhs_own[256];
-__shared__ uint8_t rhs_owner[4 * 256];
 __shared__ double rhs_wpart[256 / kWave];
+
+// One window of a wave of the low path: the values of its cnt <= 64 * N entries from base on
+// go to wval, entry base + i evaluated by lane i % 64.  Entries past the window's end load its
+// last entry instead (a valid index), so the loads carry no branch and all go out before the
+// first wait.
+template <int EM, int WRAP, bool MULTI, bool KC, int N>
+__device__ __forceinline__ void low_window(const VDesc& vd, int32_t base, int32_t cnt, int32_t lane,
+                                           const EDesc* __restrict__ ed, const double* __restrict__ u,
+                                           const double* __restrict__ vo, const double* __restrict__ p,
+                                           const double* __restrict__ wown, double* __restrict__ wval) {
+    constexpr int NP = EModel<EM>::np, NPK = NP > 0 ? NP : 1;
+    int2 sl[N];
+    uint32_t ow[N];
+    double nb[N], kk[N][NPK], own[N], v[N];
+    if constexpr (KC) {
+        // all loads before the first use of one (a decode inside the loop, or behind the
+        // branch, would wait for each)
+        uint32_t w[N];
+#pragma unroll
+        for (int j = 0; j < N; ++j) w[j] = static_cast<uint32_t>(ld_stream(vd.lnbr + base + min(j * kWave + lane, cnt - 1)));
+        if (vd.lown) {
+#pragma unroll
+            for (int j = 0; j < N; ++j) ow[j] = ld_stream(vd.lown + base + min(j * kWave + lane, cnt - 1));
+        } else {
+#pragma unroll
+            for (int j = 0; j < N; ++j) ow[j] = w[j];
+        }
+        const uint32_t mask = vd.lown ? 0x7fffffffu : (1u << kOwnerShift) - 1;
+        const uint32_t shift = vd.lown ? 0u : static_cast<uint32_t>(kOwnerShift);
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            sl[j] = make_int2(static_cast<int32_t>(w[j] & mask), static_cast<int32_t>(w[j] >> 31));
+            ow[j] = (ow[j] >> shift) & (kWave - 1);
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            const int32_t s = base + min(j * kWave + lane, cnt - 1);
+            sl[j] = vd.lslots[s];
+            ow[j] = vd.lown[s];
+        }
+    }
+    if constexpr (!MULTI) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            const int32_t s = base + min(j * kWave + lane, cnt - 1);
+#pragma unroll
+            for (int c = 0; c < NP; ++c)
+                kk[j][c] = KC ? ld_stream(vd.klow + static_cast<int64_t>(s) * NP + c) : p[(sl[j].y >> 1) + c];
+        }
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            if constexpr (is_ode_model(EM)) nb[j] = u[sl[j].x];
+            else if constexpr (EM != ND_EM_NOOP) nb[j] = vo[sl[j].x];
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < N; ++j) own[j] = wown[ow[j]];
+    if constexpr (MULTI) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            const int32_t s = base + min(j * kWave + lane, cnt - 1);
+            v[j] = slot_value_rt(ed[vd.lseb[s]], sl[j], own[j], u, vo, p);
+        }
+    } else {
+        slot_eval_n<EM, WRAP, N, NPK>(sl, nb, kk, own, v);
+    }
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+        if (j * kWave + lane < cnt) wval[j * kWave + lane] = v[j];
+}
 
 // Fused RHS for one vertex batch.  Block layout (hubs first, so the longest
 // segments start earliest):
 //   [0, nbig)                 one block per big hub (segment > big_hub_degree),
 //   [nbig, nbig + nmidb)      one wave per mid hub (segment > hub_degree),
-//   [nbig + nmidb, ...)       one vertex per thread, segment summed in reference order.
+//   [nbig + nmidb, ...)       a wave per entry of the wave table: up to 64 consecutive
+//                             vertices, one per lane, segments summed in reference order.
 // Hub segments: per-thread partial sums in a fixed order, xor-butterfly per wave,
 // wave partials combined in wave order -- deterministic run to run.
 template <int VM, int EM, int WRAP, bool MULTI, bool STAGE, bool KC>
@@ -362,36 +466,37 @@ __device__ __forceinline__ void vertex_rhs_body(const VDesc& vd, int32_t b,
         }
         b -= nmidb;
     }
-    // Low-degree vertices: wave w of block b takes the 64 consecutive vertices
-    // q0..q0+63 and their hub-free destination lists lrp/lslots.  Entries are evaluated
-    // lane-densely in per-wave LDS windows of 4*64 (loads issued together, no lane idles
+    // Low-degree vertices: each wave takes the consecutive vertices of one entry of the wave
+    // table and their hub-free destination lists lrp/lslots.  Entries are evaluated
+    // lane-densely into a per-wave LDS window of 4*64 (loads issued together, no lane idles
     // on a neighbour's long segment); then each lane sums its own segment from LDS in
     // order, so the summation order is the reference's.  The waves of a block share no
     // data and synchronise only within themselves.
+    //
+    // The table gives every wave at most one window of entries (unless a single vertex has
+    // more) and, in a network too small to fill the chip with such waves, fewer: with 64
+    // vertices per wave throughout, the waves of a Barabasi-Albert graph's oldest vertices
+    // went through a dozen windows one after the other, and a network of 1000 vertices ran
+    // on 16 waves.  Swing vertices on Barabasi-Albert graphs: 22.8 -> 8.2 us per call at 100003
+    // vertices (the host's share of a call), 39.4 -> 22.2 us at 300001, 60.6 -> 60.3 us at 1e6.
     const int32_t lane = static_cast<int32_t>(threadIdx.x & (kWave - 1));
-    const int32_t wib = static_cast<int32_t>(threadIdx.x / kWave);
-    const int32_t q0 = (b * static_cast<int32_t>(blockDim.x / kWave) + wib) * kWave;
-    const int32_t q = q0 + lane;
-    if (q0 >= vd.count) return;
-    const bool valid = q < vd.count;
-    const int32_t qv = valid ? q : q0;             // a valid vertex for the loads of idle lanes
-    const int64_t x0 = static_cast<int64_t>(vd.state0) + static_cast<int64_t>(qv) * dim;
+    const int32_t wib = __builtin_amdgcn_readfirstlane(static_cast<int32_t>(threadIdx.x / kWave));
+    const int32_t w = b * static_cast<int32_t>(blockDim.x / kWave) + wib;
+    if (w >= vd.nwave) return;
+    const int4 wd = vd.wave[w];
+    const int32_t q0 = wd.x, nq = wd.y, S0 = wd.z, S1 = wd.w;
+    const bool valid = lane < nq;
+    const int32_t q = q0 + (valid ? lane : 0);     // a valid vertex for the loads of idle lanes
+    const int64_t x0 = static_cast<int64_t>(vd.state0) + static_cast<int64_t>(q) * dim;
     if constexpr (VM == ND_VM_NOOP) {
         if (valid) vertex_emit<VM, STAGE>(du, sa, x0, u + x0, 0.0, p, dim, vd.mask[0], static_cast<int64_t>(vd.out0) + q);
     } else {
-        const int32_t* __restrict__ lrp = vd.lrp;
         // lrp[q] = offset | (hub ? 1 << 31 : 0): hub vertices keep an empty segment here and
         // their du is written by the hub paths.  One offset load per lane: a segment ends
-        // where the next lane's begins, the wave's last one at lrp[q0 + 64].
+        // where the next lane's begins, the wave's last one at S1.
         constexpr int32_t kOff = 0x7fffffff;
-        const int32_t raw = lrp[valid ? q : vd.count];
-        const int32_t tail = lrp[min(q0 + kWave, vd.count)];
+        const int32_t raw = vd.lrp[q];
         const bool hub = raw < 0;
-        const int32_t sb = raw & kOff;
-        const int32_t nxt = __shfl_down(raw, 1, kWave);
-        const int32_t se = valid ? ((lane == kWave - 1 ? tail : nxt) & kOff) : sb;
-        const int32_t S0 = __shfl(sb, 0, kWave);
-        const int32_t S1 = tail & kOff;
         // own state and parameters are loaded up front, in parallel with the offsets
         constexpr int DC = VModel<VM>::dim > 0 ? VModel<VM>::dim : 1;
         constexpr int NPV = VPar<VM>::np > 0 ? VPar<VM>::np : 1;
@@ -400,61 +505,30 @@ __device__ __forceinline__ void vertex_rhs_body(const VDesc& vd, int32_t b,
         for (int j = 0; j < DC; ++j) xs[j] = ld_stream(u + x0 + j);
 #pragma unroll
         for (int j = 0; j < NPV; ++j)
-            pvs[j] = VPar<VM>::np > 0 ? ld_stream(p + vd.param0 + static_cast<int64_t>(qv) * vd.pdim + j) : 0.0;
+            pvs[j] = VPar<VM>::np > 0 ? ld_stream(p + vd.param0 + static_cast<int64_t>(q) * vd.pdim + j) : 0.0;
         const double own = (DC == 1 || vd.mask[0] == 0) ? xs[0] : xs[DC - 1];
         double* __restrict__ wval = rhs_val + wib * 4 * kWave;
-        uint8_t* __restrict__ wowner = rhs_owner + wib * 4 * kWave;
-        const double* __restrict__ wown = rhs_own + wib * kWave;
         rhs_own[threadIdx.x] = own;
+        wave_sync();
+        const double* __restrict__ wown = rhs_own + wib * kWave;
         double acc = 0.0;
         constexpr int32_t W = 4 * kWave;
         for (int32_t base = S0; base < S1; base += W) {
-            const int32_t wend = min(base + W, S1);
-            for (int32_t s2 = max(sb, base); s2 < min(se, wend); ++s2) wowner[s2 - base] = static_cast<uint8_t>(lane);
+            const int32_t cnt = min(W, S1 - base);
+            if (cnt <= kWave) low_window<EM, WRAP, MULTI, KC, 1>(vd, base, cnt, lane, ed, u, vo, p, wown, wval);
+            else low_window<EM, WRAP, MULTI, KC, 4>(vd, base, cnt, lane, ed, u, vo, p, wown, wval);
             wave_sync();
-            constexpr int NP = EModel<EM>::np;
-            int2 sl[4];
-            double nb[4];
-            double kk[4][NP > 0 ? NP : 1];
-            // entries past the window's end load its last entry instead (a valid index), so
-            // the loads carry no branch and all go out before the first wait
+            const int32_t sb = raw & kOff, nxt = __shfl_down(raw, 1, kWave) & kOff;
+            const int32_t se = lane < nq - 1 ? nxt : S1;
+            const int32_t s0 = max(sb, base) - base, s1 = valid ? min(se, base + cnt) - base : 0;
+            for (int32_t s = s0; s < s1; s += 4) {
+                double f[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int32_t s2c = min(base + j * kWave + lane, wend - 1);
-                if constexpr (KC) {
-                    const uint32_t w = static_cast<uint32_t>(ld_stream(vd.lnbr + s2c));
-                    sl[j] = make_int2(static_cast<int32_t>(w & 0x7fffffffu), static_cast<int32_t>(w >> 31));
-                } else {
-                    sl[j] = vd.lslots[s2c];
-                }
+                for (int j = 0; j < 4; ++j) f[j] = wval[min(s + j, s1 - 1)];
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (s + j < s1) acc += f[j];
             }
-            if constexpr (!MULTI) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int32_t s2c = min(base + j * kWave + lane, wend - 1);
-#pragma unroll
-                    for (int c = 0; c < NP; ++c)
-                        kk[j][c] = KC ? ld_stream(vd.klow + static_cast<int64_t>(s2c) * NP + c) : p[(sl[j].y >> 1) + c];
-                }
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    if constexpr (is_ode_model(EM)) nb[j] = u[sl[j].x];
-                    else if constexpr (EM != ND_EM_NOOP) nb[j] = vo[sl[j].x];
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int32_t s2 = base + j * kWave + lane;
-                if (s2 < wend) {
-                    const double ow = wown[wowner[s2 - base]];
-                    double v;
-                    if constexpr (MULTI) v = slot_value_rt(ed[vd.lseb[s2]], sl[j], ow, u, vo, p);
-                    else v = slot_eval<EM, WRAP>(sl[j], nb[j], kk[j], ow);
-                    wval[s2 - base] = v;
-                }
-            }
-            wave_sync();
-            for (int32_t s2 = max(sb, base); s2 < min(se, wend); ++s2) acc += wval[s2 - base];
             wave_sync();
         }
         if (valid && !hub) vertex_emit<VM, STAGE>(du, sa, x0, xs, acc, pvs, dim, vd.mask[0], static_cast<int64_t>(vd.out0) + q);
@@ -1808,6 +1882,8 @@ struct nd_plan {
     int2* d_lslots = nullptr;
     int32_t* d_lnbr = nullptr;
     uint8_t* d_lseb = nullptr;
+    uint8_t* d_lown = nullptr;
+    int4* d_wave = nullptr;
     int32_t n_agg_hub = 0;
     std::vector<size_t> hub_offset;
     // slot-ordered edge parameters (one feed-forward edge batch with parameters)
@@ -1879,6 +1955,14 @@ void release(nd_plan* pl, void* ptr) {
     if (it != pl->allocations.end()) { (void)hipFree(*it); pl->allocations.erase(it); }
 }
 
+// Entries per wave of the low path: one window of 4*64, fewer where that would leave the
+// network with less than kLowWaves waves (two per SIMD)
+constexpr int64_t kLowWaves = 2048;
+int32_t wave_entries(int64_t nlow) {
+    const int64_t c = (nlow / kLowWaves + kWave - 1) / kWave * kWave;
+    return static_cast<int32_t>(std::max<int64_t>(kWave, std::min<int64_t>(c, 4 * kWave)));
+}
+
 // Hub lists and the hub-free destination lists follow hub_degree / big_hub_degree;
 // rebuilt when they change.  Per vertex batch: big hubs then mid hubs, each by
 // decreasing segment length; every other vertex keeps its segment in lrp/lslots.
@@ -1888,6 +1972,17 @@ int rebuild_hubs(nd_plan* pl) {
     std::vector<int2> lslots;
     std::vector<int32_t> lnbr;       // compact form of lslots when the parameters are cached
     size_t nlow = 0;
+    std::vector<uint8_t> lown;       // owner lane per entry
+    std::vector<int4> waves;
+    std::vector<size_t> wave_offset(pl->vdesc.size(), 0);
+    int64_t total_low = 0;
+    for (const VDesc& vd : pl->vdesc)
+        if (vd.model != ND_VM_NOOP && vd.depth == 1)
+            for (int32_t q = 0; q < vd.count; ++q) {
+                const int32_t len = pl->rowptr_host[vd.row0 + q + 1] - pl->rowptr_host[vd.row0 + q];
+                total_low += len > H ? 0 : len;
+            }
+    const int32_t cap = wave_entries(total_low);
     std::vector<uint8_t> lseb;
     std::vector<size_t> lrp_offset(pl->vdesc.size(), 0);
     pl->hub_offset.assign(pl->vdesc.size() + 1, 0);
@@ -1903,11 +1998,18 @@ int rebuild_hubs(nd_plan* pl) {
         lrp_offset[b] = lrp.size();
         std::vector<std::pair<int32_t, int32_t>> big, mid;   // (-length, q)
         const bool functional = vd.model != ND_VM_NOOP && vd.depth == 1;
+        wave_offset[b] = waves.size();
         for (int32_t q = 0; q < vd.count; ++q) {
             lrp.push_back(static_cast<int32_t>(nlow));
-            if (!functional) continue;
             const int32_t r = vd.row0 + q;
-            const int32_t beg = pl->rowptr_host[r], len = pl->rowptr_host[r + 1] - beg;
+            const int32_t beg = functional ? pl->rowptr_host[r] : 0, len = functional ? pl->rowptr_host[r + 1] - beg : 0;
+            const int32_t low = len > H ? 0 : len;
+            if (waves.size() == wave_offset[b] || waves.back().y == kWave ||
+                (waves.back().w > waves.back().z && waves.back().w - waves.back().z + low > cap))
+                waves.push_back(make_int4(q, 0, static_cast<int32_t>(nlow), static_cast<int32_t>(nlow)));
+            const int32_t owner = waves.back().y++;
+            waves.back().w += low;
+            if (!functional) continue;
             if (len > H) lrp.back() = static_cast<int32_t>(static_cast<uint32_t>(lrp.back()) | 0x80000000u);
             if (len > HB) big.emplace_back(-len, q);
             else if (len > H) mid.emplace_back(-len, q);
@@ -1923,11 +2025,13 @@ int rebuild_hubs(nd_plan* pl) {
                     } else {
                         lslots.push_back(pl->slots_host[k]);
                     }
+                    lown.push_back(static_cast<uint8_t>(owner));
                     ++nlow;
                     if (pl->multi) lseb.push_back(pl->slot_eb_host[k]);
                 }
         }
         lrp.push_back(static_cast<int32_t>(nlow));
+        vd.nwave = static_cast<int32_t>(waves.size() - wave_offset[b]);
         std::sort(big.begin(), big.end());
         std::sort(mid.begin(), mid.end());
         for (auto& x : big) all.push_back(x.second);
@@ -1947,6 +2051,16 @@ int rebuild_hubs(nd_plan* pl) {
     release(pl, pl->d_lnbr);
     pl->d_lnbr = nullptr;
     release(pl, pl->d_lseb);
+    release(pl, pl->d_lown);
+    release(pl, pl->d_wave);
+    pl->d_lown = nullptr;
+    pl->d_wave = nullptr;
+    // the owner lanes go into the packed entries where the output indices leave room
+    const bool packed = pl->kcache && pl->vout_len <= (size_t(1) << kOwnerShift);
+    if (packed) {
+        for (size_t k = 0; k < lnbr.size(); ++k) lnbr[k] |= static_cast<int32_t>(lown[k]) << kOwnerShift;
+        lown.clear();
+    }
     pl->d_hubs_all = nullptr;
     pl->d_agg_hub_rows = nullptr;
     pl->d_lrp = nullptr;
@@ -1958,6 +2072,8 @@ int rebuild_hubs(nd_plan* pl) {
     rc = rc ? rc : upload(pl, lslots, &pl->d_lslots);
     rc = rc ? rc : upload(pl, lnbr, &pl->d_lnbr);
     rc = rc ? rc : upload(pl, lseb, &pl->d_lseb);
+    rc = rc ? rc : upload(pl, lown, &pl->d_lown);
+    rc = rc ? rc : upload(pl, waves, &pl->d_wave);
     if (rc) return rc;
     if (pl->kcache) {
         // the cached copy and both slot layouts restart from one NaN pattern, so they agree
@@ -1981,6 +2097,8 @@ int rebuild_hubs(nd_plan* pl) {
         pl->vdesc[b].lslots = pl->d_lslots;
         pl->vdesc[b].lnbr = pl->d_lnbr;
         pl->vdesc[b].lseb = pl->d_lseb;
+        pl->vdesc[b].lown = pl->d_lown;
+        pl->vdesc[b].wave = pl->d_wave ? pl->d_wave + wave_offset[b] : nullptr;
         pl->vdesc[b].kfull = pl->d_kfull;
         pl->vdesc[b].klow = pl->d_klow;
     }
@@ -2119,7 +2237,9 @@ void launch_rhs(nd_plan* pl, bool stage, double* du, const double* u, const doub
         VDesc vd = pl->vdesc[b];
         if (vd.count == 0) continue;
         vd.t = t;
-        const int64_t nblocks = vd.nbig + blocks_for(static_cast<int64_t>(vd.nmid) * kWave, B) + blocks_for(vd.count, B);
+        const bool fused = !vd.generic && vd.depth <= 1;
+        const int64_t nblocks = vd.nbig + blocks_for(static_cast<int64_t>(vd.nmid) * kWave, B) +
+                                (fused ? blocks_for(static_cast<int64_t>(vd.nwave) * kWave, B) : blocks_for(vd.count, B));
         if (vd.generic || !pl->gkern) {
             single(b, vd, nblocks);
             continue;
