@@ -4,12 +4,19 @@
 // Per instance everything a stage touches is on-chip:
 //   registers  per-vertex state y and the Runge-Kutta stage derivatives (up to V
 //              vertices per thread);
-//   LDS        stage vertex outputs theta[n], edge parameters, the destination
-//              lists (neighbour | role bit, edge index) and their chunking.
-// A stage: write theta, barrier, evaluate chunks (<= kChunk entries of one vertex's
-// destination list each, so hubs are split over threads), barrier, each vertex sums
-// its chunk partials in order and applies its model.  Vertices whose list fits one
-// chunk are summed in the reference order (increasing output index).
+//   LDS        stage vertex outputs theta[n], edge parameters, the edge outputs in row order
+//              (each vertex's entries consecutive, in whole pairs) and the edge table.
+// A stage: write theta, barrier; evaluate each edge once, four consecutive ones per thread,
+// and store its output at both endpoints' places in their rows, barrier; each vertex sums its
+// row in the reference order (increasing output index), kChunk entries at a time, and applies
+// its model.  Rows longer than kRowMax are summed by chunks spread over the block first.
+//
+// What bounds it: vector instruction issue.  One network of 1000 vertices and 4000 edges
+// (first-order Kuramoto, RK4, 16 waves of one CU) takes 2.47 us per evaluation with the vector
+// units 67 % busy and the LDS 60 %; with an index list per row entry, a bound on every entry
+// and the longer sine it took 3.61 us.  1024 swing networks of 100 to 2000 vertices (Tsit5 to
+// t = 10, default classes) take 38.4 ms, against 69.0 ms; at four vertices per thread the
+// vector units are 60 % busy with two waves per SIMD.
 //
 // Methods: Tsit5 (Tsitouras 2011) with the PI step-size controller of
 // OrdinaryDiffEq (beta1 = 7/50, beta2 = 2/25, qmin = 1/5, qmax = 10, gamma = 9/10,
@@ -24,6 +31,7 @@
 #include <new>
 #include <vector>
 
+#include "nd_block.h"
 #include "nd_internal.h"
 #include "nd_models.h"
 
@@ -31,22 +39,41 @@ namespace {
 
 using namespace nd;
 constexpr int kWave = 64;
-constexpr int kChunk = 8;          // destination-list entries per chunk
+constexpr int kChunk = 8;          // destination-list entries summed together
+constexpr int kRowMax = 16;        // longest row one thread sums by itself
+constexpr uint32_t kRowHub = 0x80000000u;
+constexpr int kSideStreams = 3;    // with the caller's stream, as many as a process has hardware queues
+// Consecutive edges one thread evaluates together (their LDS reads and sines overlap, and
+// table records and parameters are read 16 bytes at a time); the table is padded to a
+// multiple of this with edges of no effect, so no lane of a batch needs a bound
+constexpr int kEdgeBatch = 4;
+// after an instance's row pairs: pairs that stay zero (read past a row's end) and one that the
+// padding edges write to
+constexpr int kZeroPairs = kRowMax / 2, kDumpPairs = 1;
+__host__ __device__ constexpr int pad_edges(int ne) { return (ne + kEdgeBatch - 1) & ~(kEdgeBatch - 1); }
+__host__ __device__ constexpr int pad2(int n) { return (n + 1) & ~1; }
+
+// LDS of the crossing location: a second phase buffer and three bytes per edge, whole 16 bytes
+__host__ __device__ constexpr int32_t locate_bytes(int32_t n, int32_t ne) { return (8 * n + 3 * ne + 15) & ~15; }
 
 struct InstDesc {
-    int32_t n, ne, nslot, nchunk;
-    int64_t uoff, poff, soff, csoff, cvoff, cpoff;
-    int32_t lds_bytes, cls;
+    int32_t n, ne, nhc;           // vertices, edges, chunks of the rows longer than kRowMax
+    int32_t npair;                // pairs of row entries, without the zeros and the dump
+    int64_t uoff, poff, eoff, toff, voff, hoff;   // eoff: edges before this instance, toff: table records
+    int32_t lds_bytes, tab_bytes; // dynamic LDS without the tables, and the tables'
+    int32_t limit_bytes;          // the figure an instance's size is limited by (nd_ensemble_create)
+    int32_t cls, vper;
 };
 
 struct SolveArgs {
     const InstDesc* inst;
     const int32_t* order;
-    const uint16_t* ends;         // per edge: local src, local dst (2 per edge, offset soff)
-    const uint16_t* slot_e;       // local edge index | 0x8000 if this vertex is the edge's src
-    const uint16_t* cs;           // chunk starts (nchunk + 1 per instance)
-    const uint16_t* cv;           // chunk vertex
-    const uint16_t* cptr;         // vertex -> chunk range (n + 1 per instance)
+    const uint2* tab;             // per edge, padded to a multiple of kEdgeBatch per instance: {src | dst << 16, row
+                                  // position of the src entry | of the dst entry << 16}; src and dst in bytes of theta
+    const uint32_t* row;          // per vertex: first pair of entries | pairs << 16, or for a row longer than kRowMax
+                                  // kRowHub | first chunk | chunks << 16
+    const uint32_t* hc;           // per chunk of the long rows: first pair of entries | pairs << 16
+    int32_t lds_max;              // tab and hc go to LDS where they fit as well
     double* u;
     double* p;                    // written only where a line trips (line_limit set)
     const double* limit;          // per edge (instance order), or null: no line tripping
@@ -61,31 +88,93 @@ struct SolveArgs {
 };
 
 
-__device__ __forceinline__ double block_sum(double v, double* red) {
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
-    const int t = static_cast<int>(threadIdx.x), nw = static_cast<int>(blockDim.x) / kWave;
-    if ((t & (kWave - 1)) == 0) red[t / kWave] = v;
-    __syncthreads();
-    if (t == 0) {
-        double s = red[0];
-        for (int w = 1; w < nw; ++w) s += red[w];
-        red[16] = s;
-    }
-    __syncthreads();
-    const double r = red[16];
-    __syncthreads();
-    return r;
-}
-
+// Dynamic LDS in this order (16-byte alignment up to the edge table): the vertex outputs, the
+// edge outputs in row order, the edge parameters, the reduction buffers, the crossing
+// location's arrays, the edge table (tab_lds), the long rows' chunk sums and chunks (tab_lds).
 struct Lds {
     double* theta;
-    double* epar;
-    double* fval;                 // dst-side output of each edge at the current stage
-    double* partial;
-    double* red;
-    uint16_t *ends, *eidx, *cs, *cv, *cptr;
+    double* fslot;                // edge outputs in row order: each vertex's entries are consecutive, in whole pairs
+    double* epar;                 // padded with zeros to pad_edges
+    BlockRed red;
+    const uint2* tab;             // edge table in LDS, or
+    const uint2* tab_g;           // in memory
+    double* partial;              // sums of the long rows' chunks
+    const uint32_t* hc;           // those chunks in LDS, or
+    const uint32_t* hc_g;         // in memory
+    uint32_t zero_pair;           // first of the pairs that stay zero
+    bool tab_lds;                 // the tables are in LDS
 };
+
+// loads from the LDS or the memory copy of a table.  The typed pointers keep the two apart
+// (a select of generic pointers would make both of them flat loads)
+template <typename T>
+__device__ __forceinline__ T table_load(bool lds, const void* l, const void* g, int i) {
+    typedef const __attribute__((address_space(3))) T lds_t;
+    typedef const __attribute__((address_space(1))) T mem_t;
+    T r;
+    if (lds) r = ((lds_t*)l)[i];
+    else r = ((mem_t*)g)[i];
+    return r;
+}
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// the table records of the N consecutive edges from e (a multiple of N)
+template <int N>
+__device__ __forceinline__ void edge_recs(const Lds& L, int e, uint2 (&rec)[N]) {
+    static_assert(N % 2 == 0, "records in pairs");
+#pragma unroll
+    for (int i = 0; i < N / 2; ++i) {
+        const u32x4 r = table_load<u32x4>(L.tab_lds, L.tab, L.tab_g, e / 2 + i);
+        rec[2 * i] = make_uint2(r.x, r.y);
+        rec[2 * i + 1] = make_uint2(r.z, r.w);
+    }
+}
+__device__ __forceinline__ uint2 edge_rec(const Lds& L, int e) {
+    const u32x2 r = table_load<u32x2>(L.tab_lds, L.tab, L.tab_g, e);
+    return make_uint2(r.x, r.y);
+}
+__device__ __forceinline__ double theta_at(const double* th, uint32_t bytes) {
+    return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(th) + bytes);
+}
+
+// The same value, opaque to the optimiser (FRESH): what is derived from it is computed where it is
+// used.  Otherwise every address derived from a thread's rows and index is kept in registers
+// across the whole integration and spilled (100 registers at four vertices per thread)
+template <bool FRESH, typename T>
+__device__ __forceinline__ T fresh(T x) {
+    if constexpr (FRESH) asm volatile("" : "+v"(x));
+    return x;
+}
+// where registers are short; elsewhere keeping the addresses is 5 % faster
+template <int V, int LB>
+constexpr bool kFresh = V >= 3 || (V == 2 && LB > 512);
+
+// the step controller's powers, out of line: inlined, their polynomial's constants occupy
+// registers across the whole integration
+__device__ __noinline__ double step_pow(double x, double y) { return pow(x, y); }
+// x^a and y^b in one evaluation, on the even and the odd lanes of the wave
+__device__ __forceinline__ void step_pow2(double x, double a, double y, double b, double& xa, double& yb) {
+    const bool odd = threadIdx.x & 1;
+    const double r = step_pow(odd ? y : x, odd ? b : a);
+    xa = uniform_f64(r);
+    yb = uniform_f64(dpp_f64<0xb1>(r));       // lane 0 reads lane 1
+}
+
+// A swing vertex multiplies by 1.0 / M: the quotient is formed once per solve (the same bits),
+// kept in a register and passed in M's place
+template <int VM>
+constexpr bool kInverse0 = VM == ND_VM_SWING;
+template <int VM>
+__device__ __forceinline__ void vertex_f_inv(double* dx, const double* x, double acc, const double* pv) {
+    if constexpr (kInverse0<VM>) {
+        const double w = x[1];
+        dx[0] = w;
+        dx[1] = pv[0] * (pv[2] - pv[1] * w + acc);
+    } else {
+        vertex_f<VM>(dx, x, acc, pv, VModel<VM>::dim);
+    }
+}
 
 // Vertex parameters stay in registers for the whole solve up to three vertices per
 // thread; at four they are read from memory (L1/L2-resident) in each vertex update, which
@@ -93,88 +182,189 @@ struct Lds {
 template <int V>
 constexpr bool kParamsInMemory = V >= 4;
 
-// out = f(ys) for the thread's vertices (three block barriers): each edge's output is
-// evaluated once (the src side takes it negated, AntiSymmetric), then every chunk sums
-// its entries in list order.  pv: the vertex parameters in registers, or pg: the
-// instance's vertex parameters in memory (kParamsInMemory)
-template <int VM, int EM, int V>
-__device__ __forceinline__ void rhs(const InstDesc& I, const Lds& L, const double (&ys)[V][VModel<VM>::dim],
-                                    const double (&pv)[V][VPar<VM>::np > 0 ? VPar<VM>::np : 1],
-                                    const double* __restrict__ pg, double (&out)[V][VModel<VM>::dim]) {
-    constexpr int D = VModel<VM>::dim;
-    constexpr int NPE = EModel<EM>::np;
-    const int T = static_cast<int>(blockDim.x), t = static_cast<int>(threadIdx.x);
+// fslot = the outputs of every edge at the state ys in row order, the src side negated
+// (AntiSymmetric).  Two block barriers: after the vertex outputs and after the edges.  The
+// first batch's table records and parameters do not depend on the state and are read before
+// the first barrier.
+template <int VM, int EM, int V, bool FRESH>
+__device__ __forceinline__ void edge_flows(const InstDesc& I, const Lds& L, const double (&ys)[V][VModel<VM>::dim]) {
+    constexpr int N = kEdgeBatch, NP = EModel<EM>::np;
+    const int T = static_cast<int>(blockDim.x);
+    const int t = fresh<FRESH>(static_cast<int>(threadIdx.x));
+    uint2 rec[N];
+    double pe[N][NP];
+    auto load = [&](int e) {
+        edge_recs<N>(L, e, rec);
+        const double2* ep = reinterpret_cast<const double2*>(L.epar + e * NP);
+#pragma unroll
+        for (int i = 0; i < N * NP; i += 2) {
+            const double2 x = ep[i / 2];
+            pe[i / NP][i % NP] = x.x;
+            pe[(i + 1) / NP][(i + 1) % NP] = x.y;
+        }
+    };
+    const int ne = pad_edges(I.ne);
+    int e = N * t;
+    if (e < ne) load(e);
 #pragma unroll
     for (int k = 0; k < V; ++k) {
         const int v = t + k * T;
         if (v < I.n) L.theta[v] = ys[k][0];
     }
     __syncthreads();
-    for (int e = t; e < I.ne; e += T)
-        L.fval[e] = g_dst<EM>(L.theta[L.ends[2 * e]], L.theta[L.ends[2 * e + 1]], L.epar + e * (NPE > 0 ? NPE : 1));
-    __syncthreads();
-    for (int c = t; c < I.nchunk; c += T) {
-        double acc = 0.0;
-        const int s1 = L.cs[c + 1];
-        for (int s = L.cs[c]; s < s1; ++s) {
-            const int se = L.eidx[s];
-            const double f = L.fval[se & 0x7fff];
-            acc += (se & 0x8000) ? -f : f;
+    while (e < ne) {
+        double vs[N], vd[N], y[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            vs[i] = theta_at(L.theta, rec[i].x & 0xffff);
+            vd[i] = theta_at(L.theta, rec[i].x >> 16);
         }
-        L.partial[c] = acc;
+        g_dst_n<EM, N>(vs, vd, pe, y);
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            L.fslot[rec[i].y & 0xffff] = -y[i];
+            L.fslot[rec[i].y >> 16] = y[i];
+        }
+        e += N * T;
+        if (e < ne) load(e);
     }
     __syncthreads();
+}
+
+// the entries of pairs first .. first + N - 1 of a row; pairs past its end are the zeros (an
+// address select in place of a bound on every entry)
+template <int N>
+__device__ __forceinline__ void row_read(const Lds& L, uint32_t start, int np, int first, double2 (&f)[N]) {
+    const double2* fs = reinterpret_cast<const double2*>(L.fslot);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const double2* base = fs + (first + i < np ? start : L.zero_pair);
+        f[i] = base[first + i];
+    }
+}
+template <int N>
+__device__ __forceinline__ void row_add(const double2 (&f)[N], double& part) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        part += f[i].x;
+        part += f[i].y;
+    }
+}
+
+// out = f(ys) for the thread's vertices: each edge is evaluated once, then every vertex sums
+// its own row in list order, kChunk entries at a time.  Rows longer than kRowMax (hubs) are
+// summed by chunks spread over the block first, which takes a third barrier.  row: the
+// thread's row words; pv: the vertex parameters in registers, or pg: the instance's vertex
+// parameters in memory (kParamsInMemory)
+template <int VM, int EM, int V, bool FRESH>
+__device__ __forceinline__ void rhs(const InstDesc& I, const Lds& L, const double (&ys)[V][VModel<VM>::dim],
+                                    const double (&pv)[V][VPar<VM>::np > 0 ? VPar<VM>::np : 1],
+                                    const double* __restrict__ pg, const uint32_t (&row_)[V],
+                                    double (&out)[V][VModel<VM>::dim]) {
+    const int T = static_cast<int>(blockDim.x);
+    edge_flows<VM, EM, V, FRESH>(I, L, ys);
+    const int t = fresh<FRESH>(static_cast<int>(threadIdx.x));
+    uint32_t row[V];
+#pragma unroll
+    for (int k = 0; k < V; ++k) row[k] = fresh<FRESH>(row_[k]);
+    // parameters in memory: on their way while the rows are summed (read where they are used,
+    // one vertex after the other, they cost four memory latencies per evaluation)
+    constexpr int NPV = VPar<VM>::np > 0 ? VPar<VM>::np : 1;
+    double pm[kParamsInMemory<V> ? V : 1][NPV];
+    if constexpr (kParamsInMemory<V>) {
+#pragma unroll
+        for (int k = 0; k < V; ++k)
+#pragma unroll
+            for (int j = 0; j < VPar<VM>::np; ++j)
+                pm[k][j] = kInverse0<VM> && j == 0 ? pv[k][0]
+                                                   : pg[static_cast<int64_t>(min(t + k * T, I.n - 1)) * VPar<VM>::np + j];
+    }
+    constexpr int CP = kChunk / 2;
+    for (int c = t; c < I.nhc; c += T) {
+        const uint32_t h = table_load<uint32_t>(L.tab_lds, L.hc, L.hc_g, c);
+        double2 f[CP];
+        double part = 0.0;
+        row_read<CP>(L, h & 0xffff, static_cast<int>(h >> 16), 0, f);
+        row_add<CP>(f, part);
+        L.partial[c] = part;
+    }
+    double acc[V];
+    {
+        double2 f[V][2];
+#pragma unroll
+        for (int k = 0; k < V; ++k)
+            row_read<2>(L, row[k] & 0xffff, (row[k] & kRowHub) ? 0 : static_cast<int>(row[k] >> 16), 0, f[k]);
+#pragma unroll
+        for (int k = 0; k < V; ++k) {
+            const int np = (row[k] & kRowHub) ? 0 : static_cast<int>(row[k] >> 16);
+            double part = 0.0;
+            acc[k] = 0.0;
+            row_add<2>(f[k], part);
+            if (__any(np > 2)) {
+                double2 g[2];
+                row_read<2>(L, row[k] & 0xffff, np, 2, g);
+                row_add<2>(g, part);
+                if (__any(np > CP)) {
+                    acc[k] += part;
+                    part = 0.0;
+                    double2 h[CP];
+                    row_read<CP>(L, row[k] & 0xffff, np, CP, h);
+                    row_add<CP>(h, part);
+                }
+            }
+            acc[k] += part;
+        }
+    }
+    if (I.nhc > 0) {
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < V; ++k)
+            if (row[k] & kRowHub) {
+                const int c0 = row[k] & 0xffff, nc = static_cast<int>((row[k] & ~kRowHub) >> 16);
+                double a = 0.0;
+                for (int c = 0; c < nc; c += 4) {
+                    double f[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) f[j] = L.partial[c0 + min(c + j, nc - 1)];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        if (c + j < nc) a += f[j];
+                }
+                acc[k] = a;
+            }
+    }
 #pragma unroll
     for (int k = 0; k < V; ++k) {
         const int v = t + k * T;
         if (v < I.n) {
-            double acc = 0.0;
-            const int c1 = L.cptr[v + 1];
-            for (int c = L.cptr[v]; c < c1; ++c) acc += L.partial[c];
             if constexpr (kParamsInMemory<V>)
-                vertex_f<VM>(out[k], ys[k], acc, pg + static_cast<int64_t>(v) * VPar<VM>::np, D);
+                vertex_f_inv<VM>(out[k], ys[k], acc[k], pm[k]);
             else
-                vertex_f<VM>(out[k], ys[k], acc, pv[k], D);
+                vertex_f_inv<VM>(out[k], ys[k], acc[k], pv[k]);
         }
     }
 }
 
-// fval[e] = dst-side output of every edge at the state ys (one block barrier pair)
-template <int VM, int EM, int V>
-__device__ __forceinline__ void edge_flows(const InstDesc& I, const Lds& L, const double (&ys)[V][VModel<VM>::dim]) {
-    constexpr int NPE = EModel<EM>::np;
-    const int T = static_cast<int>(blockDim.x), t = static_cast<int>(threadIdx.x);
-#pragma unroll
-    for (int k = 0; k < V; ++k) {
-        const int v = t + k * T;
-        if (v < I.n) L.theta[v] = ys[k][0];
-    }
-    __syncthreads();
-    for (int e = t; e < I.ne; e += T)
-        L.fval[e] = g_dst<EM>(L.theta[L.ends[2 * e]], L.theta[L.ends[2 * e + 1]], L.epar + e * (NPE > 0 ? NPE : 1));
-    __syncthreads();
-}
-
 // Line tripping (the component callback of the reference's cascading-failure example,
 // docs/examples/cascading_failure.jl: condition |P_line| - limit, affect K = 0), checked
-// at the end of every accepted step on the flows in fval: a line whose |flow| exceeds
+// at the end of every accepted step on the flows in fslot: a line whose |flow| exceeds
 // its limit gets its first parameter set to 0, in LDS and in p.  Returns the number of
 // lines tripped in this check (block-uniform).
 template <int VM, int EM>
-__device__ __forceinline__ int trip_lines(const SolveArgs& a, const InstDesc& I, const Lds& L) {
+__device__ __forceinline__ int trip_lines(const SolveArgs& a, const InstDesc& I, Lds& L) {
     constexpr int NPE = EModel<EM>::np > 0 ? EModel<EM>::np : 1;
     const int T = static_cast<int>(blockDim.x), t = static_cast<int>(threadIdx.x);
-    const double* lim = a.limit + I.soff / 2;
+    const double* lim = a.limit + I.eoff;
     double* pe_g = a.p + I.poff + static_cast<int64_t>(I.n) * VPar<VM>::np;
     double cnt = 0.0;
     for (int e = t; e < I.ne; e += T) {
-        if (L.epar[e * NPE] != 0.0 && fabs(L.fval[e]) > lim[e]) {
+        if (L.epar[e * NPE] != 0.0 && fabs(L.fslot[edge_rec(L, e).y >> 16]) > lim[e]) {
             L.epar[e * NPE] = 0.0;
             pe_g[static_cast<int64_t>(e) * NPE] = 0.0;
             cnt += 1.0;
         }
     }
-    return static_cast<int>(block_sum(cnt, L.red));
+    return static_cast<int>(L.red.sum(cnt));
 }
 
 // The preset-time trip of one edge (PresetTimeComponentCallback with the same affect):
@@ -196,7 +386,7 @@ __device__ __forceinline__ int trip_edge(const SolveArgs& a, const InstDesc& I, 
 // Steady-state test after an accepted step (the allDerivPass test of DiffEqCallbacks'
 // TerminateSteadyState): every |du_i| <= ss_abstol or <= ss_reltol*|u_i|.  Block-uniform.
 template <int V, int D>
-__device__ __forceinline__ bool at_steady_state(const SolveArgs& a, const InstDesc& I, const Lds& L,
+__device__ __forceinline__ bool at_steady_state(const SolveArgs& a, const InstDesc& I, Lds& L,
                                                 const double (&y)[V][D], const double (&du)[V][D]) {
     const int T = static_cast<int>(blockDim.x), t = static_cast<int>(threadIdx.x);
     double fail = 0.0;
@@ -208,7 +398,7 @@ __device__ __forceinline__ bool at_steady_state(const SolveArgs& a, const InstDe
                 const double d = fabs(du[q][j]);
                 if (!(d <= a.ss_abstol || d <= a.ss_reltol * fabs(y[q][j]))) fail = 1.0;
             }
-    return block_sum(fail, L.red) == 0.0;
+    return L.red.sum(fail) == 0.0;
 }
 
 // Line crossings (ND_LINES_CROSSING).  sign8 codes the sign of a condition value (2 for
@@ -227,7 +417,8 @@ __device__ __forceinline__ bool crossed(int8_t p, int8_t n) {
 template <int EM>
 __device__ __forceinline__ double line_cond(const Lds& L, const double* th, const double* lim, int e) {
     constexpr int NPE = EModel<EM>::np > 0 ? EModel<EM>::np : 1;
-    return fabs(g_dst<EM>(th[L.ends[2 * e]], th[L.ends[2 * e + 1]], L.epar + e * NPE)) - lim[e];
+    const uint32_t ends = edge_rec(L, e).x;
+    return fabs(g_dst<EM>(theta_at(th, ends & 0xffff), theta_at(th, ends >> 16), L.epar + e * NPE)) - lim[e];
 }
 
 // sg[e] = sign8 of every edge's condition at the state y (two block barriers)
@@ -243,23 +434,6 @@ __device__ __forceinline__ void line_signs(const InstDesc& I, const Lds& L, cons
     __syncthreads();
     for (int e = t; e < I.ne; e += T) sg[e] = sign8(line_cond<EM>(L, L.theta, lim, e));
     __syncthreads();
-}
-
-__device__ __forceinline__ double block_min(double v, double* red) {
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) v = fmin(v, __shfl_xor(v, off, kWave));
-    const int t = static_cast<int>(threadIdx.x), nw = static_cast<int>(blockDim.x) / kWave;
-    if ((t & (kWave - 1)) == 0) red[t / kWave] = v;
-    __syncthreads();
-    if (t == 0) {
-        double s = red[0];
-        for (int w = 1; w < nw; ++w) s = fmin(s, red[w]);
-        red[16] = s;
-    }
-    __syncthreads();
-    const double r = red[16];
-    __syncthreads();
-    return r;
 }
 
 // Tsitouras (2011) 5(4) coefficients: stage matrix a (row s = stage s+1), error weights
@@ -317,46 +491,51 @@ __device__ __forceinline__ double dense_at(double y0, double k1, double d2, doub
 }
 
 template <int VM, int EM, int METHOD, int V, int LB>
-__global__ void __launch_bounds__(LB) k_ensemble(SolveArgs a) {
+__device__ __forceinline__ void ensemble_body(const SolveArgs& a, int inst, const InstDesc& I, double2* smem) {
     constexpr int D = VModel<VM>::dim;
     constexpr int NPV = VPar<VM>::np > 0 ? VPar<VM>::np : 1;
     constexpr int NPE = EModel<EM>::np;
     const int T = static_cast<int>(blockDim.x), t = static_cast<int>(threadIdx.x);
-    const int inst = a.order[a.first + static_cast<int>(blockIdx.x)];
-    const InstDesc I = a.inst[inst];
-    extern __shared__ double smem[];
+    const int ne4 = pad_edges(I.ne);
     Lds L;
-    L.theta = smem;
-    L.epar = L.theta + I.n;
-    L.fval = L.epar + I.ne * NPE;
-    L.partial = L.fval + I.ne;
-    L.red = L.partial + I.nchunk;
-    L.ends = reinterpret_cast<uint16_t*>(L.red + 32);
-    L.eidx = L.ends + I.nslot;
-    L.cs = L.eidx + I.nslot;
-    L.cv = L.cs + I.nchunk + 1;
-    L.cptr = L.cv + I.nchunk;
-    for (int i = t; i < I.nslot; i += T) {
-        L.ends[i] = a.ends[I.soff + i];
-        L.eidx[i] = a.slot_e[I.soff + i];
+    L.theta = reinterpret_cast<double*>(smem);
+    L.fslot = L.theta + pad2(I.n);
+    L.zero_pair = static_cast<uint32_t>(I.npair);
+    L.epar = L.fslot + 2 * (I.npair + kZeroPairs + kDumpPairs);
+    L.red = BlockRed{L.epar + ne4 * NPE};
+    double* locate = L.red.red + 32;             // METHOD 2: the crossing location's arrays
+    constexpr bool kLocate = METHOD == 2;
+    const int32_t extra = kLocate ? locate_bytes(I.n, I.ne) : 0;
+    L.tab_lds = I.lds_bytes + extra + I.tab_bytes <= a.lds_max;
+    uint2* tab = reinterpret_cast<uint2*>(reinterpret_cast<char*>(locate) + extra);
+    L.partial = reinterpret_cast<double*>(tab + (L.tab_lds ? ne4 : 0));
+    uint32_t* hc = reinterpret_cast<uint32_t*>(L.partial + I.nhc);
+    L.tab = tab;
+    L.tab_g = a.tab + I.toff;
+    L.hc = hc;
+    L.hc_g = a.hc + I.hoff;
+    if (L.tab_lds) {
+        for (int i = t; i < ne4; i += T) tab[i] = L.tab_g[i];
+        for (int i = t; i < I.nhc; i += T) hc[i] = L.hc_g[i];
     }
-    for (int i = t; i <= I.nchunk; i += T) L.cs[i] = a.cs[I.csoff + i];
-    for (int i = t; i < I.nchunk; i += T) L.cv[i] = a.cv[I.cvoff + i];
-    for (int i = t; i <= I.n; i += T) L.cptr[i] = a.cptr[I.cpoff + i];
+    for (int i = t; i < 2 * (I.npair + kZeroPairs + kDumpPairs); i += T) L.fslot[i] = 0.0;
     const double* pe_g = a.p + I.poff + static_cast<int64_t>(I.n) * VPar<VM>::np;
-    for (int i = t; i < I.ne * NPE; i += T) L.epar[i] = pe_g[i];
+    for (int i = t; i < ne4 * NPE; i += T) L.epar[i] = i < I.ne * NPE ? pe_g[i] : 0.0;
 
     double y[V][D], pv[V][NPV];
+    uint32_t row[V];
     const double* pg = a.p + I.poff;                 // the instance's vertex parameters
 #pragma unroll
     for (int k = 0; k < V; ++k) {
         const int v = t + k * T;
+        row[k] = v < I.n ? a.row[I.voff + v] : 0;
 #pragma unroll
         for (int j = 0; j < D; ++j) y[k][j] = v < I.n ? a.u[I.uoff + static_cast<int64_t>(v) * D + j] : 0.0;
 #pragma unroll
         for (int j = 0; j < NPV; ++j)
-            pv[k][j] = (!kParamsInMemory<V> && v < I.n && VPar<VM>::np > 0)
+            pv[k][j] = ((!kParamsInMemory<V> || (kInverse0<VM> && j == 0)) && v < I.n && VPar<VM>::np > 0)
                            ? a.p[I.poff + static_cast<int64_t>(v) * VPar<VM>::np + j] : 0.0;
+        if constexpr (kInverse0<VM>) pv[k][0] = 1.0 / pv[k][0];
     }
     __syncthreads();
 
@@ -377,56 +556,60 @@ __global__ void __launch_bounds__(LB) k_ensemble(SolveArgs a) {
     double dt = a.dt0;
     const double inv_len = 1.0 / (static_cast<double>(I.n) * D);
 
+    // The right-hand side appears once in each method below, inside one loop over the
+    // evaluations: with a copy per stage the Tsit5 loop's code exceeded the instruction cache
+    // and its constants the scalar registers.  (A kernel of 9 copies: about 100 KB of code and
+    // 230 spilled scalar registers, reloaded lane by lane inside the edge loops.)
+#define ND_EACH                                        \
+    _Pragma("unroll") for (int q = 0; q < V; ++q)      \
+        _Pragma("unroll") for (int j = 0; j < D; ++j)
+    double ys[V][D], k[V][D];
     if constexpr (METHOD == 1) {
         // fixed-step classic RK4: u + dt/6*(((k1 + 2k2) + 2k3) + k4)
-        double k[V][D], acc[V][D], ys[V][D];
+        double acc[V][D];
         const int64_t nsteps = static_cast<int64_t>(llround((a.t1 - a.t0) / dt));
         const double half = 0.5 * dt, sixth = dt / 6.0;
         int64_t done = nsteps;
-        for (int64_t step = 0; step < nsteps; ++step) {
-            rhs<VM, EM, V>(I, L, y, pv, pg, k);
-#pragma unroll
-            for (int q = 0; q < V; ++q)
-#pragma unroll
-                for (int j = 0; j < D; ++j) { acc[q][j] = k[q][j]; ys[q][j] = y[q][j] + half * k[q][j]; }
-            rhs<VM, EM, V>(I, L, ys, pv, pg, k);
-#pragma unroll
-            for (int q = 0; q < V; ++q)
-#pragma unroll
-                for (int j = 0; j < D; ++j) { acc[q][j] = acc[q][j] + 2.0 * k[q][j]; ys[q][j] = y[q][j] + half * k[q][j]; }
-            rhs<VM, EM, V>(I, L, ys, pv, pg, k);
-#pragma unroll
-            for (int q = 0; q < V; ++q)
-#pragma unroll
-                for (int j = 0; j < D; ++j) { acc[q][j] = acc[q][j] + 2.0 * k[q][j]; ys[q][j] = y[q][j] + dt * k[q][j]; }
-            rhs<VM, EM, V>(I, L, ys, pv, pg, k);
-#pragma unroll
-            for (int q = 0; q < V; ++q)
-#pragma unroll
-                for (int j = 0; j < D; ++j) y[q][j] = y[q][j] + sixth * (acc[q][j] + k[q][j]);
-            nf += 4;
-            ++naccept;
-            if (a.limit) {
-                edge_flows<VM, EM, V>(I, L, y);
-                ntrip += trip_lines<VM, EM>(a, I, L);
+        ND_EACH { ys[q][j] = y[q][j]; acc[q][j] = 0.0; }
+        int stage = 0;                              // 0..3, 4: the steady-state check's evaluation
+        for (int64_t step = 0; step < nsteps;) {
+            rhs<VM, EM, V, kFresh<V, LB>>(I, L, ys, pv, pg, row, k);
+            ++nf;
+            if (stage < 3) {
+                const double hs = stage == 2 ? dt : half;
+                if (stage == 0) ND_EACH acc[q][j] = k[q][j];
+                else ND_EACH acc[q][j] = acc[q][j] + 2.0 * k[q][j];
+                ND_EACH ys[q][j] = y[q][j] + hs * k[q][j];
+                ++stage;
+                continue;
             }
-            if (ee >= 0 && step + 1 == static_cast<int64_t>(llround((te - a.t0) / dt))) ntrip += trip_edge<VM, EM>(a, I, L, ee);
-            if (a.ss) {
-                rhs<VM, EM, V>(I, L, y, pv, pg, k);
-                ++nf;
-                if (at_steady_state<V, D>(a, I, L, y, k)) {
-                    done = step + 1;
-                    retcode = 4;
-                    break;
+            if (stage == 3) {
+                ND_EACH { y[q][j] = y[q][j] + sixth * (acc[q][j] + k[q][j]); ys[q][j] = y[q][j]; }
+                ++naccept;
+                if (a.limit) {
+                    edge_flows<VM, EM, V, kFresh<V, LB>>(I, L, y);
+                    ntrip += trip_lines<VM, EM>(a, I, L);
                 }
+                if (ee >= 0 && step + 1 == static_cast<int64_t>(llround((te - a.t0) / dt))) ntrip += trip_edge<VM, EM>(a, I, L, ee);
+                if (a.ss) {
+                    stage = 4;
+                    continue;
+                }
+            } else if (at_steady_state<V, D>(a, I, L, y, k)) {
+                done = step + 1;
+                retcode = 4;
+                break;
             }
+            stage = 0;
+            ++step;
         }
         tcur = a.t0 + static_cast<double>(done) * dt;
     } else {
-        double k1[V][D], k2[V][D], k3[V][D], k4[V][D], k5[V][D], k6[V][D], k7[V][D], ys[V][D];
-        double d2[V][D], d3[V][D], d4[V][D];      // dense output (crossing location only)
-        rhs<VM, EM, V>(I, L, y, pv, pg, k1);
-        ++nf;
+        // k3..k5 hold the dense-output coefficients d2..d4 once the last evaluation has begun
+        // (crossing location), k2 the error estimate's sum over the first six stages
+        double k1[V][D], k2[V][D], k3[V][D], k4[V][D], k5[V][D], k6[V][D];
+        auto &d2 = k3, &d3 = k4, &d4 = k5;
+        ND_EACH { ys[q][j] = y[q][j]; k1[q][j] = k2[q][j] = k3[q][j] = k4[q][j] = k5[q][j] = k6[q][j] = 0.0; }
         auto wnorm2 = [&](const double (&x)[V][D], const double (&ref)[V][D]) {
             double s = 0.0;
 #pragma unroll
@@ -438,259 +621,279 @@ __global__ void __launch_bounds__(LB) k_ensemble(SolveArgs a) {
                         const double r = x[q][j] / sc;
                         s += r * r;
                     }
-            return block_sum(s, L.red);
+            return L.red.sum(s);
         };
-        if (!(dt > 0.0)) {
-            // initial step (Hairer, Norsett & Wanner, Solving ODEs I, II.4)
-            const double d0 = sqrt(wnorm2(y, y) * inv_len), d1 = sqrt(wnorm2(k1, y) * inv_len);
-            double h0 = (d0 < 1e-5 || d1 < 1e-5) ? 1e-6 : 0.01 * d0 / d1;
-            h0 = fmin(h0, a.t1 - a.t0);
-#pragma unroll
-            for (int q = 0; q < V; ++q)
-#pragma unroll
-                for (int j = 0; j < D; ++j) ys[q][j] = y[q][j] + h0 * k1[q][j];
-            rhs<VM, EM, V>(I, L, ys, pv, pg, k2);
-            ++nf;
-#pragma unroll
-            for (int q = 0; q < V; ++q)
-#pragma unroll
-                for (int j = 0; j < D; ++j) k3[q][j] = k2[q][j] - k1[q][j];
-            const double d2 = sqrt(wnorm2(k3, y) * inv_len) / h0;
-            const double m = fmax(d1, d2);
-            const double h1 = m <= 1e-15 ? fmax(1e-6, h0 * 1e-3) : pow(0.01 / m, 1.0 / 6.0);
-            dt = fmin(100.0 * h0, h1);
-        }
-        dt = fmin(dt, a.dtmax);
-        double qold = 1e-4;
+        double qold = 1e-4, d1 = 0.0, h = 0.0;
         int64_t iters = 0;
         double tstop = ee >= 0 ? te : a.t1;       // the next time a step must end on
+        bool last = false;
         // crossing location: a second phase buffer and, per edge, the condition's sign at
         // the step start (gsign) and end (gnext) and the first point of the step where it
-        // crossed (gev), in LDS after the u16 tables
-        constexpr bool kLocate = METHOD == 2;
-        const double* lim = a.limit ? a.limit + I.soff / 2 : nullptr;
+        // crossed (gev), in LDS after the reduction buffers
+        const double* lim = a.limit ? a.limit + I.eoff : nullptr;
         double* theta2 = nullptr;
         int8_t *gsign = nullptr, *gnext = nullptr, *gev = nullptr;
         if constexpr (kLocate) {
-            char* base = reinterpret_cast<char*>(smem);
-            const size_t off = (static_cast<size_t>(reinterpret_cast<char*>(L.cptr + I.n + 1) - base) + 7) & ~size_t(7);
-            theta2 = reinterpret_cast<double*>(base + off);
+            theta2 = locate;
             gsign = reinterpret_cast<int8_t*>(theta2 + I.n);
             gnext = gsign + I.ne;
             gev = gnext + I.ne;
-            if (lim) line_signs<VM, EM, V>(I, L, lim, y, gsign);
         }
-        while (tcur < a.t1) {
-            if (iters++ >= a.maxiters) { retcode = 1; break; }
-            if (dt < a.dtmin) { retcode = 2; break; }
-            const bool last = tcur + dt >= tstop;
-            const double h = last ? tstop - tcur : dt;
-#define ND_STAGE(expr)                                                        \
-    _Pragma("unroll") for (int q = 0; q < V; ++q)                             \
-        _Pragma("unroll") for (int j = 0; j < D; ++j) ys[q][j] = y[q][j] + h * (expr);
-            ND_STAGE(c_a21 * k1[q][j]);
-            rhs<VM, EM, V>(I, L, ys, pv, pg, k2);
-            ND_STAGE(c_a31 * k1[q][j] + c_a32 * k2[q][j]);
-            rhs<VM, EM, V>(I, L, ys, pv, pg, k3);
-            ND_STAGE(c_a41 * k1[q][j] + c_a42 * k2[q][j] + c_a43 * k3[q][j]);
-            rhs<VM, EM, V>(I, L, ys, pv, pg, k4);
-            ND_STAGE(c_a51 * k1[q][j] + c_a52 * k2[q][j] + c_a53 * k3[q][j] + c_a54 * k4[q][j]);
-            rhs<VM, EM, V>(I, L, ys, pv, pg, k5);
-            ND_STAGE(c_a61 * k1[q][j] + c_a62 * k2[q][j] + c_a63 * k3[q][j] + c_a64 * k4[q][j] + c_a65 * k5[q][j]);
-            rhs<VM, EM, V>(I, L, ys, pv, pg, k6);
-            ND_STAGE(c_a71 * k1[q][j] + c_a72 * k2[q][j] + c_a73 * k3[q][j] + c_a74 * k4[q][j] + c_a75 * k5[q][j] +
-                     c_a76 * k6[q][j]);
-#undef ND_STAGE
-            if constexpr (kLocate) {
-                // dense-output coefficients from k1..k6 (k7 follows); they take the place
-                // of k3..k6 in registers
-#pragma unroll
-                for (int q = 0; q < V; ++q)
-#pragma unroll
-                    for (int j = 0; j < D; ++j) {
-                        d2[q][j] = ND_R(1, 2) * k1[q][j] + ND_R(2, 2) * k2[q][j] + ND_R(3, 2) * k3[q][j] +
-                                   ND_R(4, 2) * k4[q][j] + ND_R(5, 2) * k5[q][j] + ND_R(6, 2) * k6[q][j];
-                        d3[q][j] = ND_R(1, 3) * k1[q][j] + ND_R(2, 3) * k2[q][j] + ND_R(3, 3) * k3[q][j] +
-                                   ND_R(4, 3) * k4[q][j] + ND_R(5, 3) * k5[q][j] + ND_R(6, 3) * k6[q][j];
-                        d4[q][j] = ND_R(1, 4) * k1[q][j] + ND_R(2, 4) * k2[q][j] + ND_R(3, 4) * k3[q][j] +
-                                   ND_R(4, 4) * k4[q][j] + ND_R(5, 4) * k5[q][j] + ND_R(6, 4) * k6[q][j];
-                    }
-            }
-            // error-estimate combination of k1..k6 before the last evaluation, so only
-            // y, ynew and this sum stay live across it
-#pragma unroll
-            for (int q = 0; q < V; ++q)
-#pragma unroll
-                for (int j = 0; j < D; ++j)
-                    k2[q][j] = c_bt1 * k1[q][j] + c_bt2 * k2[q][j] + c_bt3 * k3[q][j] + c_bt4 * k4[q][j] +
-                               c_bt5 * k5[q][j] + c_bt6 * k6[q][j];
-            rhs<VM, EM, V>(I, L, ys, pv, pg, k7);
-            nf += 6;
-            if constexpr (kLocate) {
-#pragma unroll
-                for (int q = 0; q < V; ++q)
-#pragma unroll
-                    for (int j = 0; j < D; ++j) {
-                        d2[q][j] = d2[q][j] + ND_R(7, 2) * k7[q][j];
-                        d3[q][j] = d3[q][j] + ND_R(7, 3) * k7[q][j];
-                        d4[q][j] = d4[q][j] + ND_R(7, 4) * k7[q][j];
-                    }
-            }
-            double s = 0.0;
-#pragma unroll
-            for (int q = 0; q < V; ++q)
-                if (t + q * T < I.n)
-#pragma unroll
-                    for (int j = 0; j < D; ++j) {
-                        const double e = h * (k2[q][j] + c_bt7 * k7[q][j]);
-                        const double sc = a.abstol + fmax(fabs(y[q][j]), fabs(ys[q][j])) * a.reltol;
-                        const double r = e / sc;
-                        s += r * r;
-                    }
-            const double eest = sqrt(block_sum(s, L.red) * inv_len);
-            const double q11 = pow(eest, 0.14);
-            if (eest <= 1.0) {
-                double qq = eest == 0.0 ? 0.1 : fmax(0.1, fmin(5.0, q11 / pow(qold, 0.08) / 0.9));
-                // a step that ends within 100 ulp of the stop time ends on it (as
-                // OrdinaryDiffEq's fixed_t_for_floatingpoint_error! does)
-                const double tn = tcur + h;
-                const bool at_stop = last || fabs(tn - tstop) < 100.0 * 2.220446049250313e-16 * fmax(fabs(tcur), fabs(tstop));
-                qold = fmax(eest, 1e-4);
-                dt = fmin(h / qq, a.dtmax);
-                ++naccept;
-                int changed = 0;
-                bool located = false;
-                if constexpr (kLocate) {
-                    if (lim) {
-                        // the condition at the points s = m/9 of the step (m = 9: the accepted
-                        // state), against its sign at the step start
-                        double first = 10.0;
-#pragma unroll 1
-                        for (int m = 1; m <= 9; ++m) {
-                            double* th = (m & 1) ? theta2 : L.theta;   // alternate: one barrier a point
-                            const double s = static_cast<double>(m) / 9.0;
-#pragma unroll
-                            for (int q = 0; q < V; ++q) {
-                                const int v = t + q * T;
-                                if (v < I.n)
-                                    th[v] = m == 9 ? ys[q][0]
-                                                   : dense_at(y[q][0], k1[q][0], d2[q][0], d3[q][0], d4[q][0], h, s);
-                            }
-                            __syncthreads();
-                            for (int e = t; e < I.ne; e += T) {
-                                const int8_t ns = sign8(line_cond<EM>(L, th, lim, e));
-                                if (m == 1) gev[e] = 0;
-                                if (gev[e] == 0 && crossed(gsign[e], ns)) {
-                                    gev[e] = static_cast<int8_t>(m);
-                                    first = fmin(first, static_cast<double>(m));
-                                }
-                                if (m == 9) gnext[e] = ns;
-                            }
+        // what the evaluation at ys is: 0 the first derivative, 1..6 the step's stages 2..7,
+        // 7 the initial step's probe, 8 the first derivative again after a trip
+        int phase = 0;
+        for (;;) {
+            rhs<VM, EM, V, kFresh<V, LB>>(I, L, ys, pv, pg, row, k);
+            ++nf;
+            bool accepted = false, begun = true;
+            if (phase >= 1 && phase <= 5) {
+                // stage derivative k_{phase+1}, then the next stage's state
+#define ND_STAGE(kn, expr)                                                   \
+    ND_EACH {                                                                \
+        kn[q][j] = k[q][j];                                                  \
+        ys[q][j] = y[q][j] + h * (expr);                                     \
+    }
+                if (phase == 1) {
+                    ND_STAGE(k2, c_a31 * k1[q][j] + c_a32 * k2[q][j])
+                } else if (phase == 2) {
+                    ND_STAGE(k3, c_a41 * k1[q][j] + c_a42 * k2[q][j] + c_a43 * k3[q][j])
+                } else if (phase == 3) {
+                    ND_STAGE(k4, c_a51 * k1[q][j] + c_a52 * k2[q][j] + c_a53 * k3[q][j] + c_a54 * k4[q][j])
+                } else if (phase == 4) {
+                    ND_STAGE(k5, c_a61 * k1[q][j] + c_a62 * k2[q][j] + c_a63 * k3[q][j] + c_a64 * k4[q][j] +
+                                     c_a65 * k5[q][j])
+                } else {
+                    ND_STAGE(k6, c_a71 * k1[q][j] + c_a72 * k2[q][j] + c_a73 * k3[q][j] + c_a74 * k4[q][j] +
+                                     c_a75 * k5[q][j] + c_a76 * k6[q][j])
+                    // before the last evaluation: the error estimate's sum and the dense
+                    // output's coefficients over k1..k6 take the place of k2..k5
+                    ND_EACH {
+                        const double e = c_bt1 * k1[q][j] + c_bt2 * k2[q][j] + c_bt3 * k3[q][j] + c_bt4 * k4[q][j] +
+                                         c_bt5 * k5[q][j] + c_bt6 * k6[q][j];
+                        if constexpr (kLocate) {
+                            const double e2 = ND_R(1, 2) * k1[q][j] + ND_R(2, 2) * k2[q][j] +
+                                              ND_R(3, 2) * k3[q][j] + ND_R(4, 2) * k4[q][j] +
+                                              ND_R(5, 2) * k5[q][j] + ND_R(6, 2) * k6[q][j];
+                            const double e3 = ND_R(1, 3) * k1[q][j] + ND_R(2, 3) * k2[q][j] +
+                                              ND_R(3, 3) * k3[q][j] + ND_R(4, 3) * k4[q][j] +
+                                              ND_R(5, 3) * k5[q][j] + ND_R(6, 3) * k6[q][j];
+                            const double e4 = ND_R(1, 4) * k1[q][j] + ND_R(2, 4) * k2[q][j] +
+                                              ND_R(3, 4) * k3[q][j] + ND_R(4, 4) * k4[q][j] +
+                                              ND_R(5, 4) * k5[q][j] + ND_R(6, 4) * k6[q][j];
+                            d2[q][j] = e2;
+                            d3[q][j] = e3;
+                            d4[q][j] = e4;
                         }
-                        first = block_min(first, L.red);
-                        if (first < 10.0) {
-                            // bisect [point mf-1, point mf] on the dense output, over the edges
-                            // that crossed at point mf, down to adjacent doubles
-                            const int mf = static_cast<int>(first);
-                            double lo = tcur + h * (static_cast<double>(mf - 1) / 9.0);
-                            double hi = tcur + h * (static_cast<double>(mf) / 9.0);
-                            bool hi_end = mf == 9;                  // hi: still the accepted state
-                            for (int it = 0; it < 256; ++it) {
-                                const double mid = lo + 0.5 * (hi - lo);
-                                if (!(mid > lo && mid < hi)) break;
-                                const double s = (mid - tcur) / h;
+                        k2[q][j] = e;
+                    }
+                }
+#undef ND_STAGE
+                ++phase;
+                continue;
+            }
+            if (phase == 6) {
+                if constexpr (kLocate) {
+                    ND_EACH {
+                        d2[q][j] = d2[q][j] + ND_R(7, 2) * k[q][j];
+                        d3[q][j] = d3[q][j] + ND_R(7, 3) * k[q][j];
+                        d4[q][j] = d4[q][j] + ND_R(7, 4) * k[q][j];
+                    }
+                }
+                double s = 0.0;
+#pragma unroll
+                for (int q = 0; q < V; ++q)
+                    if (t + q * T < I.n)
+#pragma unroll
+                        for (int j = 0; j < D; ++j) {
+                            const double e = h * (k2[q][j] + c_bt7 * k[q][j]);
+                            const double sc = a.abstol + fmax(fabs(y[q][j]), fabs(ys[q][j])) * a.reltol;
+                            const double r = e / sc;
+                            s += r * r;
+                        }
+                const double eest = sqrt(L.red.sum(s) * inv_len);
+                double q11, qold8;
+                step_pow2(eest, 0.14, qold, 0.08, q11, qold8);
+                if (eest <= 1.0) {
+                    double qq = eest == 0.0 ? 0.1 : fmax(0.1, fmin(5.0, q11 / qold8 / 0.9));
+                    // a step that ends within 100 ulp of the stop time ends on it (as
+                    // OrdinaryDiffEq's fixed_t_for_floatingpoint_error! does)
+                    const double tn = tcur + h;
+                    const bool at_stop = last || fabs(tn - tstop) < 100.0 * 2.220446049250313e-16 * fmax(fabs(tcur), fabs(tstop));
+                    qold = fmax(eest, 1e-4);
+                    dt = fmin(h / qq, a.dtmax);
+                    ++naccept;
+                    int changed = 0;
+                    bool located = false;
+                    if constexpr (kLocate) {
+                        if (lim) {
+                            // the condition at the points s = m/9 of the step (m = 9: the accepted
+                            // state), against its sign at the step start
+                            double first = 10.0;
+#pragma unroll 1
+                            for (int m = 1; m <= 9; ++m) {
+                                double* th = (m & 1) ? theta2 : L.theta;   // alternate: one barrier a point
+                                const double s = static_cast<double>(m) / 9.0;
 #pragma unroll
                                 for (int q = 0; q < V; ++q) {
                                     const int v = t + q * T;
-                                    if (v < I.n) L.theta[v] = dense_at(y[q][0], k1[q][0], d2[q][0], d3[q][0], d4[q][0], h, s);
+                                    if (v < I.n)
+                                        th[v] = m == 9 ? ys[q][0]
+                                                       : dense_at(y[q][0], k1[q][0], d2[q][0], d3[q][0], d4[q][0], h, s);
                                 }
                                 __syncthreads();
-                                double hit = 0.0;
+                                for (int e = t; e < I.ne; e += T) {
+                                    const int8_t ns = sign8(line_cond<EM>(L, th, lim, e));
+                                    if (m == 1) gev[e] = 0;
+                                    if (gev[e] == 0 && crossed(gsign[e], ns)) {
+                                        gev[e] = static_cast<int8_t>(m);
+                                        first = fmin(first, static_cast<double>(m));
+                                    }
+                                    if (m == 9) gnext[e] = ns;
+                                }
+                            }
+                            first = L.red.min(first);
+                            if (first < 10.0) {
+                                // bisect [point mf-1, point mf] on the dense output, over the edges
+                                // that crossed at point mf, down to adjacent doubles
+                                const int mf = static_cast<int>(first);
+                                double lo = tcur + h * (static_cast<double>(mf - 1) / 9.0);
+                                double hi = tcur + h * (static_cast<double>(mf) / 9.0);
+                                bool hi_end = mf == 9;                  // hi: still the accepted state
+                                for (int it = 0; it < 256; ++it) {
+                                    const double mid = lo + 0.5 * (hi - lo);
+                                    if (!(mid > lo && mid < hi)) break;
+                                    const double s = (mid - tcur) / h;
+#pragma unroll
+                                    for (int q = 0; q < V; ++q) {
+                                        const int v = t + q * T;
+                                        if (v < I.n) L.theta[v] = dense_at(y[q][0], k1[q][0], d2[q][0], d3[q][0], d4[q][0], h, s);
+                                    }
+                                    __syncthreads();
+                                    double hit = 0.0;
+                                    for (int e = t; e < I.ne; e += T)
+                                        if (gev[e] == mf && crossed(gsign[e], sign8(line_cond<EM>(L, L.theta, lim, e)))) hit = 1.0;
+                                    if (L.red.sum(hit) > 0.0) {
+                                        hi = mid;
+                                        hi_end = false;
+                                    } else {
+                                        lo = mid;
+                                    }
+                                }
+                                // the edges that crossed by hi trip; the solution moves to lo, the
+                                // left end of the bracket (DiffEqBase's LeftRootFind)
+                                const double shi = (hi - tcur) / h;
+#pragma unroll
+                                for (int q = 0; q < V; ++q) {
+                                    const int v = t + q * T;
+                                    if (v < I.n)
+                                        L.theta[v] = hi_end ? ys[q][0]
+                                                            : dense_at(y[q][0], k1[q][0], d2[q][0], d3[q][0], d4[q][0], h, shi);
+                                }
+                                __syncthreads();
+                                constexpr int NPE1 = NPE > 0 ? NPE : 1;
+                                double* pw = a.p + I.poff + static_cast<int64_t>(I.n) * VPar<VM>::np;
+                                double cnt = 0.0;
                                 for (int e = t; e < I.ne; e += T)
-                                    if (gev[e] == mf && crossed(gsign[e], sign8(line_cond<EM>(L, L.theta, lim, e)))) hit = 1.0;
-                                if (block_sum(hit, L.red) > 0.0) {
-                                    hi = mid;
-                                    hi_end = false;
-                                } else {
-                                    lo = mid;
-                                }
+                                    if (gev[e] == mf && crossed(gsign[e], sign8(line_cond<EM>(L, L.theta, lim, e)))) {
+                                        L.epar[e * NPE1] = 0.0;
+                                        pw[static_cast<int64_t>(e) * NPE1] = 0.0;
+                                        cnt += 1.0;
+                                    }
+                                ntrip += static_cast<int>(L.red.sum(cnt));
+                                const double slo = (lo - tcur) / h;
+#pragma unroll
+                                for (int q = 0; q < V; ++q)
+#pragma unroll
+                                    for (int j = 0; j < D; ++j)
+                                        y[q][j] = dense_at(y[q][j], k1[q][j], d2[q][j], d3[q][j], d4[q][j], h, slo);
+                                tcur = lo;
+                                located = true;
+                                changed = 1;                            // the state moved: new derivative
                             }
-                            // the edges that crossed by hi trip; the solution moves to lo, the
-                            // left end of the bracket (DiffEqBase's LeftRootFind)
-                            const double shi = (hi - tcur) / h;
-#pragma unroll
-                            for (int q = 0; q < V; ++q) {
-                                const int v = t + q * T;
-                                if (v < I.n)
-                                    L.theta[v] = hi_end ? ys[q][0]
-                                                        : dense_at(y[q][0], k1[q][0], d2[q][0], d3[q][0], d4[q][0], h, shi);
-                            }
-                            __syncthreads();
-                            constexpr int NPE1 = NPE > 0 ? NPE : 1;
-                            double* pw = a.p + I.poff + static_cast<int64_t>(I.n) * VPar<VM>::np;
-                            double cnt = 0.0;
-                            for (int e = t; e < I.ne; e += T)
-                                if (gev[e] == mf && crossed(gsign[e], sign8(line_cond<EM>(L, L.theta, lim, e)))) {
-                                    L.epar[e * NPE1] = 0.0;
-                                    pw[static_cast<int64_t>(e) * NPE1] = 0.0;
-                                    cnt += 1.0;
-                                }
-                            ntrip += static_cast<int>(block_sum(cnt, L.red));
-                            const double slo = (lo - tcur) / h;
-#pragma unroll
-                            for (int q = 0; q < V; ++q)
-#pragma unroll
-                                for (int j = 0; j < D; ++j)
-                                    y[q][j] = dense_at(y[q][j], k1[q][j], d2[q][j], d3[q][j], d4[q][j], h, slo);
-                            tcur = lo;
-                            located = true;
-                            changed = 1;                            // the state moved: new derivative
                         }
                     }
-                }
-                if (!located) {
-                    tcur = at_stop ? tstop : tn;
+                    if (!located) {
+                        tcur = at_stop ? tstop : tn;
 #pragma unroll
-                    for (int q = 0; q < V; ++q)
+                        for (int q = 0; q < V; ++q)
 #pragma unroll
-                        for (int j = 0; j < D; ++j) { y[q][j] = ys[q][j]; k1[q][j] = k7[q][j]; }
-                    if constexpr (kLocate) {
-                        int8_t* sw = gsign;                         // the end signs start the next step
-                        gsign = gnext;
-                        gnext = sw;
-                    } else if (a.limit) {
-                        // fval holds the flows at the accepted state (the last evaluation was at ys)
-                        const int tr = trip_lines<VM, EM>(a, I, L);
-                        ntrip += tr;
-                        changed += tr;
+                            for (int j = 0; j < D; ++j) { y[q][j] = ys[q][j]; k1[q][j] = k[q][j]; }
+                        if constexpr (kLocate) {
+                            int8_t* sw = gsign;                         // the end signs start the next step
+                            gsign = gnext;
+                            gnext = sw;
+                        } else if (a.limit) {
+                            // fslot holds the flows at the accepted state (the last evaluation was at ys)
+                            const int tr = trip_lines<VM, EM>(a, I, L);
+                            ntrip += tr;
+                            changed += tr;
+                        }
+                        if (at_stop && ee >= 0 && tstop == te) {   // the preset trip's time is reached
+                            const int tr = trip_edge<VM, EM>(a, I, L, ee);
+                            ntrip += tr;
+                            changed += tr;
+                            ee = -1;
+                            tstop = a.t1;
+                        }
                     }
-                    if (at_stop && ee >= 0 && tstop == te) {   // the preset trip's time is reached
-                        const int tr = trip_edge<VM, EM>(a, I, L, ee);
-                        ntrip += tr;
-                        changed += tr;
-                        ee = -1;
-                        tstop = a.t1;
+                    // after a trip or a move to a crossing the first-same-as-last derivative
+                    // (and the condition signs) are stale: evaluate them again
+                    if (changed > 0) {
+                        ND_EACH ys[q][j] = y[q][j];
+                        phase = 8;
+                        continue;
                     }
+                    accepted = true;
+                } else {
+                    dt = h / fmin(5.0, q11 / 0.9);
+                    ++nreject;
                 }
-                // after a trip or a move to a crossing the first-same-as-last derivative
-                // (and the condition signs) are stale: re-evaluate them
-                if (changed > 0) {
-                    rhs<VM, EM, V>(I, L, y, pv, pg, k1);
-                    ++nf;
-                    if constexpr (kLocate)
-                        if (lim) line_signs<VM, EM, V>(I, L, lim, y, gsign);
-                }
-                if (a.ss && at_steady_state<V, D>(a, I, L, y, k1)) {
-                    retcode = 4;
-                    break;
-                }
+            } else if (phase == 8) {
+                ND_EACH k1[q][j] = k[q][j];
+                if constexpr (kLocate)
+                    if (lim) line_signs<VM, EM, V>(I, L, lim, y, gsign);
+                accepted = true;
             } else {
-                dt = h / fmin(5.0, q11 / 0.9);
-                ++nreject;
+                // the start: k1, then for an automatic initial step its probe (Hairer, Norsett &
+                // Wanner, Solving ODEs I, II.4)
+                if (phase == 0) {
+                    ND_EACH k1[q][j] = k[q][j];
+                    if (!(dt > 0.0)) {
+                        const double d0 = sqrt(wnorm2(y, y) * inv_len);
+                        d1 = sqrt(wnorm2(k1, y) * inv_len);
+                        h = (d0 < 1e-5 || d1 < 1e-5) ? 1e-6 : 0.01 * d0 / d1;
+                        h = fmin(h, a.t1 - a.t0);
+                        ND_EACH ys[q][j] = y[q][j] + h * k1[q][j];
+                        phase = 7;
+                        continue;
+                    }
+                } else {
+                    ND_EACH k[q][j] = k[q][j] - k1[q][j];
+                    const double dd2 = sqrt(wnorm2(k, y) * inv_len) / h;
+                    const double m = fmax(d1, dd2);
+                    const double h1 = m <= 1e-15 ? fmax(1e-6, h * 1e-3) : uniform_f64(step_pow(0.01 / m, 1.0 / 6.0));
+                    dt = fmin(100.0 * h, h1);
+                }
+                dt = fmin(dt, a.dtmax);
+                begun = false;
+                if constexpr (kLocate)
+                    if (lim) line_signs<VM, EM, V>(I, L, lim, y, gsign);
             }
-            if (!(dt == dt)) { retcode = 3; break; }
+            if (accepted && a.ss && at_steady_state<V, D>(a, I, L, y, k1)) {
+                retcode = 4;
+                break;
+            }
+            if (begun && !(dt == dt)) { retcode = 3; break; }
+            if (!(tcur < a.t1)) break;
+            if (iters++ >= a.maxiters) { retcode = 1; break; }
+            if (dt < a.dtmin) { retcode = 2; break; }
+            last = tcur + dt >= tstop;
+            h = last ? tstop - tcur : dt;
+            ND_EACH ys[q][j] = y[q][j] + h * (c_a21 * k1[q][j]);
+            phase = 1;
         }
     }
+#undef ND_EACH
 #pragma unroll
     for (int k = 0; k < V; ++k) {
         const int v = t + k * T;
@@ -711,12 +914,36 @@ __global__ void __launch_bounds__(LB) k_ensemble(SolveArgs a) {
     }
 }
 
+template <int VM, int EM, int METHOD, int V, int LB>
+__global__ void __launch_bounds__(LB) k_ensemble(SolveArgs a) {
+    extern __shared__ double2 smem[];
+    const int inst = a.order[a.first + static_cast<int>(blockIdx.x)];
+    const InstDesc I = a.inst[inst];
+    ensemble_body<VM, EM, METHOD, V, LB>(a, inst, I, smem);
+}
+
+// Several size classes of one thread count in one launch: each instance runs with its
+// class's vertices per thread.
+template <int VM, int EM, int METHOD>
+__global__ void __launch_bounds__(512) k_ensemble_mixed(SolveArgs a) {
+    extern __shared__ double2 smem[];
+    const int inst = a.order[a.first + static_cast<int>(blockIdx.x)];
+    const InstDesc I = a.inst[inst];
+    switch (__builtin_amdgcn_readfirstlane(I.vper)) {
+    case 1: ensemble_body<VM, EM, METHOD, 1, 512>(a, inst, I, smem); break;
+    case 2: ensemble_body<VM, EM, METHOD, 2, 512>(a, inst, I, smem); break;
+    case 3: ensemble_body<VM, EM, METHOD, 3, 512>(a, inst, I, smem); break;
+    default: ensemble_body<VM, EM, METHOD, 4, 512>(a, inst, I, smem); break;
+    }
+}
+
 using EnsKernel = void (*)(SolveArgs);
 
-// Workgroups of up to 512 threads take any vper; 1024-thread workgroups (16 waves, at
-// most 128 VGPRs each) take one or two vertices per thread.
+// Workgroups of up to 512 threads take any vper (0: by instance); 1024-thread workgroups
+// (16 waves, at most 128 VGPRs each) take one or two vertices per thread.
 template <int VM, int EM, int METHOD>
 EnsKernel pick_v(int vper, int threads) {
+    if (vper == 0) return k_ensemble_mixed<VM, EM, METHOD>;
     if (threads > 512) return vper == 1 ? k_ensemble<VM, EM, METHOD, 1, 1024> : k_ensemble<VM, EM, METHOD, 2, 1024>;
     switch (vper) {
     case 1: return k_ensemble<VM, EM, METHOD, 1, 512>;
@@ -781,19 +1008,20 @@ struct nd_ensemble {
     std::vector<void*> allocs;
     InstDesc* d_inst = nullptr;
     int32_t* d_order = nullptr;
-    uint16_t *d_ends = nullptr, *d_e = nullptr, *d_cs = nullptr, *d_cv = nullptr, *d_cptr = nullptr;
+    uint2* d_tab = nullptr;
+    uint32_t *d_row = nullptr, *d_hc = nullptr;
     std::vector<int32_t> order;                     // instances grouped by class, largest first
-    int32_t cls_first[ND_ENSEMBLE_CLASSES + 1] = {};
+    int32_t cls_first[ND_ENSEMBLE_CLASSES + 1] = {};   // class c: order[cls_first[c + 1] .. cls_first[c]), the last first
     int64_t generation = 0;                         // bumped whenever the class layout changes
-    // one stream per class so the class launches overlap; forked from and joined back
-    // to the caller's stream with events (default priority, non-blocking)
-    hipStream_t cls_stream[ND_ENSEMBLE_CLASSES] = {};
+    // side streams so the class launches overlap; forked from and joined back to the
+    // caller's stream with events (default priority, non-blocking)
+    hipStream_t side_stream[kSideStreams] = {};
     hipEvent_t ev_fork = nullptr;
-    hipEvent_t ev_join[ND_ENSEMBLE_CLASSES] = {};
+    hipEvent_t ev_join[kSideStreams] = {};
     hipStream_t cap_stream = nullptr;               // origin stream of graph captures
     ~nd_ensemble() {
         for (void* p : allocs) (void)hipFree(p);
-        for (auto& x : cls_stream) if (x) (void)hipStreamDestroy(x);
+        for (auto& x : side_stream) if (x) (void)hipStreamDestroy(x);
         for (auto& x : ev_join) if (x) (void)hipEventDestroy(x);
         if (ev_fork) (void)hipEventDestroy(ev_fork);
         if (cap_stream) (void)hipStreamDestroy(cap_stream);
@@ -840,15 +1068,16 @@ int regroup(nd_ensemble* en) {
         const int c = class_of(en, en->inst[i].n);
         if (c < 0) return nd::set_error(ND_ERR_UNSUPPORTED, "instance %d: %d vertices exceed the largest class", i, en->inst[i].n);
         en->inst[i].cls = c;
+        en->inst[i].vper = en->cls_vper[c];
         byc[c].emplace_back(-en->inst[i].n, i);
     }
     en->order.clear();
-    for (int c = 0; c < ND_ENSEMBLE_CLASSES; ++c) {
-        en->cls_first[c] = static_cast<int32_t>(en->order.size());
+    en->cls_first[ND_ENSEMBLE_CLASSES] = 0;
+    for (int c = ND_ENSEMBLE_CLASSES - 1; c >= 0; --c) {
         std::sort(byc[c].begin(), byc[c].end());
         for (auto& x : byc[c]) en->order.push_back(x.second);
+        en->cls_first[c] = static_cast<int32_t>(en->order.size());
     }
-    en->cls_first[ND_ENSEMBLE_CLASSES] = static_cast<int32_t>(en->order.size());
     if (en->d_order) {
         auto it = std::find(en->allocs.begin(), en->allocs.end(), static_cast<void*>(en->d_order));
         if (it != en->allocs.end()) { (void)hipFree(*it); en->allocs.erase(it); }
@@ -880,11 +1109,10 @@ int make_args(nd_ensemble* en, double* u, double* p, double t0, double t1, const
     *a = SolveArgs{};
     a->inst = en->d_inst;
     a->order = en->d_order;
-    a->ends = en->d_ends;
-    a->slot_e = en->d_e;
-    a->cs = en->d_cs;
-    a->cv = en->d_cv;
-    a->cptr = en->d_cptr;
+    a->tab = en->d_tab;
+    a->row = en->d_row;
+    a->hc = en->d_hc;
+    a->lds_max = en->lds_max;
     a->u = u;
     a->p = p;
     a->limit = o->line_limit;
@@ -909,15 +1137,60 @@ int make_args(nd_ensemble* en, double* u, double* p, double t0, double t1, const
     return ND_OK;
 }
 
-// dynamic LDS of class c: the largest instance's tables, plus for crossing location a
-// second phase buffer and three bytes per edge (after 8-byte alignment)
+// dynamic LDS of class c: the largest need of its instances, each with its tables where they
+// fit as well (the kernel decides by the same sum)
 int32_t class_lds(const nd_ensemble* en, int c, int kmethod) {
     int32_t lds = 0;
-    for (int32_t q = en->cls_first[c]; q < en->cls_first[c + 1]; ++q) {
+    for (int32_t q = en->cls_first[c + 1]; q < en->cls_first[c]; ++q) {
         const InstDesc& I = en->inst[en->order[q]];
-        lds = std::max(lds, I.lds_bytes + (kmethod == 2 ? 8 + 8 * I.n + 3 * I.ne : 0));
+        const int32_t need = I.lds_bytes + (kmethod == 2 ? locate_bytes(I.n, I.ne) : 0);
+        lds = std::max(lds, need + I.tab_bytes <= en->lds_max ? need + I.tab_bytes : need);
     }
     return lds;
+}
+
+// the figure the instances of class c are limited by: with line crossings located, a second
+// phase buffer and three bytes per edge more.  Never below what the kernel takes without the
+// edge table.
+int32_t class_limit(const nd_ensemble* en, int c, int kmethod) {
+    int32_t lim = 0;
+    for (int32_t q = en->cls_first[c + 1]; q < en->cls_first[c]; ++q) {
+        const InstDesc& I = en->inst[en->order[q]];
+        lim = std::max(lim, I.limit_bytes + (kmethod == 2 ? 8 + 8 * I.n + 3 * I.ne : 0));
+    }
+    return lim;
+}
+
+// The launches of a solve, largest instances first.  Neighbouring classes of one thread
+// count share a launch: at 512 threads a CU holds one workgroup whatever its vertices per
+// thread, and one list of instances by decreasing size ends more evenly than several
+// launches side by side.  (1024 networks of 100 to 2000 vertices, default classes, three
+// ensembles solved in turn: 46.9 ms each with a launch and a stream per class, since streams
+// beyond the four hardware queues of a process share one and their classes run one after the
+// other; 40.2 ms so.)
+struct Launch {
+    EnsKernel kernel;
+    int32_t first, count, threads, lds;
+};
+int launches(const nd_ensemble* en, int kmethod, Launch* out) {
+    int n = 0;
+    for (int c = ND_ENSEMBLE_CLASSES - 1; c >= 0;) {
+        if (en->cls_first[c] == en->cls_first[c + 1]) { --c; continue; }
+        const int32_t threads = en->cls_threads[c];
+        int32_t vper = en->cls_vper[c], lds = 0;
+        Launch l{nullptr, en->cls_first[c + 1], 0, threads, 0};
+        for (; c >= 0; --c) {
+            if (en->cls_first[c] == en->cls_first[c + 1]) continue;
+            if (en->cls_threads[c] != threads || (threads > 512 && en->cls_vper[c] != vper)) break;
+            if (en->cls_vper[c] != vper) vper = 0;
+            lds = std::max(lds, class_lds(en, c, kmethod));
+            l.count = en->cls_first[c] - l.first;
+        }
+        l.lds = lds;
+        l.kernel = pick_ensemble(en->vk.model, en->ek.model, kmethod, vper, threads);
+        out[n++] = l;
+    }
+    return n;
 }
 
 // Streams, events and the dynamic-LDS limit of every class kernel; host-side only,
@@ -925,57 +1198,55 @@ int32_t class_lds(const nd_ensemble* en, int c, int kmethod) {
 int prepare(nd_ensemble* en, int kmethod) {
     int rc = ND_OK;
     if (!en->ev_fork) rc = hip_err(hipEventCreateWithFlags(&en->ev_fork, hipEventDisableTiming), "hipEventCreate");
-    for (int c = 0; c < ND_ENSEMBLE_CLASSES && !rc; ++c) {
-        if (!en->cls_stream[c])
-            rc = hip_err(hipStreamCreateWithFlags(&en->cls_stream[c], hipStreamNonBlocking), "hipStreamCreateWithFlags");
+    for (int c = 0; c < kSideStreams && !rc; ++c) {
+        if (!en->side_stream[c])
+            rc = hip_err(hipStreamCreateWithFlags(&en->side_stream[c], hipStreamNonBlocking), "hipStreamCreateWithFlags");
         if (!rc && !en->ev_join[c])
             rc = hip_err(hipEventCreateWithFlags(&en->ev_join[c], hipEventDisableTiming), "hipEventCreate");
     }
     if (rc) return rc;
-    EnsKernel ks[ND_ENSEMBLE_CLASSES] = {};
-    int32_t lds[ND_ENSEMBLE_CLASSES] = {};
-    for (int c = 0; c < ND_ENSEMBLE_CLASSES; ++c) {
-        if (en->cls_first[c + 1] == en->cls_first[c]) continue;
-        ks[c] = pick_ensemble(en->vk.model, en->ek.model, kmethod, en->cls_vper[c], en->cls_threads[c]);
-        if (!ks[c]) return nd::set_error(ND_ERR_UNSUPPORTED, "no ensemble kernel for these models");
-        lds[c] = class_lds(en, c, kmethod);
-        if (lds[c] > en->lds_max)
+    Launch ls[ND_ENSEMBLE_CLASSES];
+    const int n = launches(en, kmethod, ls);
+    for (int c = 0; c < ND_ENSEMBLE_CLASSES; ++c)
+        if (en->cls_first[c] > en->cls_first[c + 1] && class_limit(en, c, kmethod) > en->lds_max)
             return nd::set_error(ND_ERR_UNSUPPORTED, "class %d needs %d bytes of LDS with line crossings located "
-                                 "(device limit %d)", c, lds[c], en->lds_max);
-    }
-    // one template instance may serve several classes: give it the largest need
-    for (int c = 0; c < ND_ENSEMBLE_CLASSES; ++c) {
-        if (!ks[c]) continue;
+                                 "(device limit %d)", c, class_limit(en, c, kmethod), en->lds_max);
+    // one template instance may serve several launches: give it the largest need
+    for (int i = 0; i < n; ++i) {
+        if (!ls[i].kernel) return nd::set_error(ND_ERR_UNSUPPORTED, "no ensemble kernel for these models");
         int32_t need = 0;
-        for (int d = 0; d < ND_ENSEMBLE_CLASSES; ++d)
-            if (ks[d] == ks[c]) need = std::max(need, lds[d]);
-        rc = hip_err(hipFuncSetAttribute(reinterpret_cast<const void*>(ks[c]), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         need),
+        for (int j = 0; j < n; ++j)
+            if (ls[j].kernel == ls[i].kernel) need = std::max(need, ls[j].lds);
+        rc = hip_err(hipFuncSetAttribute(reinterpret_cast<const void*>(ls[i].kernel),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, need),
                      "hipFuncSetAttribute(LDS)");
         if (rc) return rc;
     }
     return ND_OK;
 }
 
-// Fork: every non-empty class runs on its own stream after the caller's prior work;
-// join: the caller's stream waits for all of them.  Largest class first.
+// The first launch (the largest instances) runs on the caller's stream, up to three more on
+// side streams forked from it and joined back with events, any others behind the first.  All
+// launches come before the first wait, which is a barrier in the caller's hardware queue.
 int launch_classes(nd_ensemble* en, SolveArgs a, int kmethod, hipStream_t s) {
-    int rc = hip_err(hipEventRecord(en->ev_fork, s), "hipEventRecord");
-    for (int c = ND_ENSEMBLE_CLASSES - 1; c >= 0 && !rc; --c) {
-        const int32_t cnt = en->cls_first[c + 1] - en->cls_first[c];
-        if (cnt == 0) continue;
-        EnsKernel k = pick_ensemble(en->vk.model, en->ek.model, kmethod, en->cls_vper[c], en->cls_threads[c]);
-        hipStream_t cs = en->cls_stream[c];
-        rc = hip_err(hipStreamWaitEvent(cs, en->ev_fork, 0), "hipStreamWaitEvent");
+    Launch ls[ND_ENSEMBLE_CLASSES];
+    const int n = launches(en, kmethod, ls);
+    const int nside = std::min<int>(kSideStreams, n - 1);
+    int rc = nside > 0 ? hip_err(hipEventRecord(en->ev_fork, s), "hipEventRecord") : ND_OK;
+    for (int i = 0; i < n && !rc; ++i) {
+        const int side = i >= 1 && i <= nside ? i - 1 : -1;
+        hipStream_t cs = side >= 0 ? en->side_stream[side] : s;
+        if (side >= 0) rc = hip_err(hipStreamWaitEvent(cs, en->ev_fork, 0), "hipStreamWaitEvent");
         if (rc) break;
-        a.first = en->cls_first[c];
-        a.count = cnt;
-        hipLaunchKernelGGL(k, dim3(static_cast<unsigned>(cnt)), dim3(static_cast<unsigned>(en->cls_threads[c])),
-                           static_cast<unsigned>(class_lds(en, c, kmethod)), cs, a);
+        a.first = ls[i].first;
+        a.count = ls[i].count;
+        hipLaunchKernelGGL(ls[i].kernel, dim3(static_cast<unsigned>(a.count)), dim3(static_cast<unsigned>(ls[i].threads)),
+                           static_cast<unsigned>(ls[i].lds), cs, a);
         rc = hip_err(hipGetLastError(), "ensemble launch");
-        rc = rc ? rc : hip_err(hipEventRecord(en->ev_join[c], cs), "hipEventRecord");
-        rc = rc ? rc : hip_err(hipStreamWaitEvent(s, en->ev_join[c], 0), "hipStreamWaitEvent");
+        if (!rc && side >= 0) rc = hip_err(hipEventRecord(en->ev_join[side], cs), "hipEventRecord");
     }
+    for (int i = 0; i < nside && !rc; ++i)
+        rc = hip_err(hipStreamWaitEvent(s, en->ev_join[i], 0), "hipStreamWaitEvent");
     return rc;
 }
 
@@ -1008,7 +1279,8 @@ int nd_ensemble_create(int32_t ninst, const int64_t* nv, const int64_t* ne, cons
     en->vk = *vkind;
     en->ek = *ekind;
     en->dim = vkind->dim;
-    std::vector<uint16_t> ends, eix, cs, cv, cptr;
+    std::vector<uint2> tab;
+    std::vector<uint32_t> rows, hc;
     int64_t eoff = 0, uoff = 0, poff = 0;
     for (int32_t i = 0; i < ninst; ++i) {
         const int64_t n = nv[i], m = ne[i];
@@ -1029,48 +1301,57 @@ int nd_ensemble_create(int32_t ninst, const int64_t* nv, const int64_t* ne, cons
             deg[d + 1]++;
         }
         for (int64_t v = 0; v < n; ++v) deg[v + 1] += deg[v];
-        std::vector<int32_t> fill(deg.begin(), deg.end() - 1);
-        std::vector<uint16_t> le(static_cast<size_t>(2 * m));
-        for (int64_t e = 0; e < m; ++e) {
-            const int64_t s = src[eoff + e] - 1, d = dst[eoff + e] - 1;
-            le[fill[s]++] = static_cast<uint16_t>(e | 0x8000);
-            le[fill[d]++] = static_cast<uint16_t>(e);
-            ends.push_back(static_cast<uint16_t>(s));
-            ends.push_back(static_cast<uint16_t>(d));
-        }
         InstDesc I{};
         I.n = static_cast<int32_t>(n);
         I.ne = static_cast<int32_t>(m);
-        I.nslot = static_cast<int32_t>(2 * m);
         I.uoff = uoff;
         I.poff = poff;
-        I.soff = static_cast<int64_t>(eix.size());      // offset of both eix and ends (2 m entries each)
-        I.csoff = static_cast<int64_t>(cs.size());
-        I.cvoff = static_cast<int64_t>(cv.size());
-        I.cpoff = static_cast<int64_t>(cptr.size());
-
-        eix.insert(eix.end(), le.begin(), le.end());
-        int32_t nch = 0;
+        I.eoff = eoff;
+        I.toff = static_cast<int64_t>(tab.size());
+        I.voff = static_cast<int64_t>(rows.size());
+        I.hoff = static_cast<int64_t>(hc.size());
+        // rows of whole pairs; a row longer than kRowMax is cut into chunks of kChunk entries
+        std::vector<uint32_t> fill(static_cast<size_t>(n));
+        int64_t nch = 0, nhc = 0, npair = 0;
         for (int64_t v = 0; v < n; ++v) {
-            cptr.push_back(static_cast<uint16_t>(nch));
-            for (int32_t b = deg[v]; b < deg[v + 1]; b += kChunk) {
-                cs.push_back(static_cast<uint16_t>(b));
-                cv.push_back(static_cast<uint16_t>(v));
-                ++nch;
+            const uint32_t len = static_cast<uint32_t>(deg[v + 1] - deg[v]), pairs = (len + 1) / 2;
+            const uint32_t chunks = (len + kChunk - 1) / kChunk, first = static_cast<uint32_t>(npair);
+            nch += chunks;
+            fill[static_cast<size_t>(v)] = 2 * first;
+            if (len <= kRowMax) {
+                rows.push_back(first | pairs << 16);
+            } else {
+                rows.push_back(kRowHub | static_cast<uint32_t>(nhc) | chunks << 16);
+                for (uint32_t b = 0; b < pairs; b += kChunk / 2)
+                    hc.push_back((first + b) | std::min<uint32_t>(kChunk / 2, pairs - b) << 16);
+                nhc += chunks;
             }
+            npair += pairs;
         }
-        cptr.push_back(static_cast<uint16_t>(nch));
-        cs.push_back(static_cast<uint16_t>(2 * m));
-        if (nch > 65535) {
-            delete en;
-            return nd::set_error(ND_ERR_UNSUPPORTED, "instance %d: too many chunks", i);
+        const uint32_t dump = static_cast<uint32_t>(2 * (npair + kZeroPairs));
+        I.npair = static_cast<int32_t>(npair);
+        for (int64_t e = 0; e < pad_edges(static_cast<int>(m)); ++e) {
+            if (e >= m) {
+                tab.push_back(make_uint2(0, dump | dump << 16));
+                continue;
+            }
+            const uint32_t s = static_cast<uint32_t>(src[eoff + e] - 1), d = static_cast<uint32_t>(dst[eoff + e] - 1);
+            const uint32_t ps = fill[s]++, pd = fill[d]++;
+            tab.push_back(make_uint2(8 * s | (8 * d) << 16, ps | pd << 16));
         }
-        I.nchunk = nch;
+        I.nhc = static_cast<int32_t>(nhc);
         const int npe = epar(ekind->model);
-        I.lds_bytes = static_cast<int32_t>(8 * (n + m * npe + m + nch + 32) + 2 * (2 * 2 * m + 2 * nch + 1 + n + 1));
-        if (I.lds_bytes > lds_max) {
+        I.lds_bytes = static_cast<int32_t>(8 * (pad2(static_cast<int>(n)) + 2 * (npair + kZeroPairs + kDumpPairs) +
+                                                pad_edges(static_cast<int>(m)) * npe + 32 + nhc));
+        I.tab_bytes = static_cast<int32_t>(8 * pad_edges(static_cast<int>(m)) + 4 * nhc);
+        // The limit on an instance's size: 8 bytes per vertex, edge parameter, edge and 8-entry
+        // chunk of the destination lists and 2 per entry of 16-bit index tables.  An instance
+        // within it takes less without its tables: a row of odd length costs 8 bytes more than
+        // its entries and its chunks at least 4 (12 from 17 entries on) less than there
+        I.limit_bytes = static_cast<int32_t>(8 * (n + m * npe + m + nch + 32) + 2 * (2 * 2 * m + 2 * nch + 1 + n + 1));
+        if (I.limit_bytes > lds_max) {
             delete en;
-            return nd::set_error(ND_ERR_UNSUPPORTED, "instance %d needs %d bytes of LDS (device limit %d)", i, I.lds_bytes,
+            return nd::set_error(ND_ERR_UNSUPPORTED, "instance %d needs %d bytes of LDS (device limit %d)", i, I.limit_bytes,
                                  lds_max);
         }
         en->inst.push_back(I);
@@ -1082,11 +1363,9 @@ int nd_ensemble_create(int32_t ninst, const int64_t* nv, const int64_t* ne, cons
     en->total_params = poff;
     int rc = regroup(en);
     rc = rc ? rc : up(en, en->inst, &en->d_inst);
-    rc = rc ? rc : up(en, ends, &en->d_ends);
-    rc = rc ? rc : up(en, eix, &en->d_e);
-    rc = rc ? rc : up(en, cs, &en->d_cs);
-    rc = rc ? rc : up(en, cv, &en->d_cv);
-    rc = rc ? rc : up(en, cptr, &en->d_cptr);
+    rc = rc ? rc : up(en, tab, &en->d_tab);
+    rc = rc ? rc : up(en, rows, &en->d_row);
+    rc = rc ? rc : up(en, hc, &en->d_hc);
     if (rc) { delete en; return rc; }
     *out = en;
     return ND_OK;
