@@ -86,32 +86,57 @@ __device__ __forceinline__ double wave_reduce(double v, Op op) {
 // two buffers of 16 doubles in turn, and every thread combines them in wave order.  A
 // buffer is written again two reductions later, behind the barrier of the reduction in
 // between, which every thread reaches only after it has read this one.
-struct BlockRed {
-    double* red;        // 32 doubles of LDS
+// NW: the waves that contribute (the first ones), 0 for all of the launch's.
+template <int NW = 0>
+struct BlockRedN {
+    double* red;        // LDS: 32 doubles, 64 with sum2
     int turn = 0;
+    int stride = 16;    // doubles per buffer: 32 with sum2
 
+    template <typename Op>
+    __device__ __forceinline__ double combine(const double* buf, int nw, Op op) {
+        // all reads go out together; in-order combination, the same on every thread.  The
+        // result is handed over through scalar registers, so branches on it are scalar ones
+        constexpr int M = NW > 0 ? NW : 16;
+        double x[M];
+#pragma unroll
+        for (int w = 0; w < M; ++w) x[w] = buf[NW > 0 || w < nw ? w : 0];
+        double s = x[0];
+#pragma unroll
+        for (int w = 1; w < M; ++w)
+            if (NW > 0 || w < nw) s = op(s, x[w]);
+        return uniform_f64(s);
+    }
     template <typename Op>
     __device__ __forceinline__ double reduce(double v, Op op) {
         v = wave_reduce(v, op);
-        double* buf = red + 16 * turn;
+        double* buf = red + stride * turn;
         turn ^= 1;
         const int t = static_cast<int>(threadIdx.x), nw = static_cast<int>(blockDim.x) / 64;
-        if ((t & 63) == 0) buf[t / 64] = v;
+        if ((t & 63) == 0 && (NW == 0 || t < NW * 64)) buf[t / 64] = v;
         __syncthreads();
-        // all reads go out together; in-order combination, the same on every thread.  The
-        // result is handed over through scalar registers, so branches on it are scalar ones
-        double x[16];
-#pragma unroll
-        for (int w = 0; w < 16; ++w) x[w] = buf[w < nw ? w : 0];
-        double s = x[0];
-#pragma unroll
-        for (int w = 1; w < 16; ++w)
-            if (w < nw) s = op(s, x[w]);
-        return uniform_f64(s);
+        return combine(buf, nw, op);
     }
     __device__ __forceinline__ double sum(double v) { return reduce(v, SumOp{}); }
     __device__ __forceinline__ double min(double v) { return reduce(v, MinOp{}); }
     __device__ __forceinline__ double max_nan(double v) { return reduce(v, MaxNanOp{}); }
+    // two sums behind one barrier (stride 32)
+    __device__ __forceinline__ void sum2(double& v, double& w) {
+        v = wave_reduce(v, SumOp{});
+        w = wave_reduce(w, SumOp{});
+        double* buf = red + stride * turn;
+        turn ^= 1;
+        const int t = static_cast<int>(threadIdx.x), nw = static_cast<int>(blockDim.x) / 64;
+        if ((t & 63) == 0 && (NW == 0 || t < NW * 64)) {
+            buf[t / 64] = v;
+            buf[16 + t / 64] = w;
+        }
+        __syncthreads();
+        v = combine(buf, nw, SumOp{});
+        w = combine(buf + 16, nw, SumOp{});
+    }
 };
+
+using BlockRed = BlockRedN<0>;
 
 }  // namespace nd

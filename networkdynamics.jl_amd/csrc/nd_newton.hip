@@ -11,9 +11,27 @@
 // mean-zero subspace, then backtracks (halving) until the max-norm of the scaled
 // residual F_i / scale_i decreases.  Converged when max_i |F_i / scale_i| <= tol.
 //
-// On chip: theta and the CG search vector in LDS (neighbour gathers), per-vertex
-// CG vectors in registers (V vertices per thread), destination lists and weights
-// in global memory (L2 / MALL resident per grid).
+// Layout: the rows (a vertex's lines) are taken in order of decreasing length and stored in
+// slices of 64, column by column: entry j of the slice's 64 rows is one contiguous column of
+// 64, padded to the slice's longest row (a few per cent after the sort).  Every read of a
+// column is one contiguous access of its wave, and all columns' reads are independent.
+//
+// Who does what: thread t sums the rows at positions t, t + 512, ... of that order and hands
+// each result over through LDS to the thread that owns the vertex; vertices t, t + 512, ...
+// belong to thread t in the caller's order.  Vector updates and all reductions run in that
+// order, so a solve does not depend on how rows are stored.
+//
+// On chip: two vectors of the grid in LDS (theta or the CG search vector for the neighbour
+// gathers, and the row results); the first columns' weights and neighbours in the LDS that is
+// left (all of them up to about 2000 vertices), the other columns' in memory; the per-vertex CG
+// vectors in registers (V vertices per thread).
+//
+// What bounds it: a CG iteration on 5000 vertices (30000 entries) is four block barriers and
+// a gather of 8 random bytes per entry from LDS, between loads of the columns that are not
+// in LDS whose latency two waves per SIMD hide in part: 8.4 us an iteration, vector units 41 %
+// busy (450 vertices: 2.6 us).  With a row per thread read entry by entry it took 29 us.
+// Whole solves of 256 grids of 500 to 5000 vertices: 59 -> 19 ms.  Sixteen waves (the upper
+// eight only summing rows) were slower: 14.9 us, the 128 registers a wave then has spill.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -21,26 +39,30 @@
 #include <new>
 #include <vector>
 
+#include "nd_block.h"
 #include "nd_internal.h"
+#include "nd_math.h"
 
 namespace {
 
 constexpr int kWave = 64;
 constexpr int kThreads = 512;
+constexpr int kColBytes = kWave * (sizeof(double) + sizeof(uint16_t));   // one column in LDS
 
 struct GridDesc {
-    int32_t n, nslot;
-    int64_t voff;        // vertex offset (theta, P, scale)
-    int64_t roff;        // rowptr offset (n + 1 entries)
-    int64_t soff;        // slot offset
+    int32_t n, ncol;     // vertices, columns of all slices
+    int64_t voff;        // vertex offset (theta, P, scale, perm)
+    int64_t coff;        // column offset
+    int64_t soff;        // slice offset
 };
 
 struct NewtonArgs {
     const GridDesc* grid;
-    const int32_t* rowptr;   // local slot offsets
-    const int32_t* nbr;      // local neighbour
-    const int32_t* slot_edge;// global edge index of each slot
-    double* w;               // per-slot weight scratch
+    const int2* slice;       // per slice of 64 positions: {first column, columns}
+    const uint16_t* perm;    // vertex of each row position
+    const uint16_t* nbr;     // per entry: 8 x the neighbour (padding: 8 x the row's own vertex)
+    const int32_t* slot_edge;// global edge index per entry, -1 for padding
+    double* w;               // weight per entry (columns that do not fit LDS)
     double* theta;
     const double* P;
     const double* scale;
@@ -50,164 +72,234 @@ struct NewtonArgs {
     double tol, cg_rtol, eta_max;
     int32_t max_newton, cg_maxiter;
     int32_t linearized, inexact;
-    int32_t first;
+    int32_t first, lds;      // dynamic LDS of the launch
 };
 
-// max that propagates NaN (fmax drops it): a residual with a NaN entry must read as NaN,
-// never as converged
-__device__ __forceinline__ double max_nan(double a, double b) { return (b > a || b != b) ? b : a; }
+using namespace nd;
 
-__device__ __forceinline__ double block_reduce(double v, double* red, bool is_max) {
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) {
-        const double o = __shfl_xor(v, off, kWave);
-        v = is_max ? max_nan(v, o) : v + o;
-    }
-    const int t = static_cast<int>(threadIdx.x), nw = static_cast<int>(blockDim.x) / kWave;
-    if ((t & (kWave - 1)) == 0) red[t / kWave] = v;
-    __syncthreads();
-    if (t == 0) {
-        double s = red[0];
-        for (int w = 1; w < nw; ++w) s = is_max ? max_nan(s, red[w]) : s + red[w];
-        red[16] = s;
-    }
-    __syncthreads();
-    const double r = red[16];
-    __syncthreads();
-    return r;
+// a / b from y = 1.0 / b, both correctly rounded: one correction of the rounded product
+// a * y by its remainder gives the rounded quotient (Markstein 1990), with three operations
+// in place of a division's dozen
+__device__ __forceinline__ double quotient(double a, double b, double y) {
+    const double q = a * y;
+    return __builtin_fma(__builtin_fma(-q, b, a), y, q);
 }
 
 template <int V>
 __global__ void __launch_bounds__(kThreads) k_newton(NewtonArgs a) {
-    const int T = static_cast<int>(blockDim.x), t = static_cast<int>(threadIdx.x);
+    constexpr int T = kThreads, WPB = kThreads / kWave;
+    const int t = static_cast<int>(threadIdx.x), lane = t & (kWave - 1);
+    const int wv = __builtin_amdgcn_readfirstlane(t / kWave);
     const int g = a.first + static_cast<int>(blockIdx.x);
     const GridDesc G = a.grid[g];
+    const int n = G.n;
     extern __shared__ double sm[];
-    double* th = sm;            // theta (n)
-    double* pv = th + G.n;      // CG search vector (n)
-    double* red = pv + G.n;     // 32
-    const int32_t* rp = a.rowptr + G.roff;
-    const int32_t* nb = a.nbr + G.soff;
-    const int32_t* se = a.slot_edge + G.soff;
-    double* w = a.w + G.soff;
+    double* buf = sm;                          // theta or the CG search vector
+    double* rowv = buf + n;                    // row results: F, the Jacobi diagonal, L_w p
+    BlockRedN<kThreads / kWave> red{rowv + n, 0, 32};
+    // the first columns' weights and neighbours, as many as fit
+    const int cols_lds = min((a.lds - 8 * (2 * n + 64)) / kColBytes, G.ncol);
+    double* wl = rowv + n + 64 + lane;
+    uint16_t* nl = reinterpret_cast<uint16_t*>(rowv + n + 64 + cols_lds * kWave) + lane;
+    const int2* sl = a.slice + G.soff;
+    const uint16_t* nb = a.nbr + G.coff * kWave + lane;
+    const int32_t* se = a.slot_edge + G.coff * kWave + lane;
+    double* wg = a.w + G.coff * kWave + lane;
+    auto at = [&](int bytes) { return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(buf) + bytes); };
 
-    double x[V], F[V], r[V], d[V], dg[V];
-    const double* Pg = a.P + G.voff;
-    const double* scg = a.scale + G.voff;
+    for (int c = wv; c < cols_lds; c += WPB) nl[c * kWave] = nb[c * kWave];
+    // slice k of this wave, kept on lane k: {first column, columns}, columns < 0 in memory
+    static_assert(V <= kWave, "a slice per lane");
+    int2 mine = make_int2(0, 0);
+    if (lane < V && lane * T + wv * kWave < n) mine = sl[lane * WPB + wv];
+    if (mine.x + mine.y > cols_lds) mine.y = -mine.y;
+    auto slice_of = [&](int k) {
+        return make_int2(__builtin_amdgcn_readlane(mine.x, k), __builtin_amdgcn_readlane(mine.y, k));
+    };
+    // neighbours and weights of the columns c .. c + 3 of a slice, past its last column c1 that one
+    auto fetch = [&](bool mem, int c, int c1, int (&jn)[4], double (&ws)[4]) {
+        if (mem) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) jn[u] = nb[min(c + u, c1) * kWave];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) ws[u] = wg[min(c + u, c1) * kWave];
+        } else {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) jn[u] = nl[min(c + u, c1) * kWave];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) ws[u] = wl[min(c + u, c1) * kWave];
+        }
+    };
+    double* th = a.theta + G.voff;             // the accepted theta (read and written by its owners)
+    double d[V], r[V], dg[V], dgi[V];
+    int row[V];                                // vertex of the thread's rows, -1 beyond the last
 #pragma unroll
     for (int k = 0; k < V; ++k) {
         const int v = t + k * T;
-        const bool ok = v < G.n;
-        x[k] = ok ? a.theta[G.voff + v] : 0.0;
-        if (ok) th[v] = x[k];
+        row[k] = v < n ? a.perm[G.voff + v] : -1;
+        if (v < n) buf[v] = th[v];
     }
     __syncthreads();
 
-    // F(theta) for the thread's vertices from th[]; returns max |F/scale| over the grid.
-    // The library sin/cos stay here: with V residual slots unrolled, the inlined
-    // reduction of nd_math.h and its out-of-line call made the V = 10 instance spill.
-    auto residual = [&](double (&out)[V]) {
-        double m = 0.0;
-#pragma unroll
-        for (int k = 0; k < V; ++k) {
-            const int v = t + k * T;
-            out[k] = 0.0;
-            if (v < G.n) {
-                const double own = th[v];
-                double acc = 0.0;
-                if (a.linearized)
-                    for (int s = rp[v]; s < rp[v + 1]; ++s) acc += a.K[se[s]] * (th[nb[s]] - own);
-                else
-                    for (int s = rp[v]; s < rp[v + 1]; ++s) acc += a.K[se[s]] * sin(th[nb[s]] - own);
-                out[k] = Pg[v] + acc;
-                m = max_nan(m, fabs(out[k] / scg[v]));
+    // term(column, weight, theta_j - theta_i) for the entries of the thread's row k, in row
+    // order, at the theta in buf.  The next entry's loads are on their way meanwhile.
+    auto row_terms = [&](int k, double own, auto term) {
+        const int2 S = slice_of(k);
+        const int c0 = S.x, nc = abs(S.y);
+        int e1 = nc > 0 ? se[c0 * kWave] : -1;
+        int j1 = nc > 0 ? nb[c0 * kWave] : 0;
+        double k1 = e1 >= 0 ? a.K[e1] : 0.0;
+#pragma unroll 1
+        for (int j = 0; j < nc; ++j) {
+            const int jn = j1;
+            const double kv = k1;
+            if (j + 1 < nc) {
+                e1 = se[(c0 + j + 1) * kWave];
+                j1 = nb[(c0 + j + 1) * kWave];
+                k1 = e1 >= 0 ? a.K[e1] : 0.0;
             }
+            term(c0 + j, kv, at(jn) - own);
         }
-        return block_reduce(m, red, true);
     };
 
-    double res = residual(F);
+    // F(theta) of every vertex into rowv, from the theta in buf; returns max |F/scale| over the
+    // grid.  The library sin and cos, called out of line: a handful of evaluations per solve,
+    // whose registers the CG loop needs.
+    auto residual = [&]() {
+        double m = 0.0;
+#pragma unroll 1
+        for (int k = 0; k < V; ++k) {
+            if (k * T + wv * kWave >= n) break;
+            const int i = t + k * T;
+            if (i < n) {
+                const int v = a.perm[G.voff + i];
+                double acc = 0.0;
+                if (a.linearized) row_terms(k, buf[v], [&](int, double kv, double D) { acc += kv * D; });
+                else row_terms(k, buf[v], [&](int, double kv, double D) { acc += kv * sin_far(D); });
+                const double F = a.P[G.voff + v] + acc;
+                rowv[v] = F;
+                m = MaxNanOp{}(m, fabs(F / a.scale[G.voff + v]));
+            }
+        }
+        return red.max_nan(m);
+    };
+
+    double res = residual();
     int it = 0, cg_total = 0, retcode = 0;
     while (res > a.tol) {
         if (it >= a.max_newton) { retcode = 1; break; }
         ++it;
-        // weights and Jacobi diagonal at the current theta
+        double fmean = 0.0;
 #pragma unroll
         for (int k = 0; k < V; ++k) {
             const int v = t + k * T;
-            dg[k] = 1.0;
-            if (v < G.n) {
-                const double own = th[v];
+            r[k] = v < n ? rowv[v] : 0.0;
+            fmean += r[k];
+        }
+        fmean = red.sum(fmean) / n;                 // its barrier: rowv may be written again
+        // weights and Jacobi diagonal at the current theta
+#pragma unroll 1
+        for (int k = 0; k < V; ++k) {
+            if (k * T + wv * kWave >= n) break;
+            const int i = t + k * T;
+            if (i < n) {
+                const int v = a.perm[G.voff + i];
                 double dsum = 0.0;
-                for (int s = rp[v]; s < rp[v + 1]; ++s) {
-                    const double ws = a.linearized ? a.K[se[s]] : a.K[se[s]] * cos(th[nb[s]] - own);
-                    w[s] = ws;
+                const bool mem = slice_of(k).y < 0;
+                row_terms(k, buf[v], [&](int c, double kv, double D) {
+                    const double ws = a.linearized ? kv : kv * cos_far(D);
+                    if (!mem) wl[c * kWave] = ws;
+                    else wg[c * kWave] = ws;
                     dsum += ws;
-                }
-                dg[k] = dsum > 0.0 ? dsum : 1.0;
+                });
+                rowv[v] = dsum > 0.0 ? dsum : 1.0;
             }
         }
+        __syncthreads();
         // CG for L_w d = F, d mean-zero (F sums to zero when P is balanced)
-        double fmean = 0.0;
-#pragma unroll
-        for (int k = 0; k < V; ++k) if (t + k * T < G.n) fmean += F[k];
-        fmean = block_reduce(fmean, red, false) / G.n;
         double rz = 0.0, rr0 = 0.0;
 #pragma unroll
         for (int k = 0; k < V; ++k) {
+            const int v = t + k * T;
             d[k] = 0.0;
-            r[k] = (t + k * T < G.n) ? F[k] - fmean : 0.0;
-            rz += r[k] * (r[k] / dg[k]);
+            r[k] = v < n ? r[k] - fmean : 0.0;
+            dg[k] = v < n ? rowv[v] : 1.0;
+            dgi[k] = 1.0 / dg[k];
+            const double z = quotient(r[k], dg[k], dgi[k]);
+            if (v < n) buf[v] = z;
+            rz += r[k] * z;
             rr0 += r[k] * r[k];
         }
-        rz = block_reduce(rz, red, false);
-        rr0 = block_reduce(rr0, red, false);
+        red.sum2(rz, rr0);
         const double eta = a.inexact ? fmax(a.cg_rtol, fmin(a.eta_max, res)) : a.cg_rtol;
         const double stop2 = eta * eta * rr0;
         double rr = rr0;
-#pragma unroll
-        for (int k = 0; k < V; ++k) {
-            const int v = t + k * T;
-            if (v < G.n) pv[v] = r[k] / dg[k];
-        }
-        __syncthreads();
         int cg = 0;
         while (rr > stop2 && cg < a.cg_maxiter) {
             ++cg;
-            double q[V], pq = 0.0;
+            // L_w p of the thread's rows, two rows and four columns of each at a time: eight
+            // neighbours and weights are on their way together.  Columns past a row's last
+            // repeat it and are not added.
+#pragma unroll
+            for (int k = 0; k < V; k += 2) {
+                if (k * T + wv * kWave < n) {       // whole waves without rows do nothing
+                    const int2 Sa = slice_of(k), Sb = slice_of(k + 1);    // empty beyond the last slice
+                    const int na = abs(Sa.y), nb_ = abs(Sb.y), ca = Sa.x + na - 1, cb = Sb.x + nb_ - 1;
+                    const double oa = buf[max(row[k], 0)], ob = buf[max(row[k + 1], 0)];
+                    double sa = 0.0, sb = 0.0;
+                    for (int j = 0; j < max(na, nb_); j += 4) {
+                        int ja[4], jb[4];
+                        double wa[4], wb[4], pa[4], pb[4];
+                        if (j < na) fetch(Sa.y < 0, Sa.x + j, ca, ja, wa);
+                        if (j < nb_) fetch(Sb.y < 0, Sb.x + j, cb, jb, wb);
+                        if (j < na) {
+#pragma unroll
+                            for (int u = 0; u < 4; ++u) pa[u] = at(ja[u]);
+                        }
+                        if (j < nb_) {
+#pragma unroll
+                            for (int u = 0; u < 4; ++u) pb[u] = at(jb[u]);
+                        }
+#pragma unroll
+                        for (int u = 0; u < 4; ++u)
+                            if (j + u < na) sa += wa[u] * (oa - pa[u]);
+#pragma unroll
+                        for (int u = 0; u < 4; ++u)
+                            if (j + u < nb_) sb += wb[u] * (ob - pb[u]);
+                    }
+                    if (row[k] >= 0) rowv[row[k]] = sa;
+                    if (row[k + 1] >= 0) rowv[row[k + 1]] = sb;
+                }
+            }
+            __syncthreads();
+            double q[V], pi[V], pq = 0.0;
 #pragma unroll
             for (int k = 0; k < V; ++k) {
                 const int v = t + k * T;
-                q[k] = 0.0;
-                if (v < G.n) {
-                    const double pi = pv[v];
-                    double acc = 0.0;
-                    for (int s = rp[v]; s < rp[v + 1]; ++s) acc += w[s] * (pi - pv[nb[s]]);
-                    q[k] = acc;
-                    pq += pi * acc;
-                }
+                pi[k] = v < n ? buf[v] : 0.0;
+                q[k] = v < n ? rowv[v] : 0.0;
+                pq += pi[k] * q[k];
             }
-            pq = block_reduce(pq, red, false);
+            pq = red.sum(pq);
             const double alpha = rz / pq;
             double rzn = 0.0, rrn = 0.0;
 #pragma unroll
             for (int k = 0; k < V; ++k) {
-                const int v = t + k * T;
-                if (v < G.n) {
-                    d[k] += alpha * pv[v];
-                    r[k] -= alpha * q[k];
-                    rzn += r[k] * (r[k] / dg[k]);
-                    rrn += r[k] * r[k];
-                }
+                d[k] += alpha * pi[k];
+                r[k] -= alpha * q[k];
+                q[k] = quotient(r[k], dg[k], dgi[k]);
+                rzn += r[k] * q[k];
+                rrn += r[k] * r[k];
             }
-            rzn = block_reduce(rzn, red, false);
-            rr = block_reduce(rrn, red, false);
+            red.sum2(rzn, rrn);
+            rr = rrn;
             const double beta = rzn / rz;
             rz = rzn;
 #pragma unroll
             for (int k = 0; k < V; ++k) {
                 const int v = t + k * T;
-                if (v < G.n) pv[v] = r[k] / dg[k] + beta * pv[v];
+                pi[k] = q[k] + beta * pi[k];
+                if (v < n) buf[v] = pi[k];
             }
             __syncthreads();
         }
@@ -218,26 +310,22 @@ __global__ void __launch_bounds__(kThreads) k_newton(NewtonArgs a) {
 #pragma unroll
             for (int k = 0; k < V; ++k) {
                 const int v = t + k * T;
-                if (v < G.n) th[v] = x[k] + step * d[k];
+                if (v < n) buf[v] = th[v] + step * d[k];
             }
             __syncthreads();
-            nres = residual(F);
+            nres = residual();
             if (nres < res || ls == 29) break;
             step *= 0.5;
         }
 #pragma unroll
         for (int k = 0; k < V; ++k) {
-            x[k] = (t + k * T < G.n) ? x[k] + step * d[k] : 0.0;
+            const int v = t + k * T;
+            if (v < n) th[v] = th[v] + step * d[k];
         }
         if (!(nres < res)) { res = nres; retcode = 2; break; }
         res = nres;
     }
     if (!(res == res)) retcode = 3;         // a NaN residual never counts as converged
-#pragma unroll
-    for (int k = 0; k < V; ++k) {
-        const int v = t + k * T;
-        if (v < G.n) a.theta[G.voff + v] = x[k];
-    }
     if (t == 0) {
         nd_newton_stat s;
         s.residual = res;
@@ -262,8 +350,12 @@ struct nd_fixpoint {
     std::vector<int32_t> small, large;      // grid indices by class (V = 4 / V = 10)
     std::vector<void*> allocs;
     GridDesc* d_grid = nullptr;
-    int32_t *d_rp = nullptr, *d_nb = nullptr, *d_se = nullptr, *d_order = nullptr;
+    int2* d_slice = nullptr;
+    uint16_t *d_perm = nullptr, *d_nb = nullptr;
+    int32_t *d_se = nullptr, *d_order = nullptr;
     double* d_w = nullptr;
+    int lds_max = 0;
+    int32_t lds[2] = {0, 0};                // dynamic LDS of the two classes' launches
     int64_t total_vertices = 0, total_edges = 0;
     // the two size classes run on their own streams, forked from and joined back to the
     // caller's stream with events, so the large grids start while small ones still run
@@ -304,7 +396,13 @@ int nd_fixpoint_create(int32_t ngrid, const int64_t* nv, const int64_t* ne, cons
     if (!f) return nd::set_error(ND_ERR_ALLOC, "allocation failed");
     (void)hipGetDevice(&f->device);
     f->ngrid = ngrid;
-    std::vector<int32_t> rp, nb, sedge;
+    int lds_max = 0;
+    if (hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, f->device) != hipSuccess || lds_max <= 0)
+        lds_max = 64 * 1024;
+    f->lds_max = lds_max;
+    std::vector<int2> slices;
+    std::vector<uint16_t> perm, nb;
+    std::vector<int32_t> sedge;
     int64_t voff = 0, eoff = 0;
     for (int32_t gi = 0; gi < ngrid; ++gi) {
         const int64_t n = nv[gi], m = ne[gi];
@@ -314,10 +412,9 @@ int nd_fixpoint_create(int32_t ngrid, const int64_t* nv, const int64_t* ne, cons
         }
         GridDesc G{};
         G.n = static_cast<int32_t>(n);
-        G.nslot = static_cast<int32_t>(2 * m);
         G.voff = voff;
-        G.roff = static_cast<int64_t>(rp.size());
-        G.soff = static_cast<int64_t>(nb.size());
+        G.coff = static_cast<int64_t>(nb.size()) / kWave;
+        G.soff = static_cast<int64_t>(slices.size());
         std::vector<int32_t> deg(static_cast<size_t>(n) + 1, 0);
         for (int64_t e = 0; e < m; ++e) {
             const int64_t s = src[eoff + e] - 1, d = dst[eoff + e] - 1;
@@ -326,17 +423,49 @@ int nd_fixpoint_create(int32_t ngrid, const int64_t* nv, const int64_t* ne, cons
             deg[d + 1]++;
         }
         for (int64_t v = 0; v < n; ++v) deg[v + 1] += deg[v];
-        std::vector<int32_t> fill(deg.begin(), deg.end() - 1), lnb(static_cast<size_t>(2 * m)), lse(static_cast<size_t>(2 * m));
+        // rows by decreasing length (ties in vertex order), in slices of 64
+        int32_t longest = 0;
+        for (int64_t v = 0; v < n; ++v) longest = std::max(longest, deg[v + 1] - deg[v]);
+        std::vector<int32_t> first(static_cast<size_t>(longest) + 2, 0), pos(static_cast<size_t>(n));
+        for (int64_t v = 0; v < n; ++v) first[longest - (deg[v + 1] - deg[v]) + 1]++;
+        for (size_t l = 1; l < first.size(); ++l) first[l] += first[l - 1];
+        const size_t p0 = perm.size();
+        perm.resize(p0 + static_cast<size_t>(n));
+        for (int32_t v = 0; v < static_cast<int32_t>(n); ++v) {
+            pos[v] = first[longest - (deg[v + 1] - deg[v])]++;
+            perm[p0 + pos[v]] = static_cast<uint16_t>(v);
+        }
+        int32_t col = 0;
+        const size_t s0 = slices.size(), e0 = nb.size();
+        for (int32_t i = 0; i < static_cast<int32_t>(n); i += kWave) {
+            const int32_t v = perm[p0 + i], width = deg[v + 1] - deg[v];
+            slices.push_back(make_int2(col, width));
+            col += width;
+        }
+        nb.resize(e0 + static_cast<size_t>(col) * kWave);
+        sedge.resize(nb.size(), -1);
+        for (size_t s = s0; s < slices.size(); ++s)
+            for (int32_t l = 0; l < kWave; ++l) {
+                const size_t i = (s - s0) * kWave + l;
+                const uint16_t own = static_cast<uint16_t>(8 * (i < static_cast<size_t>(n) ? perm[p0 + i] : 0));
+                for (int32_t j = 0; j < slices[s].y; ++j) nb[e0 + static_cast<size_t>(slices[s].x + j) * kWave + l] = own;
+            }
+        std::vector<int32_t> fill(static_cast<size_t>(n), 0);
+        auto entry = [&](int64_t v, int64_t other, int64_t e) {
+            const int32_t i = pos[v], c = slices[s0 + i / kWave].x + fill[v]++;
+            const size_t k = e0 + static_cast<size_t>(c) * kWave + i % kWave;
+            nb[k] = static_cast<uint16_t>(8 * other);
+            sedge[k] = static_cast<int32_t>(eoff + e);
+        };
         for (int64_t e = 0; e < m; ++e) {
             const int64_t s = src[eoff + e] - 1, d = dst[eoff + e] - 1;
-            lnb[fill[s]] = static_cast<int32_t>(d);
-            lse[fill[s]++] = static_cast<int32_t>(eoff + e);
-            lnb[fill[d]] = static_cast<int32_t>(s);
-            lse[fill[d]++] = static_cast<int32_t>(eoff + e);
+            entry(s, d, e);
+            entry(d, s, e);
         }
-        rp.insert(rp.end(), deg.begin(), deg.end());
-        nb.insert(nb.end(), lnb.begin(), lnb.end());
-        sedge.insert(sedge.end(), lse.begin(), lse.end());
+        G.ncol = col;
+        // the vectors, the reduction buffers and as many columns of weights as there is room for
+        const int cls = n <= 4 * kThreads ? 0 : 1;
+        f->lds[cls] = std::max(f->lds[cls], static_cast<int32_t>(std::min<int64_t>(lds_max, 8 * (2 * n + 64) + static_cast<int64_t>(kColBytes) * col)));
         f->grids.push_back(G);
         (n <= 4 * kThreads ? f->small : f->large).push_back(gi);
         voff += n;
@@ -357,7 +486,8 @@ int nd_fixpoint_create(int32_t ngrid, const int64_t* nv, const int64_t* ne, cons
     order.insert(order.end(), f->large.begin(), f->large.end());
     int rc = upv(f, ordered, &f->d_grid);
     rc = rc ? rc : upv(f, order, &f->d_order);
-    rc = rc ? rc : upv(f, rp, &f->d_rp);
+    rc = rc ? rc : upv(f, slices, &f->d_slice);
+    rc = rc ? rc : upv(f, perm, &f->d_perm);
     rc = rc ? rc : upv(f, nb, &f->d_nb);
     rc = rc ? rc : upv(f, sedge, &f->d_se);
     if (!rc && !nb.empty()) {
@@ -382,7 +512,8 @@ int nd_fixpoint_solve(nd_fixpoint* f, double* theta, const double* P, const doub
     if (dev != f->device) return nd::set_error(ND_ERR_ARGUMENT, "solver lives on device %d", f->device);
     NewtonArgs a{};
     a.grid = f->d_grid;
-    a.rowptr = f->d_rp;
+    a.slice = f->d_slice;
+    a.perm = f->d_perm;
     a.nbr = f->d_nb;
     a.slot_edge = f->d_se;
     a.w = f->d_w;
@@ -410,12 +541,12 @@ int nd_fixpoint_solve(nd_fixpoint* f, double* theta, const double* P, const doub
     if (rc) return rc;
     size_t lds_s = 0, lds_l = 0;
     if (ns) {
-        lds_s = (2 * static_cast<size_t>(f->grids[f->small[0]].n) + 32) * sizeof(double);
+        lds_s = static_cast<size_t>(f->lds[0]);
         rc = herr(hipFuncSetAttribute(reinterpret_cast<const void*>(k_newton<4>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                       static_cast<int>(lds_s)), "hipFuncSetAttribute");
     }
     if (!rc && nl) {
-        lds_l = (2 * static_cast<size_t>(f->grids[f->large[0]].n) + 32) * sizeof(double);
+        lds_l = static_cast<size_t>(f->lds[1]);
         rc = herr(hipFuncSetAttribute(reinterpret_cast<const void*>(k_newton<10>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                       static_cast<int>(lds_l)), "hipFuncSetAttribute");
     }
@@ -427,6 +558,7 @@ int nd_fixpoint_solve(nd_fixpoint* f, double* theta, const double* P, const doub
         rc = herr(hipStreamWaitEvent(cs, f->ev_fork, 0), "hipStreamWaitEvent");
         if (rc) return rc;
         a.first = static_cast<int32_t>(ns);
+        a.lds = f->lds[1];
         hipLaunchKernelGGL(k_newton<10>, dim3(static_cast<unsigned>(nl)), dim3(kThreads), lds_l, cs, a);
         rc = herr(hipGetLastError(), "newton launch");
         rc = rc ? rc : herr(hipEventRecord(f->ev_join[1], cs), "hipEventRecord");
@@ -438,6 +570,7 @@ int nd_fixpoint_solve(nd_fixpoint* f, double* theta, const double* P, const doub
         rc = herr(hipStreamWaitEvent(cs, f->ev_fork, 0), "hipStreamWaitEvent");
         if (rc) return rc;
         a.first = 0;
+        a.lds = f->lds[0];
         hipLaunchKernelGGL(k_newton<4>, dim3(static_cast<unsigned>(ns)), dim3(kThreads), lds_s, cs, a);
         rc = herr(hipGetLastError(), "newton launch");
         rc = rc ? rc : herr(hipEventRecord(f->ev_join[0], cs), "hipEventRecord");
