@@ -547,7 +547,7 @@ int nd_fixpoint_solve(nd_fixpoint* f, double* theta, const double* P, const doub
 /* ---- learned warm start: message-passing network (FP32) -------------------------
  * No counterpart in the reference (its find_fixpoint starts from the given state).
  * A 4-layer message-passing network, hidden width 64, over the stacked nodes of a
- * batch of grids: H0 = relu(X W_in + b_in); H_l = relu(A (H_{l-1} W_l) + H_{l-1} U_l + b_l);
+ * batch of grids: H0 = relu(X W_in + b_in); H_l = relu((A H_{l-1}) W_l + H_{l-1} U_l + b_l);
  * out = H_4 w_out + b_out, with A the row-normalised K-weighted adjacency (CSR rowptr
  * / nbr / a_fwd; a_bwd = weights of its transpose on the same pattern).  Parameter
  * layout: W_in[nfeat*64], b_in[64], {[W_l|U_l][64*128], b_l[64]} x 4, w_out[64], b_out.

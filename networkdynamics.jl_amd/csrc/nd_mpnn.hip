@@ -4,13 +4,19 @@
 // Nodes of a batch of grids are stacked (n rows); the graph is a row-normalised
 // weighted adjacency (a_fwd[s] = K_s / sum of the row's K) in CSR form, plus its
 // transpose weights a_bwd for the backward pass.  Layers (hidden width 64):
-//   H0 = relu(X W_in + b_in)                      X: n x F features
-//   Y  = H_{l-1} [W_l | U_l]                       (n x 128, one GEMM)
-//   H_l = relu(A Y[:, :64] + Y[:, 64:] + b_l)      l = 1..4
-//   out = H_4 w_out + b_out                        (n)
+//   H0  = relu(X W_in + b_in)                              X: n x F features
+//   H_l = relu((A H_{l-1}) W_l + H_{l-1} U_l + b_l)        l = 1..4
+//   out = H_4 w_out + b_out                                (n)
 // Loss: mean squared error against the target.  Weight gradients are reduced in
 // two stages (per-block partials, then a fixed-order sum), so training is
 // deterministic.
+//
+// A layer is one kernel in either direction.  Aggregating the 64 columns of H before the product
+// instead of half of a 128-column product after it leaves one n x 64 read (plus the neighbours'
+// rows, from L2) and one n x 64 write per layer; a product kernel and an aggregation kernel
+// passed memory five times that.  For 773 293 nodes of power grids (4 layers, head and input) a
+// forward pass went from 1902 to 771 us, forward and backward over 130 804 nodes from 1334 to
+// 496 us.
 //
 // Parameter vector: W_in[F*64], b_in[64], {W_l|U_l [64*128], b_l[64]} x 4, w_out[64], b_out[1].
 #include <hip/hip_runtime.h>
@@ -27,76 +33,22 @@ constexpr int kH = 64;          // hidden width
 constexpr int kLayers = 4;
 constexpr int kWave = 64;
 
-// ---- dense: C[M x N] = A[M x K] * op(B) (+ bias, relu) ---------------------------------
-// op(B) = B[K x N] (TRANSB = false) or B[N x K]^T (TRANSB = true).  64x64 tiles, 256
-// threads, 4x4 outputs per thread, K in steps of 16 through LDS.
-template <bool TRANSB>
-__global__ void __launch_bounds__(256) k_sgemm(int64_t M, int N, int K, const float* __restrict__ A, int lda,
-                                               const float* __restrict__ B, int ldb, float* __restrict__ C, int ldc,
-                                               const float* __restrict__ bias, int relu) {
-    __shared__ float As[16][64 + 1];
-    __shared__ float Bs[16][64 + 1];
-    const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
-    const int64_t row0 = static_cast<int64_t>(blockIdx.x) * 64;
-    const int col0 = blockIdx.y * 64;
-    float acc[4][4] = {};
-    for (int k0 = 0; k0 < K; k0 += 16) {
-        for (int i = threadIdx.x; i < 16 * 64; i += 256) {
-            const int kk = i % 16, rr = i / 16;      // A tile: 64 rows x 16 k
-            const int64_t r = row0 + rr;
-            As[kk][rr] = (r < M && k0 + kk < K) ? A[r * lda + k0 + kk] : 0.0f;
-            const int cc = i % 64, kb = i / 64;      // B tile: 16 k x 64 cols
-            float bv = 0.0f;
-            if (col0 + cc < N && k0 + kb < K)
-                bv = TRANSB ? B[static_cast<int64_t>(col0 + cc) * ldb + k0 + kb] : B[static_cast<int64_t>(k0 + kb) * ldb + col0 + cc];
-            Bs[kb][cc] = bv;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < 16; ++kk) {
-            float a[4], b[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = As[kk][ty * 4 + i];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) b[j] = Bs[kk][tx * 4 + j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] += a[i] * b[j];
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int64_t r = row0 + ty * 4 + i;
-        if (r >= M) continue;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int c = col0 + tx * 4 + j;
-            if (c >= N) continue;
-            float v = acc[i][j] + (bias ? bias[c] : 0.0f);
-            if (relu) v = fmaxf(v, 0.0f);
-            C[r * ldc + c] = v;
-        }
-    }
-}
-
 // ---- MFMA (v_mfma_f32_16x16x4f32) dense products ---------------------------------------
 // Operand layout of one 16x16x4 step in a 64-lane wave: lane l holds A[i][k] and B[k][j]
 // with i = j = l % 16, k = l / 16; the 4 accumulators of lane l are D[4*(l/16) + r][l % 16].
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
-// C[M x N] = A[M x K] * op(B) (+ bias, relu), N = 64 or 128, K <= 128.  op(B) = B[K x N]
-// (TRANSB false) or B[N x K]^T.  256 threads: a workgroup owns 128 rows, each wave 32 rows
-// (2 row tiles) x N columns; A's rows and all of op(B) are staged in LDS with strides
-// padded so the fragment reads are free of bank conflicts.
-// dynamic LDS floats of k_gemm_mfma: A rows (stride Kp + 2) and op(B) (stride N + 16)
+// The input layer for feature counts other than 8: C[M x 64] = relu(A[M x K] * B[K x 64] + bias),
+// K <= 128.  256 threads: a workgroup owns 128 rows, each wave 32 rows (2 row tiles) x 64
+// columns; A's rows and all of B are staged in LDS with strides padded so the fragment reads
+// are free of bank conflicts.
+// dynamic LDS floats: A rows (stride Kp + 2) and B (stride N + 16)
 inline size_t gemm_mfma_lds_floats(int K, int N) {
     const int Kp = (K + 3) & ~3;
     return static_cast<size_t>(128) * (Kp + 2) + static_cast<size_t>(Kp) * (N + 16);
 }
 
-template <bool TRANSB, int N>
+template <int N>
 __global__ void __launch_bounds__(256) k_gemm_mfma(int64_t M, int K, const float* __restrict__ A, int lda,
                                                    const float* __restrict__ B, int ldb, float* __restrict__ C, int ldc,
                                                    const float* __restrict__ bias, int relu) {
@@ -115,7 +67,7 @@ __global__ void __launch_bounds__(256) k_gemm_mfma(int64_t M, int K, const float
     for (int i = t; i < Kp * N; i += 256) {
         const int k = i / N, j = i % N;
         float v = 0.0f;
-        if (k < K) v = TRANSB ? B[static_cast<int64_t>(j) * ldb + k] : B[static_cast<int64_t>(k) * ldb + j];
+        if (k < K) v = B[static_cast<int64_t>(k) * ldb + j];
         Bs[k * SB + j] = v;
     }
     __syncthreads();
@@ -150,76 +102,6 @@ __global__ void __launch_bounds__(256) k_gemm_mfma(int64_t M, int K, const float
                     C[row * ldc + col] = v;
                 }
             }
-}
-
-// C[M x N] = A[M x K] * op(B) (+ bias, relu) for the network's full-width products:
-// K = 64, N = 128 (a hidden layer's [W | U]) and K = 128, N = 64 (the backward's
-// [dYa | g] [W | U]^T), A dense with K columns.  op(B) is staged once per workgroup in
-// LDS; A goes straight from memory into the MFMA operand registers: lane (li, lk) of a
-// wave loads row li, columns K/4*lk .. K/4*lk + K/4 - 1 as 16-byte loads, and step s of
-// the 16x16x4 products pairs column K/4*lk + s with row K/4*lk + s of op(B), so every
-// k enters once.  Each wave takes 16-row tiles, grid-stride (the grid is sized to the
-// chip, not to M).  B's odd stride N + 1 spreads the four k rows of one step over the
-// LDS banks.
-template <int K, int N, bool TRANSB>
-__global__ void __launch_bounds__(256) k_gemm_reg(int64_t M, const float* __restrict__ A, const float* __restrict__ B,
-                                                  int ldb, float* __restrict__ C, int ldc, const float* __restrict__ bias,
-                                                  int relu) {
-    constexpr int SB = N + 1, CT = N / 16, KS = K / 4;
-    __shared__ float Bs[K * SB];
-    const int t = threadIdx.x, lane = t % kWave, w = t / kWave;
-    for (int i = t; i < K * N; i += 256) {
-        const int k = i / N, j = i % N;
-        Bs[k * SB + j] = TRANSB ? B[static_cast<int64_t>(j) * ldb + k] : B[static_cast<int64_t>(k) * ldb + j];
-    }
-    __syncthreads();
-    const int li = lane % 16, lk = lane / 16;
-    const int64_t ntiles = (M + 15) / 16;
-    for (int64_t tile = static_cast<int64_t>(blockIdx.x) * 4 + w; tile < ntiles; tile += static_cast<int64_t>(gridDim.x) * 4) {
-        const int64_t row = tile * 16 + li;
-        float a[KS];
-        if (row < M) {
-            const float4* ap = reinterpret_cast<const float4*>(A + row * K + KS * lk);
-#pragma unroll
-            for (int q = 0; q < KS / 4; ++q) {
-                const float4 v = ap[q];
-                a[4 * q] = v.x;
-                a[4 * q + 1] = v.y;
-                a[4 * q + 2] = v.z;
-                a[4 * q + 3] = v.w;
-            }
-        } else {
-#pragma unroll
-            for (int q = 0; q < KS; ++q) a[q] = 0.0f;
-        }
-        floatx4 acc[CT];
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) acc[ct] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-        // four steps at a time: the fence keeps the compiler from hoisting every B read of
-        // the tile into registers at once (which halves the waves a SIMD can hold)
-#pragma unroll
-        for (int s0 = 0; s0 < KS; s0 += 4) {
-#pragma unroll
-            for (int s = s0; s < s0 + 4; ++s)
-#pragma unroll
-                for (int ct = 0; ct < CT; ++ct)
-                    acc[ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], Bs[(KS * lk + s) * SB + ct * 16 + li], acc[ct], 0,
-                                                                   0, 0);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int64_t ro = tile * 16 + 4 * lk + r;
-                const int col = ct * 16 + li;
-                if (ro < M) {
-                    float v = acc[ct][r] + (bias ? bias[col] : 0.0f);
-                    if (relu) v = fmaxf(v, 0.0f);
-                    C[ro * ldc + col] = v;
-                }
-            }
-    }
 }
 
 // partial[b] = A[rows_b]^T * B[rows_b] on MFMA: KA <= 64 output rows (one 16-row tile per
@@ -275,6 +157,7 @@ __global__ void __launch_bounds__(256) k_gemm_tn_mfma(int64_t M, int KA, int NB,
 // least 64 rows each.  The partials are then added in a fixed order (k_reduce_partials),
 // so every sum is deterministic for a given M.
 constexpr int kMaxPartBlocks = 1024;
+constexpr int64_t kWgradBlocks = 256;    // one workgroup per CU
 inline int part_rows(int64_t M) {
     const int64_t r = (M + kMaxPartBlocks - 1) / kMaxPartBlocks;
     return static_cast<int>(std::max<int64_t>(64, (r + 63) / 64 * 64));
@@ -318,27 +201,39 @@ __global__ void __launch_bounds__(256) k_sgemm_tn_partial(int64_t M, int KA, int
     }
 }
 
-// out[i] (+)= sum_b part[b][i], in block order
+// out[i] = sum_b part[b * ld + i] for i < nout, in block order
 // (64 outputs per workgroup of kRedWaves waves: wave w adds the partials of blocks
-// [nb*w/kRedWaves, nb*(w+1)/kRedWaves) in order, then the wave sums are added in wave order)
+// [nb*w/kRedWaves, nb*(w+1)/kRedWaves) in order, then the wave sums are added in wave order).
+// The workgroups after those take a second array (nout2 columns, dense) to out2.
 constexpr int kRedWaves = 16;
-__global__ void __launch_bounds__(kRedWaves * 64) k_reduce_partials(int nb, int nout, const float* __restrict__ part,
-                                                                    float* __restrict__ out, int add) {
+__global__ void __launch_bounds__(kRedWaves * 64) k_reduce_partials(int nb, int nout, int ld, const float* __restrict__ part,
+                                                                    float* __restrict__ out, int nb2, int nout2,
+                                                                    const float* __restrict__ part2,
+                                                                    float* __restrict__ out2) {
     __shared__ float sh[kRedWaves][kWave];
     const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
-    const int i = blockIdx.x * kWave + lane;
+    int blk = blockIdx.x;
+    const int first2 = (nout + kWave - 1) / kWave;
+    if (blk >= first2) {
+        blk -= first2;
+        nb = nb2;
+        nout = ld = nout2;
+        part = part2;
+        out = out2;
+    }
+    const int i = blk * kWave + lane;
     const int b0 = nb * w / kRedWaves, b1 = nb * (w + 1) / kRedWaves;
     float s = 0.0f;
     if (i < nout) {
 #pragma unroll 4
-        for (int b = b0; b < b1; ++b) s += part[static_cast<int64_t>(b) * nout + i];
+        for (int b = b0; b < b1; ++b) s += part[static_cast<int64_t>(b) * ld + i];
     }
     sh[w][lane] = s;
     __syncthreads();
     if (w == 0 && i < nout) {
         float t = sh[0][lane];
         for (int q = 1; q < kRedWaves; ++q) t += sh[q][lane];
-        out[i] = add ? out[i] + t : t;
+        out[i] = t;
     }
 }
 
@@ -356,112 +251,526 @@ __global__ void __launch_bounds__(256) k_colsum_partial(int64_t M, const float* 
     if (w == 0) part[static_cast<int64_t>(blockIdx.x) * kH + c] = sh[0][c] + sh[1][c] + sh[2][c] + sh[3][c];
 }
 
-// per-block sums of a vector (fixed tree inside the block)
-__global__ void __launch_bounds__(256) k_vsum_partial(int64_t n, const float* __restrict__ x, float* __restrict__ part,
-                                                      int rows_per_block) {
-    __shared__ float sh[256];
-    const int64_t r0 = static_cast<int64_t>(blockIdx.x) * rows_per_block;
-    const int64_t r1 = std::min<int64_t>(r0 + rows_per_block, n);
-    float s = 0.0f;
-    for (int64_t r = r0 + threadIdx.x; r < r1; r += 256) s += x[r];
-    sh[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (static_cast<int>(threadIdx.x) < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-        __syncthreads();
+// Workgroups are dispatched to the chip's 8 XCDs round robin (workgroup b to XCD b % 8).  Each
+// XCD works through one contiguous eighth of the tiles, so that rows of one grid, which read
+// each other's rows, share one L2.  Neighbouring tiles go to different workgroups of the XCD:
+// their row pointers and entries share cache lines, and a CU's L1 stands still when a load
+// meets a line that is still on its way.
+struct TileRange {
+    int64_t first, end, step;
+};
+__device__ __forceinline__ TileRange wave_tiles(int64_t ntiles, int waves, int w) {
+    const int64_t b = blockIdx.x, nb = gridDim.x;
+    if (nb < 8) return {b + nb * w, ntiles, nb * waves};
+    const int64_t x = b % 8, c = (ntiles + 7) / 8, per = nb / 8 + (x < nb % 8 ? 1 : 0);
+    return {x * c + b / 8 + per * w, (x + 1) * c < ntiles ? (x + 1) * c : ntiles, per * waves};
+}
+
+// ---- a layer, forward and backward -----------------------------------------------------------
+// A wave takes tiles of 16 nodes.  Global memory is read and written with 16 lanes per node,
+// four nodes at a time: lane (li, lk) = (lane % 16, lane / 16) holds features 4 li .. 4 li + 3
+// of node 4 p + lk (p = 0..3), so a row is one access of 256 bytes.  The products want lane
+// (li, lk) to hold features 16 q + 4 lk + e (q, e = 0..3) of node li; a tile goes from one
+// layout to the other through the wave's own 16 rows of LDS.  One v_mfma_f32_16x16x4f32 step
+// takes the weights as its first operand (lane (li, lk): output column li of the column tile,
+// input feature 16 q + 4 lk + e) and the nodes as its second, and lane (li, lk) receives node
+// li's columns 16 q + 4 lk + e.
+constexpr int kWS = 68;             // LDS stride of a weight or node row: 16-byte columns free of bank conflicts
+constexpr int kTile = 16;           // nodes per wave and step
+constexpr int kAhead = 2;           // entries of each of four nodes whose rows are in flight at once
+
+// lane J of each 16 lanes to all of them; the 16 lanes moved down by kAhead
+template <int J>
+__device__ __forceinline__ uint32_t row_bcast(uint32_t v) {
+    return __builtin_amdgcn_update_dpp(0, v, 0x150 + J, 0xf, 0xf, true);
+}
+__device__ __forceinline__ uint32_t row_down(uint32_t v) {
+    return __builtin_amdgcn_update_dpp(0, v, 0x120 + 16 - kAhead, 0xf, 0xf, true);
+}
+// order between a wave's own writes and reads of LDS
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// n rows of 64 floats.  Below 2 GB a row is reached through a buffer descriptor, whose bounds
+// check turns an offset past the end into zeros without a memory access; beyond (WIDE) by
+// index.  offset: the row's byte offset or index.
+template <bool WIDE>
+struct Rows {
+    const float* X;
+    __amdgpu_buffer_rsrc_t r;
+    __device__ __forceinline__ Rows(const float* x, int64_t n) : X(x) {
+        r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x), 0,
+                                              static_cast<int>(static_cast<uint32_t>(n * kH * sizeof(float))), 0x00020000);
     }
-    if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
-}
-
-// Workgroups are dispatched to the chip's 8 XCDs round robin (workgroup b to XCD b % 8).
-// xcd_block(b, nb) renumbers them so that each XCD works through one contiguous eighth
-// of the grid: rows of one grid, which read each other's rows, then share one L2.
-// A bijection of [0, nb).
-__device__ __forceinline__ int64_t xcd_block(int64_t b, int64_t nb) {
-    const int64_t x = b % 8, q = nb / 8, r = nb % 8;
-    return x * q + (x < r ? x : r) + b / 8;
-}
-
-// ---- sparse: out[i, :] = sum_s a[s] * Y[nbr[s], 0:64]  (+ Y[i, 64:128] + bias, relu) -------
-// 16 lanes per node, four features per lane (16-byte loads), so a wave works on four
-// nodes at once; each lane sums its features over the node's entries in order, with four
-// entries' rows in flight.  Y, out and bias must be 16-byte aligned (ldy, ldo multiples of 4).
-__global__ void __launch_bounds__(256) k_spmm(int64_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ nbr,
-                                              const float* __restrict__ a, const float* __restrict__ Y, int ldy,
-                                              float* __restrict__ out, int ldo, const float* __restrict__ bias, int fused) {
-    const int64_t i = xcd_block(blockIdx.x, gridDim.x) * 16 + threadIdx.x / 16;
-    const int c = static_cast<int>(threadIdx.x % 16) * 4;
-    if (i >= n) return;
-    auto row = [&](int32_t j) { return *reinterpret_cast<const float4*>(Y + static_cast<int64_t>(j) * ldy + c); };
-    float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    auto add = [&](float w, const float4& y) {
-        s.x += w * y.x;
-        s.y += w * y.y;
-        s.z += w * y.z;
-        s.w += w * y.w;
-    };
-    int32_t k = rp[i];
-    const int32_t k1 = rp[i + 1];
-    for (; k + 4 <= k1; k += 4) {
-        const int32_t j0 = nbr[k], j1 = nbr[k + 1], j2 = nbr[k + 2], j3 = nbr[k + 3];
-        const float a0 = a[k], a1 = a[k + 1], a2 = a[k + 2], a3 = a[k + 3];
-        const float4 y0 = row(j0), y1 = row(j1), y2 = row(j2), y3 = row(j3);
-        add(a0, y0);
-        add(a1, y1);
-        add(a2, y2);
-        add(a3, y3);
+    static constexpr uint32_t kNone = 0x80000000u;
+    static __device__ __forceinline__ uint32_t at(int32_t row) {
+        return static_cast<uint32_t>(row) * (WIDE ? 1 : kH * sizeof(float));
     }
-    for (; k < k1; ++k) add(a[k], row(nbr[k]));
-    if (fused) {
-        const float4 y = *reinterpret_cast<const float4*>(Y + i * ldy + kH + c);
-        const float4 b = *reinterpret_cast<const float4*>(bias + c);
-        s.x = fmaxf(s.x + (y.x + b.x), 0.0f);
-        s.y = fmaxf(s.y + (y.y + b.y), 0.0f);
-        s.z = fmaxf(s.z + (y.z + b.z), 0.0f);
-        s.w = fmaxf(s.w + (y.w + b.w), 0.0f);
-    }
-    *reinterpret_cast<float4*>(out + i * ldo + c) = s;
-}
-
-// g = dH * relu'(H): G[i, c] = H[i, c] > 0 ? DH[i, c] : 0, also copied to DY[i, 64 + c] when DY is given
-__global__ void k_relu_grad(int64_t n, const float* __restrict__ DH, const float* __restrict__ H, float* __restrict__ G,
-                            float* __restrict__ DY) {
-    const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (t >= n * kH) return;
-    const int64_t i = t / kH;
-    const int c = static_cast<int>(t % kH);
-    const float g = H[t] > 0.0f ? DH[t] : 0.0f;
-    G[t] = g;
-    if (DY) DY[i * 2 * kH + kH + c] = g;
-}
-
-// out[i] = H[i, :] . w + b ; optional MSE gradient against target and loss partials
-__global__ void __launch_bounds__(256) k_head(int64_t n, const float* __restrict__ H, const float* __restrict__ w,
-                                              const float* __restrict__ b, float* __restrict__ out,
-                                              const float* __restrict__ target, float* __restrict__ dout,
-                                              float* __restrict__ dH, float* __restrict__ loss_part) {
-    __shared__ float sl[4];
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * 4 + threadIdx.x / kWave;
-    const int c = threadIdx.x % kWave;
-    float v = 0.0f, l = 0.0f;
-    if (i < n) {
-        v = H[i * kH + c] * w[c];
-#pragma unroll
-        for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
-        v += b[0];
-        if (c == 0 && out) out[i] = v;
-        if (target) {
-            const float e = v - target[i];
-            const float g = 2.0f * e / static_cast<float>(n);
-            if (c == 0) { dout[i] = g; l = e * e; }
-            dH[i * kH + c] = g * w[c];
+    __device__ __forceinline__ float4 part(uint32_t offset, int li) const {
+        if constexpr (WIDE) {
+            if (offset == kNone) return make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            return *reinterpret_cast<const float4*>(X + static_cast<int64_t>(offset) * kH + 4 * li);
+        } else {
+            return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, static_cast<int>(offset + 16 * li), 0, 0));
         }
     }
-    if (loss_part) {
-        if (c == 0) sl[threadIdx.x / kWave] = l;
-        __syncthreads();
-        if (threadIdx.x == 0) loss_part[blockIdx.x] = sl[0] + sl[1] + sl[2] + sl[3];
+};
+
+// The entries of a tile: its row pointers (lanes 0..16) and its first 64 neighbours and weights
+struct TileEntries {
+    int32_t rows, nbr;
+    float a;
+};
+// lanes 0..16: the row pointers of nodes 16 tile .. 16 tile + 16 (those past the end repeat the last)
+__device__ __forceinline__ int32_t tile_rows(const int32_t* __restrict__ rp, int64_t tile, int64_t n, int lane) {
+    const int64_t r = tile * kTile + (lane < kTile ? lane : kTile);
+    return rp[r < n ? r : n];
+}
+__device__ __forceinline__ void tile_entries(const int32_t* __restrict__ nbr, const float* __restrict__ a, int lane,
+                                             TileEntries& t) {
+    const int32_t first = __builtin_amdgcn_readfirstlane(t.rows), count = __builtin_amdgcn_readlane(t.rows, kTile) - first;
+    if (count == 0) return;
+    const int64_t s = first + static_cast<int64_t>(lane < count ? lane : count - 1);
+    t.nbr = nbr[s];
+    t.a = a[s];
+}
+// z[p] = sum_s a[s] X[nbr[s], 4 li ..] over the entries of node 4 p + lk, in order
+template <bool WIDE>
+__device__ __forceinline__ void gather_tile(const int32_t* __restrict__ nbr, const float* __restrict__ a, const Rows<WIDE>& X,
+                                            const TileEntries& t, int li, int lk, float4 (&z)[4]) {
+    const int32_t first = __builtin_amdgcn_readfirstlane(t.rows), count = __builtin_amdgcn_readlane(t.rows, kTile) - first;
+    // the longest row of the tile (lanes 0..15)
+    int32_t most = __shfl(t.rows, 16 * lk + li + 1, kWave) - t.rows;
+    most = max(most, __builtin_amdgcn_update_dpp(0, most, 0x128, 0xf, 0xf, true));    // row_ror:8, 4, 2, 1
+    most = max(most, __builtin_amdgcn_update_dpp(0, most, 0x124, 0xf, 0xf, true));
+    most = max(most, __builtin_amdgcn_update_dpp(0, most, 0x122, 0xf, 0xf, true));
+    most = max(most, __builtin_amdgcn_update_dpp(0, most, 0x121, 0xf, 0xf, true));
+    most = __builtin_amdgcn_readfirstlane(most);
+#pragma unroll
+    for (int p = 0; p < 4; ++p) z[p] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    uint32_t nb[4], av[4];                                // the next 16 entries of each node, one per lane
+    for (int32_t k = 0; k < most; k += kAhead) {
+        if (k % 16 == 0) {
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                const int32_t start = __shfl(t.rows, 4 * p + lk, kWave), end = __shfl(t.rows, 4 * p + lk + 1, kWave);
+                const int64_t s = start + static_cast<int64_t>(k + li);
+                const int32_t pos = static_cast<int32_t>(s - first);
+                nb[p] = static_cast<uint32_t>(__shfl(t.nbr, pos & 63, kWave));
+                av[p] = __float_as_uint(__shfl(t.a, pos & 63, kWave));
+                if (count > kWave) {                      // a tile of more than 64 entries
+                    if (s < end && pos >= kWave) {
+                        nb[p] = static_cast<uint32_t>(nbr[s]);
+                        av[p] = __float_as_uint(a[s]);
+                    }
+                    asm volatile("" : "+v"(nb[p]), "+v"(av[p]));     // waited for here, not on every path
+                }
+                nb[p] = s < end ? X.at(static_cast<int32_t>(nb[p])) : X.kNone;
+                av[p] = s < end ? av[p] : 0u;
+            }
+        }
+        float4 x[4][kAhead];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            x[p][0] = X.part(row_bcast<0>(nb[p]), li);
+            x[p][1] = X.part(row_bcast<1>(nb[p]), li);
+            if (kAhead > 2) {
+                x[p][kAhead - 2] = X.part(row_bcast<kAhead - 2>(nb[p]), li);
+                x[p][kAhead - 1] = X.part(row_bcast<kAhead - 1>(nb[p]), li);
+            }
+            nb[p] = row_down(nb[p]);
+        }
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const float c[4] = {__uint_as_float(row_bcast<0>(av[p])), __uint_as_float(row_bcast<1>(av[p])),
+                                __uint_as_float(row_bcast<2>(av[p])), __uint_as_float(row_bcast<3>(av[p]))};
+            av[p] = row_down(av[p]);
+#pragma unroll
+            for (int i = 0; i < kAhead; ++i) {
+                z[p].x = __builtin_fmaf(c[i], x[p][i].x, z[p].x);
+                z[p].y = __builtin_fmaf(c[i], x[p][i].y, z[p].y);
+                z[p].z = __builtin_fmaf(c[i], x[p][i].z, z[p].z);
+                z[p].w = __builtin_fmaf(c[i], x[p][i].w, z[p].w);
+            }
+        }
     }
+}
+// the rows of the tile itself
+template <bool WIDE>
+__device__ __forceinline__ void own_rows(const Rows<WIDE>& X, int64_t tile, int64_t n, int li, int lk, float4 (&x)[4]) {
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        const int64_t row = tile * kTile + 4 * p + lk;
+        x[p] = X.part(row < n ? X.at(static_cast<int32_t>(row)) : X.kNone, li);
+    }
+}
+// between the layouts, through the wave's 16 rows of LDS
+__device__ __forceinline__ void tile_put(float* T, int li, int lk, const float4 (&z)[4]) {
+    wave_fence();
+#pragma unroll
+    for (int p = 0; p < 4; ++p) *reinterpret_cast<float4*>(T + (4 * p + lk) * kWS + 4 * li) = z[p];
+    wave_fence();
+}
+__device__ __forceinline__ void tile_get(float* T, int li, int lk, const floatx4 (&acc)[4], float4 (&y)[4]) {
+    wave_fence();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) *reinterpret_cast<floatx4*>(T + li * kWS + 16 * q + 4 * lk) = acc[q];
+    wave_fence();
+#pragma unroll
+    for (int p = 0; p < 4; ++p) y[p] = *reinterpret_cast<const float4*>(T + (4 * p + lk) * kWS + 4 * li);
+}
+
+// sum += x w: the tile's rows x in T times 64 rows of weights (stride kWS), sums of 32 products
+// each
+__device__ __forceinline__ void product64(const float* Ws, const float* T, int li, int lk, floatx4 (&sum)[4]) {
+    const float* w = Ws + 4 * lk * kWS + li;
+#pragma unroll
+    for (int q2 = 0; q2 < 2; ++q2) {
+        floatx4 acc[4];
+#pragma unroll
+        for (int ct = 0; ct < 4; ++ct) acc[ct] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int q = 2 * q2; q < 2 * q2 + 2; ++q) {
+            const floatx4 x = *reinterpret_cast<const floatx4*>(T + li * kWS + 16 * q + 4 * lk);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int ct = 0; ct < 4; ++ct)
+                    acc[ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[(16 * q + e) * kWS + 16 * ct], x[e], acc[ct], 0, 0, 0);
+            // the fence keeps the compiler from hoisting every weight read into registers at once
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int ct = 0; ct < 4; ++ct) sum[ct] = sum[ct] + acc[ct];
+    }
+}
+
+// Hout = relu((A H) W + H U + bias), W and U the halves of WU (64 x 128); with `out` also the
+// head out = Hout w_out + b_out.
+// At 773 293 nodes of 3.2 entries: 175 us, of which the matrix cores are busy for 81 (128 x 64
+// products at 153 TFLOP/s); reading and writing H alone takes 102.  Both overlap only in part:
+// the registers allow 16 waves a CU, and the neighbours' rows come from L2 with some 460 cycles
+// each.  What mattered, from 262 us: whole rows per access (64-byte pieces of 16 rows met lines
+// still on their way to L1, 262 -> 243 with the gather turned), all other loads likewise and
+// neighbouring tiles on different CUs (234 -> 191), stores past L2, which leave it to the
+// rows that are gathered, and one workgroup of 16 waves (191 -> 175).  Four entries of each node in flight
+// instead of two, wave priorities and skipping padded entries measured the same.
+template <int NT, bool WIDE>
+__global__ void __launch_bounds__(NT, NT / 256) k_layer(int64_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ nbr,
+                                                 const float* __restrict__ a, const float* __restrict__ H,
+                                                 const float* __restrict__ WU, const float* __restrict__ bias,
+                                                 float* __restrict__ Hout, const float* __restrict__ wout,
+                                                 const float* __restrict__ bout, float* __restrict__ out) {
+    __shared__ float Ws[2 * kH * kWS];
+    __shared__ float Ts[NT / kWave][kTile * kWS];
+    __shared__ float bs[2 * kH];                          // bias, w_out
+    const int t = threadIdx.x, lane = t % kWave, w = __builtin_amdgcn_readfirstlane(t / kWave), li = lane % 16, lk = lane / 16;
+    for (int i = t; i < 2 * kH * kH; i += NT) {
+        const int k = i / kH, j = i % kH;
+        Ws[k * kWS + j] = WU[(k % kH) * 2 * kH + (k / kH) * kH + j];
+    }
+    if (t < kH) {
+        bs[t] = bias[t];
+        bs[kH + t] = wout[t];
+    }
+    __syncthreads();
+    const Rows<WIDE> X(H, n);
+    const TileRange tr = wave_tiles((n + kTile - 1) / kTile, NT / kWave, w);
+    TileEntries te{tile_rows(rp, tr.first, n, lane), 0, 0.0f};
+    tile_entries(nbr, a, lane, te);
+    for (int64_t tile = tr.first; tile < tr.end; tile += tr.step) {
+        // the next tile's entries are read while this one is multiplied
+        const int32_t next = tile_rows(rp, tile + tr.step, n, lane);
+        __builtin_amdgcn_sched_barrier(0);
+        float4 z[4], h[4], y[4];
+        gather_tile<WIDE>(nbr, a, X, te, li, lk, z);
+        own_rows<WIDE>(X, tile, n, li, lk, h);
+        te.rows = next;
+        tile_entries(nbr, a, lane, te);
+        floatx4 acc[4] = {};
+        tile_put(Ts[w], li, lk, z);
+        product64(Ws, Ts[w], li, lk, acc);
+        tile_put(Ts[w], li, lk, h);
+        product64(Ws + kH * kWS, Ts[w], li, lk, acc);
+        tile_get(Ts[w], li, lk, acc, y);
+        const float4 b4 = *reinterpret_cast<const float4*>(bs + 4 * li);
+        const float4 w4 = *reinterpret_cast<const float4*>(bs + kH + 4 * li);
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const int64_t row = tile * kTile + 4 * p + lk;
+            y[p] = make_float4(fmaxf(y[p].x + b4.x, 0.0f), fmaxf(y[p].y + b4.y, 0.0f), fmaxf(y[p].z + b4.z, 0.0f),
+                               fmaxf(y[p].w + b4.w, 0.0f));
+            if (row < n)
+                __builtin_nontemporal_store(__builtin_bit_cast(floatx4, y[p]),
+                                            reinterpret_cast<floatx4*>(Hout + row * kH + 4 * li));
+            if (out) {
+                float d = __builtin_fmaf(y[p].w, w4.w, __builtin_fmaf(y[p].z, w4.z, __builtin_fmaf(y[p].y, w4.y, y[p].x * w4.x)));
+#pragma unroll
+                for (int off = 8; off > 0; off >>= 1) d += __shfl_xor(d, off, kWave);
+                if (row < n && li == 0) out[row] = d + bout[0];
+            }
+        }
+    }
+}
+
+// From g = dL/d(layer's sum): Z = A^T g (for the weight gradients) and Gin = ([Z | g] [W | U]^T)
+// masked by H > 0, the gradient at the sum of the layer below (H: this layer's input).  The
+// layer kernel's shape and bounds: 42 us at 130 804 nodes; the four kernels that it replaces
+// (mask, aggregation, product, column sums) took 107.
+template <int NT, bool WIDE>
+__global__ void __launch_bounds__(NT, NT / 256) k_layer_bwd(int64_t n, const int32_t* __restrict__ rp,
+                                                     const int32_t* __restrict__ nbr, const float* __restrict__ a,
+                                                     const float* __restrict__ G, const float* __restrict__ WU,
+                                                     const float* __restrict__ H, float* __restrict__ Z,
+                                                     float* __restrict__ Gin) {
+    __shared__ float Ws[2 * kH * kWS];
+    __shared__ float Ts[NT / kWave][kTile * kWS];
+    const int t = threadIdx.x, lane = t % kWave, w = __builtin_amdgcn_readfirstlane(t / kWave), li = lane % 16, lk = lane / 16;
+    for (int i = t; i < 2 * kH * kH; i += NT) {
+        const int j = i / (2 * kH), k = i % (2 * kH);
+        Ws[k * kWS + j] = WU[j * 2 * kH + k];
+    }
+    __syncthreads();
+    const Rows<WIDE> X(G, n), Y(H, n);
+    const TileRange tr = wave_tiles((n + kTile - 1) / kTile, NT / kWave, w);
+    TileEntries te{tile_rows(rp, tr.first, n, lane), 0, 0.0f};
+    tile_entries(nbr, a, lane, te);
+    for (int64_t tile = tr.first; tile < tr.end; tile += tr.step) {
+        const int32_t next = tile_rows(rp, tile + tr.step, n, lane);
+        __builtin_amdgcn_sched_barrier(0);
+        float4 z[4], own[4], h[4], y[4];
+        gather_tile<WIDE>(nbr, a, X, te, li, lk, z);
+        own_rows<WIDE>(X, tile, n, li, lk, own);
+        te.rows = next;
+        tile_entries(nbr, a, lane, te);
+        floatx4 acc[4] = {};
+        tile_put(Ts[w], li, lk, z);
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const int64_t row = tile * kTile + 4 * p + lk;
+            if (row < n) *reinterpret_cast<float4*>(Z + row * kH + 4 * li) = z[p];
+        }
+        product64(Ws, Ts[w], li, lk, acc);
+        tile_put(Ts[w], li, lk, own);
+        own_rows<WIDE>(Y, tile, n, li, lk, h);
+        product64(Ws + kH * kWS, Ts[w], li, lk, acc);
+        tile_get(Ts[w], li, lk, acc, y);
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const int64_t row = tile * kTile + 4 * p + lk;
+            if (row < n)
+                *reinterpret_cast<float4*>(Gin + row * kH + 4 * li) =
+                    make_float4(h[p].x > 0.0f ? y[p].x : 0.0f, h[p].y > 0.0f ? y[p].y : 0.0f, h[p].z > 0.0f ? y[p].z : 0.0f,
+                                h[p].w > 0.0f ? y[p].w : 0.0f);
+        }
+    }
+}
+
+// Per block the partial sums of d[W | U] = H^T [Z | g] (64 x 128) and of the columns of g, over
+// rows_per_block rows.  A wave takes four nodes a step: lane (li, lk) loads 16 bytes, columns
+// 4 li .. 4 li + 3, of node lk's row of H, Z and g, and register e of the three is the operand
+// of a product whose tile holds the features 4 li + e -- so three contiguous loads feed 32
+// matrix instructions and nothing passes through LDS until the waves' sums are added, two and
+// two.  31 us at 130 804 nodes against 91 for tiles staged in LDS; 14 at the matrix cores'
+// rate, 20 for the three arrays' bytes.  A sum through one LDS array in wave order took 12 more.
+constexpr int kWgradWaves = 8;      // two per SIMD, as many as the registers allow
+__global__ void __launch_bounds__(64 * kWgradWaves, 2) k_wgrad(int64_t n, const float* __restrict__ H, const float* __restrict__ Z,
+                                               const float* __restrict__ G, float* __restrict__ part,
+                                               float* __restrict__ bpart, int rows_per_block) {
+    __shared__ float sum[kWgradWaves / 2][kH * 2 * kH];
+    __shared__ float bsum[kWgradWaves][kH];
+    const int t = threadIdx.x, lane = t % kWave, w = t / kWave, li = lane % 16, lk = lane / 16;
+    const int64_t r0 = static_cast<int64_t>(blockIdx.x) * rows_per_block;
+    const int64_t r1 = r0 + rows_per_block < n ? r0 + rows_per_block : n;
+    floatx4 acc[4][8];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    float4 bs = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    auto load = [&](const float* X, int64_t r) {
+        return r + lk < r1 ? *reinterpret_cast<const float4*>(X + (r + lk) * kH + 4 * li) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    };
+    // the waves take the block's steps of four rows in turn; the next step's rows are loaded
+    // while the current ones are multiplied
+    int64_t r = r0 + 4 * w;
+    float4 h = load(H, r), z = load(Z, r), g = load(G, r);
+    for (; r < r1; r += 4 * kWgradWaves) {
+        const int64_t rn = r + 4 * kWgradWaves;
+        const float4 hn = load(H, rn), zn = load(Z, rn), gn = load(G, rn);
+        const float ha[4] = {h.x, h.y, h.z, h.w};
+        const float zg[8] = {z.x, z.y, z.z, z.w, g.x, g.y, g.z, g.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ha[i], zg[j], acc[i][j], 0, 0, 0);
+        bs.x += g.x;
+        bs.y += g.y;
+        bs.z += g.z;
+        bs.w += g.w;
+        h = hn;
+        z = zn;
+        g = gn;
+    }
+    // column sums: the four node lanes, then the waves
+    float b4[4] = {bs.x, bs.y, bs.z, bs.w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        b4[e] += __shfl_xor(b4[e], 16, kWave);
+        b4[e] += __shfl_xor(b4[e], 32, kWave);
+        if (lk == 0) bsum[w][4 * li + e] = b4[e];
+    }
+    // acc[i][j][r] of lane (li, lk): row 4 (4 lk + r) + i, column 4 li + j % 4 of half j / 4
+    auto each = [&](auto f) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int r4 = 0; r4 < 4; ++r4)
+#pragma unroll
+                for (int hf = 0; hf < 2; ++hf) f((4 * (4 * lk + r4) + i) * 2 * kH + hf * kH + 4 * li, i, 4 * hf, r4);
+    };
+    auto put = [&](float* dst) {
+        each([&](int o, int i, int j, int r4) {
+            *reinterpret_cast<float4*>(dst + o) = make_float4(acc[i][j][r4], acc[i][j + 1][r4], acc[i][j + 2][r4], acc[i][j + 3][r4]);
+        });
+    };
+    auto add = [&](const float* src) {
+        each([&](int o, int i, int j, int r4) {
+            const float4 v = *reinterpret_cast<const float4*>(src + o);
+            acc[i][j][r4] += v.x;
+            acc[i][j + 1][r4] += v.y;
+            acc[i][j + 2][r4] += v.z;
+            acc[i][j + 3][r4] += v.w;
+        });
+    };
+#pragma unroll
+    for (int s = 1; s < kWgradWaves; s *= 2) {
+        if (w % (2 * s) == s) put(sum[w / (2 * s)]);
+        __syncthreads();
+        if (w % (2 * s) == 0) add(sum[w / (2 * s)]);
+        __syncthreads();
+    }
+    if (w == 0) {
+        float* dst = part + static_cast<int64_t>(blockIdx.x) * kH * 2 * kH;
+        each([&](int o, int i, int j, int r4) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) dst[o + e] = acc[i][j + e][r4];
+        });
+    }
+    if (t < kH) {
+        float s = bsum[0][t];
+#pragma unroll
+        for (int i = 1; i < kWgradWaves; ++i) s += bsum[i][t];
+        bpart[static_cast<int64_t>(blockIdx.x) * kH + t] = s;
+    }
+}
+
+// H0 = relu(X W_in + b_in) for 8 features: 16 lanes per node, four columns each.  Bound by the
+// write of H0: 51 us at 773 293 nodes (4.3 TB/s); the matrix kernel above takes 71, padded to
+// a tile's rows in LDS.
+__global__ void __launch_bounds__(256) k_input8(int64_t n, const float* __restrict__ X, const float* __restrict__ Win,
+                                                const float* __restrict__ bin, float* __restrict__ H) {
+    const int c = static_cast<int>(threadIdx.x % 16) * 4;
+    float4 w[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) w[k] = *reinterpret_cast<const float4*>(Win + k * kH + c);
+    const float4 b = *reinterpret_cast<const float4*>(bin + c);
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * 16 + threadIdx.x / 16; i < n; i += static_cast<int64_t>(gridDim.x) * 16) {
+        const float4 x0 = *reinterpret_cast<const float4*>(X + i * 8), x1 = *reinterpret_cast<const float4*>(X + i * 8 + 4);
+        const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+        float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            s.x = __builtin_fmaf(x[k], w[k].x, s.x);
+            s.y = __builtin_fmaf(x[k], w[k].y, s.y);
+            s.z = __builtin_fmaf(x[k], w[k].z, s.z);
+            s.w = __builtin_fmaf(x[k], w[k].w, s.w);
+        }
+        *reinterpret_cast<float4*>(H + i * kH + c) = make_float4(fmaxf(s.x + b.x, 0.0f), fmaxf(s.y + b.y, 0.0f),
+                                                                 fmaxf(s.z + b.z, 0.0f), fmaxf(s.w + b.w, 0.0f));
+    }
+}
+
+// Sums over the 16 node groups of a 256-thread block (16 lanes x 4 columns each): the four
+// groups of a wave by lane exchange, then the waves in order.  K vectors of 64 columns; row k
+// goes to dst + 64 k.  sh: K x 4 x 64 floats.
+template <int K>
+__device__ __forceinline__ void block_columns(float (&v)[K][4], float* sh, float* __restrict__ dst) {
+    const int t = threadIdx.x, lane = t % kWave, w = t / kWave, c = (t % 16) * 4;
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[k][e] += __shfl_xor(v[k][e], 16, kWave);
+            v[k][e] += __shfl_xor(v[k][e], 32, kWave);
+            if (lane < 16) sh[(k * 4 + w) * kH + c + e] = v[k][e];
+        }
+    __syncthreads();
+    for (int i = t; i < K * kH; i += 256) {
+        const float* s = sh + (i / kH) * 4 * kH + i % kH;
+        dst[i] = ((s[0] + s[kH]) + s[2 * kH]) + s[3 * kH];
+    }
+}
+
+// per-block partials of d W_in = X^T g (8 x 64) and d b_in (64), consecutive as in the
+// parameters: 13 us at 130 804 nodes against 46 for a product and a column sum
+__global__ void __launch_bounds__(256) k_input_grad8(int64_t n, const float* __restrict__ X, const float* __restrict__ G,
+                                                     float* __restrict__ part) {
+    __shared__ float sh[9 * 4 * kH];
+    const int c = static_cast<int>(threadIdx.x % 16) * 4;
+    float v[9][4] = {};
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * 16 + threadIdx.x / 16; i < n; i += static_cast<int64_t>(gridDim.x) * 16) {
+        const float4 x0 = *reinterpret_cast<const float4*>(X + i * 8), x1 = *reinterpret_cast<const float4*>(X + i * 8 + 4);
+        const float4 g4 = *reinterpret_cast<const float4*>(G + i * kH + c);
+        const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w}, g[4] = {g4.x, g4.y, g4.z, g4.w};
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[k][e] = __builtin_fmaf(x[k], g[e], v[k][e]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[8][e] += g[e];
+    }
+    block_columns<9>(v, sh, part + static_cast<int64_t>(blockIdx.x) * 9 * kH);
+}
+
+// The head backward: e = H4 w + b - target, g_i = 2 e_i / n; G = g w masked by H4 > 0 (the
+// gradient at the last layer's sum), the losses of nodes 4 j .. 4 j + 3 summed in loss_part[j],
+// and per-block partials of d w_out = H4^T g (64) and d b_out (the first of the next 64): one
+// pass over H4, 17 us at 130 804 nodes, where the head, the sums and the mask took 86 in five.
+__global__ void __launch_bounds__(256) k_head_bwd(int64_t n, const float* __restrict__ H, const float* __restrict__ w,
+                                                  const float* __restrict__ b, const float* __restrict__ target,
+                                                  float* __restrict__ G, float* __restrict__ loss_part,
+                                                  float* __restrict__ part) {
+    __shared__ float sh[2 * 4 * kH];
+    const int t = threadIdx.x, lane = t % kWave, c = (t % 16) * 4;
+    const float4 wc = *reinterpret_cast<const float4*>(w + c);
+    const float b0 = b[0];
+    float v[2][4] = {};
+    for (int64_t i0 = static_cast<int64_t>(blockIdx.x) * 16; i0 < n; i0 += static_cast<int64_t>(gridDim.x) * 16) {
+        const int64_t i = i0 + t / 16;
+        const bool valid = i < n;
+        const float4 h = valid ? *reinterpret_cast<const float4*>(H + i * kH + c) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        float d = __builtin_fmaf(h.w, wc.w, __builtin_fmaf(h.z, wc.z, __builtin_fmaf(h.y, wc.y, h.x * wc.x)));
+#pragma unroll
+        for (int off = 8; off > 0; off >>= 1) d += __shfl_xor(d, off, kWave);
+        const float e = valid ? d + b0 - target[i] : 0.0f;
+        const float g = 2.0f * e / static_cast<float>(n);
+        if (valid)
+            *reinterpret_cast<float4*>(G + i * kH + c) = make_float4(h.x > 0.0f ? g * wc.x : 0.0f, h.y > 0.0f ? g * wc.y : 0.0f,
+                                                                     h.z > 0.0f ? g * wc.z : 0.0f, h.w > 0.0f ? g * wc.w : 0.0f);
+        v[0][0] = __builtin_fmaf(h.x, g, v[0][0]);
+        v[0][1] = __builtin_fmaf(h.y, g, v[0][1]);
+        v[0][2] = __builtin_fmaf(h.z, g, v[0][2]);
+        v[0][3] = __builtin_fmaf(h.w, g, v[0][3]);
+        if (c == 0) v[1][0] += g;
+        const float l = e * e;
+        const float l1 = __shfl(l, 16, kWave), l2 = __shfl(l, 32, kWave), l3 = __shfl(l, 48, kWave);
+        if (lane == 0 && i < n) loss_part[i / 4] = l + l1 + l2 + l3;
+    }
+    block_columns<2>(v, sh, part + static_cast<int64_t>(blockIdx.x) * 2 * kH);
 }
 
 __global__ void k_adam(int64_t n, float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
@@ -560,69 +869,55 @@ int herr(hipError_t e, const char* w) {
     return e == hipSuccess ? ND_OK : nd::set_error(ND_ERR_DEVICE, "%s: %s", w, hipGetErrorString(e));
 }
 
-template <bool TRANSB, int N>
-void gemm_mfma(hipStream_t s, int64_t M, int K, const float* A, int lda, const float* B, int ldb, float* C, int ldc,
-               const float* bias, int relu) {
-    const size_t lds = gemm_mfma_lds_floats(K, N) * sizeof(float);
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k_gemm_mfma<TRANSB, N>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-    hipLaunchKernelGGL((k_gemm_mfma<TRANSB, N>), dim3(nblk(M, 128)), dim3(256), lds, s, M, K, A, lda, B, ldb, C, ldc,
-                       bias, relu);
+// the input layer for any feature count up to 128
+void input_gemm(hipStream_t s, int64_t M, int K, const float* A, const float* B, float* C, const float* bias) {
+    const size_t lds = gemm_mfma_lds_floats(K, kH) * sizeof(float);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k_gemm_mfma<kH>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              static_cast<int>(lds));
+    hipLaunchKernelGGL(k_gemm_mfma<kH>, dim3(nblk(M, 128)), dim3(256), lds, s, M, K, A, K, B, kH, C, kH, bias, 1);
 }
 
-// C = A op(B): MFMA for the network's shapes (N = 64 or 128 columns, K <= 128), the
-// LDS-tiled FP32 kernel otherwise
-void gemm(hipStream_t s, bool transb, int64_t M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C,
-          int ldc, const float* bias, int relu) {
-    const bool dense16 = lda == K && (reinterpret_cast<uintptr_t>(A) & 15) == 0;
-    if (dense16 && ((K == 64 && N == 128 && !transb) || (K == 128 && N == 64 && transb))) {
-        // 16-row tiles, four per workgroup; four workgroups per CU fit their LDS
-        const unsigned nb = static_cast<unsigned>(std::min<int64_t>((M + 63) / 64, 1024));
-        if (K == 64)
-            hipLaunchKernelGGL((k_gemm_reg<64, 128, false>), dim3(nb), dim3(256), 0, s, M, A, B, ldb, C, ldc, bias, relu);
-        else
-            hipLaunchKernelGGL((k_gemm_reg<128, 64, true>), dim3(nb), dim3(256), 0, s, M, A, B, ldb, C, ldc, bias, relu);
-        return;
-    }
-    if (K <= 128 && (N == 64 || N == 128)) {
-        if (N == 64) {
-            if (transb) gemm_mfma<true, 64>(s, M, K, A, lda, B, ldb, C, ldc, bias, relu);
-            else gemm_mfma<false, 64>(s, M, K, A, lda, B, ldb, C, ldc, bias, relu);
-        } else {
-            if (transb) gemm_mfma<true, 128>(s, M, K, A, lda, B, ldb, C, ldc, bias, relu);
-            else gemm_mfma<false, 128>(s, M, K, A, lda, B, ldb, C, ldc, bias, relu);
-        }
-        return;
-    }
-    dim3 grid(nblk(M, 64), nblk(N, 64));
-    if (transb) hipLaunchKernelGGL(k_sgemm<true>, grid, dim3(256), 0, s, M, N, K, A, lda, B, ldb, C, ldc, bias, relu);
-    else hipLaunchKernelGGL(k_sgemm<false>, grid, dim3(256), 0, s, M, N, K, A, lda, B, ldb, C, ldc, bias, relu);
+// persistent workgroups over `groups` pieces of work, at most `most` of them
+unsigned persistent(int64_t groups, int64_t most) { return static_cast<unsigned>(std::max<int64_t>(1, std::min(groups, most))); }
+
+// The layer kernels run one workgroup per CU, of as many waves (16 nodes each) as that takes, up
+// to 16: the weights are staged once per workgroup, and 16 waves are what the registers allow a
+// CU anyway.  A forward pass over 485 / 15 327 / 30 850 / 77 268 / 773 293 nodes took 51 / 58 /
+// 107 / 187 / 1099 us with 4 waves a workgroup (and up to four workgroups a CU), 52 / 59 / 92 /
+// 129 / 805 with 8 (up to two) and 69 / 83 / 91 / 106 / 772 with 16.
+struct LayerShape {
+    unsigned blocks;
+    int threads;
+    bool wide;      // 2 GB of rows and more
+};
+LayerShape layer_shape(int64_t n) {
+    constexpr int64_t kCus = 256;
+    const int threads = n <= kCus * 64 ? 256 : n <= kCus * 128 ? 512 : 1024;
+    return {persistent((n + threads / 4 - 1) / (threads / 4), kCus), threads, n >= int64_t(1) << 23};
 }
 
-// out (+)= A^T B over all M rows: per-block partials, then a fixed-order sum (deterministic).
-// MFMA for KA <= 64 and 16 <= NB <= 128; the FP32 VALU kernel for the thin cases.
+bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
+// out = A^T B over all M rows (KA <= 128, NB = 64): per-block partials, then a fixed-order sum
+// (deterministic).  MFMA for KA <= 64, the FP32 VALU kernel above.
 void gemm_tn(hipStream_t s, int64_t M, int KA, int NB, const float* A, int lda, const float* B, int ldb, float* part,
-             float* out, int add) {
+             float* out) {
     const int rows = part_rows(M);
     const unsigned nb = std::max(1u, nblk(M, rows));
-    if (KA <= 64 && NB >= 16 && NB <= 128) {
-        const int nbt = (NB + 15) / 16;
-        if (nbt <= 4)
-            hipLaunchKernelGGL(k_gemm_tn_mfma<4>, dim3(nb), dim3(256), 0, s, M, KA, NB, A, lda, B, ldb, part, rows);
-        else
-            hipLaunchKernelGGL(k_gemm_tn_mfma<8>, dim3(nb), dim3(256), 0, s, M, KA, NB, A, lda, B, ldb, part, rows);
-    } else {
+    if (KA <= 64)
+        hipLaunchKernelGGL(k_gemm_tn_mfma<4>, dim3(nb), dim3(256), 0, s, M, KA, NB, A, lda, B, ldb, part, rows);
+    else
         hipLaunchKernelGGL(k_sgemm_tn_partial, dim3(nb), dim3(256), 0, s, M, KA, NB, A, lda, B, ldb, part, rows);
-    }
     hipLaunchKernelGGL(k_reduce_partials, dim3(nblk(KA * NB, kWave)), dim3(kRedWaves * 64), 0, s, static_cast<int>(nb),
-                       KA * NB, part, out, add);
+                       KA * NB, KA * NB, part, out, 0, 0, nullptr, nullptr);
 }
 
 void colsum(hipStream_t s, int64_t M, const float* G, int ldg, float* part, float* out) {
     const int rows = part_rows(M);
     const unsigned nb = std::max(1u, nblk(M, rows));
     hipLaunchKernelGGL(k_colsum_partial, dim3(nb), dim3(256), 0, s, M, G, ldg, part, rows);
-    hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kRedWaves * 64), 0, s, static_cast<int>(nb), kH, part, out, 0);
+    hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kRedWaves * 64), 0, s, static_cast<int>(nb), kH, kH, part, out, 0, 0,
+                       nullptr, nullptr);
 }
 
 }  // namespace
@@ -632,8 +927,8 @@ extern "C" {
 int64_t nd_mp_param_count(int32_t nfeat) { return offsets(nfeat).total; }
 
 int64_t nd_mp_workspace_floats(int64_t nnodes) {
-    // activations H0..H4 (5*64) + Y (128) per node, backward: g (64), [dYa|g] (128), dH (64),
-    // head gradient (1) + partial buffers
+    // per node: activations H0..H4 (5*64), the column sums' partials (128), two gradients in
+    // turn and A^T g (3*64 of 4*64 + 1); then the partial sums
     const int64_t nb = std::min<int64_t>(kMaxPartBlocks, (nnodes + 63) / 64);
     return nnodes * (5 * kH + 2 * kH + kH + 2 * kH + kH + 1) + (nb + 2) * (kH * 2 * kH) + nnodes / 4 + 8;
 }
@@ -647,15 +942,20 @@ int nd_mp_forward(int64_t n, const int32_t* rowptr, const int32_t* nbr, const fl
     hipStream_t s = static_cast<hipStream_t>(stream);
     const Offsets o = offsets(nfeat);
     float* H = work;                        // H_l at H + l*n*64
-    float* Y = work + 5 * n * kH;           // n x 128
-    gemm(s, false, n, kH, nfeat, X, nfeat, params + o.win, kH, H, kH, params + o.bin, 1);
+    const LayerShape sh = layer_shape(n);
+    const auto layer = sh.wide ? k_layer<1024, true> : sh.threads == 1024 ? k_layer<1024, false>
+                                                   : sh.threads == 512    ? k_layer<512, false> : k_layer<256, false>;
+    if (nfeat == 8 && aligned16(X))
+        hipLaunchKernelGGL(k_input8, dim3(persistent((n + 15) / 16, 2048)), dim3(256), 0, s, n, X, params + o.win,
+                           params + o.bin, H);
+    else
+        input_gemm(s, n, nfeat, X, params + o.win, H, params + o.bin);
     for (int l = 0; l < kLayers; ++l) {
-        gemm(s, false, n, 2 * kH, kH, H + l * n * kH, kH, params + o.wl[l], 2 * kH, Y, 2 * kH, nullptr, 0);
-        hipLaunchKernelGGL(k_spmm, dim3(nblk(n, 16)), dim3(256), 0, s, n, rowptr, nbr, a_fwd, Y, 2 * kH,
-                           H + (l + 1) * n * kH, kH, params + o.bl[l], 1);
+        const bool last = l == kLayers - 1;
+        hipLaunchKernelGGL(layer, dim3(sh.blocks), dim3(sh.threads), 0, s, n, rowptr, nbr, a_fwd,
+                           H + l * n * kH, params + o.wl[l], params + o.bl[l], H + (l + 1) * n * kH, params + o.wout,
+                           params + o.bout, last ? out : nullptr);
     }
-    hipLaunchKernelGGL(k_head, dim3(nblk(n, 4)), dim3(256), 0, s, n, H + 4 * n * kH, params + o.wout, params + o.bout,
-                       out, nullptr, nullptr, nullptr, nullptr);
     return herr(hipGetLastError(), "nd_mp_forward");
 }
 
@@ -672,35 +972,42 @@ int nd_mp_backward(int64_t n, const int32_t* rowptr, const int32_t* nbr, const f
     hipStream_t s = static_cast<hipStream_t>(stream);
     const Offsets o = offsets(nfeat);
     float* H = work;
-    float* G = work + 5 * n * kH + n * 2 * kH;   // g: n x 64
-    float* DY = G + n * kH;                       // [dYa | g]: n x 128
-    float* DH = DY + n * 2 * kH;                  // dH: n x 64
-    float* dout = DH + n * kH;                    // n
-    float* part = dout + n;                       // partials
-    hipLaunchKernelGGL(k_head, dim3(nblk(n, 4)), dim3(256), 0, s, n, H + 4 * n * kH, params + o.wout, params + o.bout,
-                       nullptr, target, dout, DH, loss_part);
-    gemm_tn(s, n, kH, 1, H + 4 * n * kH, kH, dout, 1, part, grads + o.wout, 0);
-    {
-        const int rows = part_rows(n);
-        const unsigned nb = std::max(1u, nblk(n, rows));
-        hipLaunchKernelGGL(k_vsum_partial, dim3(nb), dim3(256), 0, s, n, dout, part, rows);
-        hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kRedWaves * 64), 0, s, static_cast<int>(nb), 1, part,
-                           grads + o.bout, 0);
-    }
+    float* G = work + 5 * n * kH + n * 2 * kH;   // gradients at the layers' sums, in turn: n x 64 each
+    float* G2 = G + n * kH;
+    float* Z = G2 + n * kH;                       // A^T g: n x 64
+    float* part = G + n * (kH + 2 * kH + kH + 1); // partials
+    float* bpart = work + 5 * n * kH;             // column-sum partials
+    const LayerShape sh = layer_shape(n);
+    const auto layer_bwd = sh.wide ? k_layer_bwd<1024, true> : sh.threads == 1024 ? k_layer_bwd<1024, false>
+                                                           : sh.threads == 512    ? k_layer_bwd<512, false> : k_layer_bwd<256, false>;
+    const unsigned hb = persistent((n + 15) / 16, kMaxPartBlocks);
+    hipLaunchKernelGGL(k_head_bwd, dim3(hb), dim3(256), 0, s, n, H + 4 * n * kH, params + o.wout, params + o.bout, target, G,
+                       loss_part, part);
+    // w_out's 64 gradients and b_out's follow each other in the parameters and in a partial
+    hipLaunchKernelGGL(k_reduce_partials, dim3(2), dim3(kRedWaves * 64), 0, s, static_cast<int>(hb), kH + 1, 2 * kH, part,
+                       grads + o.wout, 0, 0, nullptr, nullptr);
+    const int64_t wblocks = persistent((n + 63) / 64, kWgradBlocks);
+    const int64_t wstep = 4 * kWgradWaves * wblocks;
+    const int rows = static_cast<int>((n + wstep - 1) / wstep) * 4 * kWgradWaves;
+    const unsigned wb = nblk(n, rows);
     for (int l = kLayers - 1; l >= 0; --l) {
-        // g = dH_{l+1} * relu'(H_{l+1}), into G and the right half of [dYa | g]
-        hipLaunchKernelGGL(k_relu_grad, dim3(nblk(n * kH, 256)), dim3(256), 0, s, n, DH, H + (l + 1) * n * kH, G, DY);
-        colsum(s, n, G, kH, part, grads + o.bl[l]);
-        // dYa = A^T g into the left half
-        hipLaunchKernelGGL(k_spmm, dim3(nblk(n, 16)), dim3(256), 0, s, n, rowptr, nbr, a_bwd, G, kH, DY, 2 * kH,
-                           nullptr, 0);
-        // d[W|U] = H_l^T [dYa | g];  dH_l = [dYa | g] [W|U]^T
-        gemm_tn(s, n, kH, 2 * kH, H + l * n * kH, kH, DY, 2 * kH, part, grads + o.wl[l], 0);
-        gemm(s, true, n, kH, 2 * kH, DY, 2 * kH, params + o.wl[l], 2 * kH, DH, kH, nullptr, 0);
+        hipLaunchKernelGGL(layer_bwd, dim3(sh.blocks), dim3(sh.threads), 0, s, n, rowptr, nbr, a_bwd,
+                           G, params + o.wl[l], H + l * n * kH, Z, G2);
+        hipLaunchKernelGGL(k_wgrad, dim3(wb), dim3(64 * kWgradWaves), 0, s, n, H + l * n * kH, Z, G, part, bpart, rows);
+        hipLaunchKernelGGL(k_reduce_partials, dim3(nblk(kH * 2 * kH, kWave) + 1), dim3(kRedWaves * 64), 0, s,
+                           static_cast<int>(wb), kH * 2 * kH, kH * 2 * kH, part, grads + o.wl[l], static_cast<int>(wb), kH,
+                           bpart, grads + o.bl[l]);
+        std::swap(G, G2);
     }
-    hipLaunchKernelGGL(k_relu_grad, dim3(nblk(n * kH, 256)), dim3(256), 0, s, n, DH, H, G, nullptr);
-    colsum(s, n, G, kH, part, grads + o.bin);
-    gemm_tn(s, n, nfeat, kH, X, nfeat, G, kH, part, grads + o.win, 0);
+    if (nfeat == 8 && aligned16(X)) {
+        const unsigned ib = persistent((n + 15) / 16, kMaxPartBlocks);
+        hipLaunchKernelGGL(k_input_grad8, dim3(ib), dim3(256), 0, s, n, X, G, part);
+        hipLaunchKernelGGL(k_reduce_partials, dim3(nblk(9 * kH, kWave)), dim3(kRedWaves * 64), 0, s, static_cast<int>(ib),
+                           9 * kH, 9 * kH, part, grads + o.win, 0, 0, nullptr, nullptr);
+    } else {
+        colsum(s, n, G, kH, part, grads + o.bin);
+        gemm_tn(s, n, nfeat, kH, X, nfeat, G, kH, part, grads + o.win);
+    }
     return herr(hipGetLastError(), "nd_mp_backward");
 }
 
