@@ -98,6 +98,8 @@ template <int K> __device__ __forceinline__ DualK<K> dualk_const(double x) {
     for (int j = 0; j < K; ++j) r.d[j] = x == x ? 0.0 : x;
     return r;
 }
+template <> __device__ __forceinline__ DualK<1> nan_of<DualK<1>>() { return dualk_const<1>(__builtin_nan("")); }
+template <> __device__ __forceinline__ DualK<1> zero_of<DualK<1>>() { return dualk_const<1>(0.0); }
 template <> __device__ __forceinline__ DualK<4> nan_of<DualK<4>>() { return dualk_const<4>(__builtin_nan("")); }
 template <> __device__ __forceinline__ DualK<8> nan_of<DualK<8>>() { return dualk_const<8>(__builtin_nan("")); }
 template <> __device__ __forceinline__ DualK<4> zero_of<DualK<4>>() { return dualk_const<4>(0.0); }

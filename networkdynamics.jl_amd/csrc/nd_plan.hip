@@ -630,26 +630,8 @@ __global__ void __launch_bounds__(256) k_edge_ode(EDesc e, const double* __restr
 // ---- Jacobian-vector product: the RHS evaluated on dual numbers u + eps*v -------------
 // du = f(u) and jv = J(u) v in one pass; the value part is the plain RHS with every
 // segment summed in the reference order (no hub trees), the tangent part follows the
-// forward-mode rules of each operation.  One thread per vertex.
-template <int EM, int WRAP>
-__device__ __forceinline__ Dual slot_value_dual(int2 s, Dual own, const double* __restrict__ u,
-                                                const double* __restrict__ v, const double* __restrict__ vo,
-                                                const double* __restrict__ dvo, const double* __restrict__ p) {
-    if constexpr (EM == ND_EM_NOOP) {
-        return dual_nan();
-    } else if constexpr (is_ode_model(EM)) {
-        return ode_side_rt(WRAP, Dual{u[s.x], v[s.x]}, s.y & 1);
-    } else {
-        const Dual nbr{vo[s.x], dvo[s.x]};
-        const double* pe = p + (s.y >> 1);
-        if (s.y & 1) {
-            const Dual y = g_dst<EM, Dual>(own, nbr, pe);
-            return WRAP == ND_WRAP_SYMMETRIC ? y : -y;
-        }
-        return g_dst<EM, Dual>(nbr, own, pe);
-    }
-}
-
+// forward-mode rules of each operation.  The fused vertex batches: k_vertex_jvp, after the
+// K-tangent edge kernels.
 __device__ __forceinline__ Dual slot_value_dual_rt(const EDesc& e, int2 s, Dual own, const double* __restrict__ u,
                                                    const double* __restrict__ v, const double* __restrict__ vo,
                                                    const double* __restrict__ dvo, const double* __restrict__ p) {
@@ -664,36 +646,17 @@ __device__ __forceinline__ Dual slot_value_dual_rt(const EDesc& e, int2 s, Dual 
     return g_dst_rt<Dual>(e.model, nbr, own, pe);
 }
 
-template <int VM, int EM, int WRAP, bool MULTI>
-__global__ void __launch_bounds__(256) k_vertex_jvp(VDesc vd, const int32_t* __restrict__ rowptr,
-                                                    const int2* __restrict__ slots, const uint8_t* __restrict__ slot_eb,
-                                                    const EDesc* __restrict__ ed, const double* __restrict__ u,
-                                                    const double* __restrict__ v, const double* __restrict__ vo,
-                                                    const double* __restrict__ dvo, const double* __restrict__ p,
-                                                    double* __restrict__ du, double* __restrict__ jv) {
-    constexpr int DIMC = VModel<VM>::dim;
+// batches whose f does nothing in networks of the generic kernels
+__global__ void __launch_bounds__(256) k_vertex_noop_jvp(VDesc vd, const int32_t* __restrict__, const int2* __restrict__,
+                                                         const uint8_t* __restrict__, const EDesc* __restrict__,
+                                                         const double* __restrict__, const double* __restrict__,
+                                                         const double* __restrict__, const double* __restrict__,
+                                                         const double* __restrict__, double* __restrict__ du,
+                                                         double* __restrict__ jv) {
     const int32_t q = static_cast<int32_t>(blockIdx.x * blockDim.x + threadIdx.x);
     if (q >= vd.count) return;
-    const int dim = DIMC > 0 ? DIMC : vd.dim;
-    const int64_t x0 = static_cast<int64_t>(vd.state0) + static_cast<int64_t>(q) * dim;
-    if constexpr (VM == ND_VM_NOOP) {
-        for (int j = 0; j < dim; ++j) { du[x0 + j] = 0.0; jv[x0 + j] = 0.0; }
-    } else {
-        Dual x[DIMC];
-#pragma unroll
-        for (int j = 0; j < DIMC; ++j) x[j] = Dual{u[x0 + j], v[x0 + j]};
-        const Dual own = x[vd.mask[0]];
-        Dual acc{0.0, 0.0};
-        const int32_t beg = rowptr[vd.row0 + q], end = rowptr[vd.row0 + q + 1];
-        for (int32_t s = beg; s < end; ++s) {
-            if constexpr (MULTI) acc = acc + slot_value_dual_rt(ed[slot_eb[s]], slots[s], own, u, v, vo, dvo, p);
-            else acc = acc + slot_value_dual<EM, WRAP>(slots[s], own, u, v, vo, dvo, p);
-        }
-        Dual dx[DIMC];
-        vertex_f<VM, Dual>(dx, x, acc, p + vd.param0 + static_cast<int64_t>(q) * vd.pdim, DIMC);
-#pragma unroll
-        for (int j = 0; j < DIMC; ++j) { du[x0 + j] = dx[j].v; jv[x0 + j] = dx[j].d; }
-    }
+    const int64_t x0 = static_cast<int64_t>(vd.state0) + static_cast<int64_t>(q) * vd.dim;
+    for (int j = 0; j < vd.dim; ++j) { du[x0 + j] = 0.0; jv[x0 + j] = 0.0; }
 }
 
 // du, jv of ODE edges (the dual form of k_edge_ode); eo, deo: the endpoint outputs and
@@ -770,28 +733,53 @@ struct JvpKArgs {
     int32_t k;
 };
 
+// x and the K tangents of the state (OUT: of the vertex outputs) at i.  The columns past k repeat the
+// last one: every load is unconditional, and their results are not stored.
+template <int K, bool OUT>
+__device__ __forceinline__ DualK<K> jvp_load(const JvpKArgs& a, int64_t i) {
+    const double* __restrict__ x = OUT ? a.vo : a.u;
+    const double* __restrict__ dx = OUT ? a.dvo : a.v;
+    const int64_t ld = OUT ? a.ldo : a.ldu;
+    DualK<K> r;
+    r.v = x[i];
+#pragma unroll
+    for (int j = 0; j < K; ++j) r.d[j] = (dx + (j < a.k ? j : a.k - 1) * ld)[i];
+    return r;
+}
+
 template <int EM, int WRAP, int K>
-__device__ __forceinline__ DualK<K> slot_value_k(int2 s, DualK<K> own, const JvpKArgs& a) {
+__device__ __forceinline__ DualK<K> slot_value_k(int2 s, const DualK<K>& own, const JvpKArgs& a) {
     if constexpr (EM == ND_EM_NOOP) {
         return nan_of<DualK<K>>();
     } else if constexpr (is_ode_model(EM)) {
-        return ode_side_k<K>(WRAP, dk_load<K>(a.u, a.v, a.ldu, a.k, s.x), s.y & 1);
+        return ode_side_k<K>(WRAP, jvp_load<K, false>(a, s.x), s.y & 1);
     } else {
-        const DualK<K> nbr = dk_load<K>(a.vo, a.dvo, a.ldo, a.k, s.x);
-        const double* pe = a.p + (s.y >> 1);
-        if (s.y & 1) {
-            const DualK<K> y = g_dst<EM, DualK<K>>(own, nbr, pe);
-            return WRAP == ND_WRAP_SYMMETRIC ? y : -y;
+        // one evaluation for either direction: a wave holds entries of both
+        const DualK<K> nbr = jvp_load<K, true>(a, s.x);
+        const bool is_src = s.y & 1;
+        DualK<K> from, to;
+        from.v = is_src ? own.v : nbr.v;
+        to.v = is_src ? nbr.v : own.v;
+#pragma unroll
+        for (int j = 0; j < K; ++j) {
+            from.d[j] = is_src ? own.d[j] : nbr.d[j];
+            to.d[j] = is_src ? nbr.d[j] : own.d[j];
         }
-        return g_dst<EM, DualK<K>>(nbr, own, pe);
+        DualK<K> y = g_dst<EM, DualK<K>>(from, to, a.p + (s.y >> 1));
+        const DualK<K> m = -y;
+        const bool neg = is_src && WRAP != ND_WRAP_SYMMETRIC;
+        y.v = neg ? m.v : y.v;
+#pragma unroll
+        for (int j = 0; j < K; ++j) y.d[j] = neg ? m.d[j] : y.d[j];
+        return y;
     }
 }
 
 template <int K>
-__device__ __forceinline__ DualK<K> slot_value_k_rt(const EDesc& e, int2 s, DualK<K> own, const JvpKArgs& a) {
+__device__ __forceinline__ DualK<K> slot_value_k_rt(const EDesc& e, int2 s, const DualK<K>& own, const JvpKArgs& a) {
     if (e.model == ND_EM_NOOP) return nan_of<DualK<K>>();
-    if (e.ode) return ode_side_k<K>(e.wrap, dk_load<K>(a.u, a.v, a.ldu, a.k, s.x), s.y & 1);
-    const DualK<K> nbr = dk_load<K>(a.vo, a.dvo, a.ldo, a.k, s.x);
+    if (e.ode) return ode_side_k<K>(e.wrap, jvp_load<K, false>(a, s.x), s.y & 1);
+    const DualK<K> nbr = jvp_load<K, true>(a, s.x);
     const double* pe = a.p + (s.y >> 1);
     if (s.y & 1) {
         const DualK<K> y = g_dst_rt<DualK<K>>(e.model, own, nbr, pe);
@@ -800,36 +788,118 @@ __device__ __forceinline__ DualK<K> slot_value_k_rt(const EDesc& e, int2 s, Dual
     return g_dst_rt<DualK<K>>(e.model, nbr, own, pe);
 }
 
-// the K-tangent form of k_vertex_jvp: one thread per vertex
-template <int VM, int EM, int WRAP, bool MULTI, int K>
-__global__ void __launch_bounds__(256) k_vertex_jvpk(VDesc vd, const int32_t* __restrict__ rowptr,
-                                                     const int2* __restrict__ slots, const uint8_t* __restrict__ slot_eb,
-                                                     const EDesc* __restrict__ ed, JvpKArgs a) {
+// order between LDS writes and reads of lanes of one wave
+__device__ __forceinline__ void wave_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+// Up to kGroupMax vertex batches in one launch: batch i owns the blocks first[i] ..
+// first[i + 1] - 1, first one per row of more than kJvpRow entries (positions hubs[i]), then one
+// per 32 vertices.
+constexpr int kJvpRow = 64, kJvpLanes = 8;
+struct JvpGroup {
+    VDesc vd[kGroupMax];
+    const int32_t* hubs[kGroupMax];
+    int32_t nhub[kGroupMax];
+    int32_t first[kGroupMax + 1];
+    int32_t n;
+};
+
+// du (col 0) and column col of jv of vertex q from its aggregate
+template <int VM>
+__device__ __forceinline__ void jvp_vertex(const VDesc& vd, int32_t q, int col, Dual acc, const JvpKArgs& a) {
     constexpr int DIMC = VModel<VM>::dim;
-    const int32_t q = static_cast<int32_t>(blockIdx.x * blockDim.x + threadIdx.x);
-    if (q >= vd.count) return;
     const int dim = DIMC > 0 ? DIMC : vd.dim;
     const int64_t x0 = static_cast<int64_t>(vd.state0) + static_cast<int64_t>(q) * dim;
+    double* jv = a.jv + col * a.ldu;
     if constexpr (VM == ND_VM_NOOP) {
-        for (int j = 0; j < dim; ++j) dk_store<K>(a.du, a.jv, a.ldu, a.k, x0 + j, dualk_const<K>(0.0));
-    } else {
-        DualK<K> x[DIMC];
-#pragma unroll
-        for (int j = 0; j < DIMC; ++j) x[j] = dk_load<K>(a.u, a.v, a.ldu, a.k, x0 + j);
-        DualK<K> own = x[0];          // x[mask] by selects: a runtime index would put x in scratch
-#pragma unroll
-        for (int j = 1; j < DIMC; ++j)
-            if (vd.mask[0] == j) own = x[j];
-        DualK<K> acc = dualk_const<K>(0.0);
-        const int32_t beg = rowptr[vd.row0 + q], end = rowptr[vd.row0 + q + 1];
-        for (int32_t s = beg; s < end; ++s) {
-            if constexpr (MULTI) acc = acc + slot_value_k_rt<K>(ed[slot_eb[s]], slots[s], own, a);
-            else acc = acc + slot_value_k<EM, WRAP, K>(slots[s], own, a);
+        for (int j = 0; j < dim; ++j) {
+            if (col == 0) a.du[x0 + j] = 0.0;
+            jv[x0 + j] = 0.0;
         }
-        DualK<K> dx[DIMC];
-        vertex_f<VM, DualK<K>>(dx, x, acc, a.p + vd.param0 + static_cast<int64_t>(q) * vd.pdim, DIMC);
+    } else {
+        Dual x[DIMC], dx[DIMC];
 #pragma unroll
-        for (int j = 0; j < DIMC; ++j) dk_store<K>(a.du, a.jv, a.ldu, a.k, x0 + j, dx[j]);
+        for (int j = 0; j < DIMC; ++j) x[j] = Dual{a.u[x0 + j], a.v[col * a.ldu + x0 + j]};
+        vertex_f<VM, Dual>(dx, x, acc, a.p + vd.param0 + static_cast<int64_t>(q) * vd.pdim, DIMC);
+#pragma unroll
+        for (int j = 0; j < DIMC; ++j) {
+            if (col == 0) a.du[x0 + j] = dx[j].v;
+            jv[x0 + j] = dx[j].d;
+        }
+    }
+}
+
+// The fused vertex batches, k <= K tangents: 8 lanes per vertex, or a whole workgroup for a row
+// of more than kJvpRow entries.  A lane evaluates one entry on all K tangents at once (the sine and
+// cosine once per entry, 2 + K independent loads), the results pass through LDS, and lane j sums
+// the value and tangent j in the order of the row.
+// Bound by the neighbours' loads, K + 1 cache lines an entry.  Eight tangents of 1e5 vertices on
+// a geometric graph (two batches, 4 entries a row): 48 us, one tangent 15; a thread per vertex,
+// one launch per batch, took 75 and 52 (its few waves wait on one entry at a time, and evaluate
+// both directions of an edge where a wave holds both).  Preferential attachment, 100 003
+// vertices and rows up to about 900: 56 and 33 against 1037 and 652, one thread per row.
+// 2 / 4 / 8 lanes per vertex: 54 / 50 / 48 us for eight tangents, 15.3 / 14.0 / 14.6 for one;
+// lanes that share a vertex's entries and split its tangents, 57 to 60.
+template <int EM, int WRAP, bool MULTI, int K>
+__global__ void __launch_bounds__(256) k_vertex_jvp(JvpGroup g, const int32_t* __restrict__ rowptr,
+                                                    const int2* __restrict__ slots, const uint8_t* __restrict__ slot_eb,
+                                                    const EDesc* __restrict__ ed, JvpKArgs a) {
+    __shared__ double buf[256 * (K + 1)];
+    int i = 0;
+    while (i + 1 < g.n && static_cast<int32_t>(blockIdx.x) >= g.first[i + 1]) ++i;
+    const VDesc& vd = g.vd[i];
+    const int32_t b = static_cast<int32_t>(blockIdx.x) - g.first[i];
+    const bool hub = b < g.nhub[i];
+    const int t = threadIdx.x, lane = hub ? t : t % kJvpLanes, width = hub ? 256 : kJvpLanes, base = t - lane;
+    const int32_t q = hub ? g.hubs[i][b] : (b - g.nhub[i]) * (256 / kJvpLanes) + t / kJvpLanes;
+    if (q >= vd.count) return;
+    static_assert(K <= kJvpLanes, "a lane sums one tangent");
+    Dual acc{0.0, 0.0};
+    if (vd.model != ND_VM_NOOP) {
+        const int32_t beg = rowptr[vd.row0 + q], end = rowptr[vd.row0 + q + 1];
+        if (!hub && end - beg > kJvpRow) return;
+        const DualK<K> own = jvp_load<K, false>(a, static_cast<int64_t>(vd.state0) + static_cast<int64_t>(q) * vd.dim + vd.mask[0]);
+        for (int32_t s0 = beg; s0 < end; s0 += width) {
+            const int32_t s = s0 + lane, count = end - s0 < width ? end - s0 : width;
+            if (lane < count) {
+                DualK<K> y;
+                if constexpr (MULTI) y = slot_value_k_rt<K>(ed[slot_eb[s]], slots[s], own, a);
+                else y = slot_value_k<EM, WRAP, K>(slots[s], own, a);
+                double* to = buf + t * (K + 1);
+                to[0] = y.v;
+#pragma unroll
+                for (int j = 0; j < K; ++j) to[1 + j] = y.d[j];
+            }
+            if (hub) __syncthreads();
+            else wave_order();
+            if (lane < K) {
+                const double* from = buf + base * (K + 1);
+                for (int e0 = 0; e0 < count; e0 += 8) {
+                    Dual y[8];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) y[e] = Dual{from[(e0 + e) * (K + 1)], from[(e0 + e) * (K + 1) + 1 + lane]};
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const Dual sum = acc + y[e];
+                        acc.v = e0 + e < count ? sum.v : acc.v;
+                        acc.d = e0 + e < count ? sum.d : acc.d;
+                    }
+                }
+            }
+            if (hub) __syncthreads();
+            else wave_order();
+        }
+    }
+    if (lane >= a.k) return;
+    switch (vd.model) {
+    case ND_VM_DIFFUSION: return jvp_vertex<ND_VM_DIFFUSION>(vd, q, lane, acc, a);
+    case ND_VM_KURAMOTO: return jvp_vertex<ND_VM_KURAMOTO>(vd, q, lane, acc, a);
+    case ND_VM_SWING: return jvp_vertex<ND_VM_SWING>(vd, q, lane, acc, a);
+    case ND_VM_SWING_UNIT_DAMPING: return jvp_vertex<ND_VM_SWING_UNIT_DAMPING>(vd, q, lane, acc, a);
+    case ND_VM_LOAD: return jvp_vertex<ND_VM_LOAD>(vd, q, lane, acc, a);
+    default: return jvp_vertex<ND_VM_NOOP>(vd, q, lane, acc, a);
     }
 }
 
@@ -1639,48 +1709,6 @@ VertexBufKernel pick_vertex_f_buf(int vm) {
 using JvpKernel = void (*)(VDesc, const int32_t*, const int2*, const uint8_t*, const EDesc*, const double*,
                            const double*, const double*, const double*, const double*, double*, double*);
 
-template <int VM>
-JvpKernel pick_jvp_edge(int em, int wrap, bool multi) {
-    if (multi) return k_vertex_jvp<VM, ND_EM_NOOP, ND_WRAP_NONE, true>;
-    const bool sym = wrap == ND_WRAP_SYMMETRIC;
-    switch (em) {
-    case ND_EM_KURAMOTO:
-        return sym ? k_vertex_jvp<VM, ND_EM_KURAMOTO, ND_WRAP_SYMMETRIC, false>
-                   : k_vertex_jvp<VM, ND_EM_KURAMOTO, ND_WRAP_ANTISYMMETRIC, false>;
-    case ND_EM_STATIC_LINE:
-        return sym ? k_vertex_jvp<VM, ND_EM_STATIC_LINE, ND_WRAP_SYMMETRIC, false>
-                   : k_vertex_jvp<VM, ND_EM_STATIC_LINE, ND_WRAP_ANTISYMMETRIC, false>;
-    case ND_EM_DIFFUSION:
-        return sym ? k_vertex_jvp<VM, ND_EM_DIFFUSION, ND_WRAP_SYMMETRIC, false>
-                   : k_vertex_jvp<VM, ND_EM_DIFFUSION, ND_WRAP_ANTISYMMETRIC, false>;
-    case ND_EM_DIFFUSION_WEIGHTED:
-        return sym ? k_vertex_jvp<VM, ND_EM_DIFFUSION_WEIGHTED, ND_WRAP_SYMMETRIC, false>
-                   : k_vertex_jvp<VM, ND_EM_DIFFUSION_WEIGHTED, ND_WRAP_ANTISYMMETRIC, false>;
-    case ND_EM_DIFFUSION_FIDUCIAL:
-        return k_vertex_jvp<VM, ND_EM_DIFFUSION_FIDUCIAL, ND_WRAP_ANTISYMMETRIC, false>;
-    case ND_EM_ODE_SIN_DIFFUSION:
-    case ND_EM_ODE_SIN_DIFFUSION_FAST:
-    case ND_EM_ODE_LINEAR:
-    case ND_EM_ODE_LAG:
-    case ND_EM_EXT_DRIVEN:
-        return wrap == ND_WRAP_ANTISYMMETRIC ? k_vertex_jvp<VM, ND_EM_ODE_LINEAR, ND_WRAP_ANTISYMMETRIC, false>
-                                             : k_vertex_jvp<VM, ND_EM_ODE_LINEAR, ND_WRAP_FIDUCIAL, false>;
-    default:
-        return k_vertex_jvp<VM, ND_EM_NOOP, ND_WRAP_NONE, false>;
-    }
-}
-
-JvpKernel pick_jvp_kernel(int vm, int em, int wrap, bool multi) {
-    switch (vm) {
-    case ND_VM_DIFFUSION: return pick_jvp_edge<ND_VM_DIFFUSION>(em, wrap, multi);
-    case ND_VM_KURAMOTO: return pick_jvp_edge<ND_VM_KURAMOTO>(em, wrap, multi);
-    case ND_VM_SWING: return pick_jvp_edge<ND_VM_SWING>(em, wrap, multi);
-    case ND_VM_SWING_UNIT_DAMPING: return pick_jvp_edge<ND_VM_SWING_UNIT_DAMPING>(em, wrap, multi);
-    case ND_VM_LOAD: return pick_jvp_edge<ND_VM_LOAD>(em, wrap, multi);
-    default: return k_vertex_jvp<ND_VM_NOOP, ND_EM_NOOP, ND_WRAP_NONE, false>;
-    }
-}
-
 JvpKernel pick_gen_jvp(int vm) {
     switch (vm) {
     case ND_VM_DIFFUSION: return k_vertex_gen_jvp<ND_VM_DIFFUSION>;
@@ -1696,7 +1724,7 @@ JvpKernel pick_gen_jvp(int vm) {
     case ND_VM_INDUCTOR_INJECTOR: return k_vertex_gen_jvp<ND_VM_INDUCTOR_INJECTOR>;
     case ND_VM_CRL: return k_vertex_gen_jvp<ND_VM_CRL>;
     case ND_VM_FHN: return k_vertex_gen_jvp<ND_VM_FHN>;
-    default: return k_vertex_jvp<ND_VM_NOOP, ND_EM_NOOP, ND_WRAP_NONE, false>;
+    default: return k_vertex_noop_jvp;
     }
 }
 
@@ -1712,52 +1740,43 @@ EdgeOdeJvpKernel pick_edge_ode_jvp(int em) {
     }
 }
 
-using JvpKKernel = void (*)(VDesc, const int32_t*, const int2*, const uint8_t*, const EDesc*, JvpKArgs);
+using VertexJvpKernel = void (*)(JvpGroup, const int32_t*, const int2*, const uint8_t*, const EDesc*, JvpKArgs);
 
-template <int VM, int K>
-JvpKKernel pick_jvpk_edge(int em, int wrap, bool multi) {
-    if (multi) return k_vertex_jvpk<VM, ND_EM_NOOP, ND_WRAP_NONE, true, K>;
+template <int K>
+VertexJvpKernel pick_vertex_jvp(int em, int wrap, bool multi) {
+    if (multi) return k_vertex_jvp<ND_EM_NOOP, ND_WRAP_NONE, true, K>;
     const bool sym = wrap == ND_WRAP_SYMMETRIC;
     switch (em) {
     case ND_EM_KURAMOTO:
-        return sym ? k_vertex_jvpk<VM, ND_EM_KURAMOTO, ND_WRAP_SYMMETRIC, false, K>
-                   : k_vertex_jvpk<VM, ND_EM_KURAMOTO, ND_WRAP_ANTISYMMETRIC, false, K>;
+        return sym ? k_vertex_jvp<ND_EM_KURAMOTO, ND_WRAP_SYMMETRIC, false, K>
+                   : k_vertex_jvp<ND_EM_KURAMOTO, ND_WRAP_ANTISYMMETRIC, false, K>;
     case ND_EM_STATIC_LINE:
-        return sym ? k_vertex_jvpk<VM, ND_EM_STATIC_LINE, ND_WRAP_SYMMETRIC, false, K>
-                   : k_vertex_jvpk<VM, ND_EM_STATIC_LINE, ND_WRAP_ANTISYMMETRIC, false, K>;
+        return sym ? k_vertex_jvp<ND_EM_STATIC_LINE, ND_WRAP_SYMMETRIC, false, K>
+                   : k_vertex_jvp<ND_EM_STATIC_LINE, ND_WRAP_ANTISYMMETRIC, false, K>;
     case ND_EM_DIFFUSION:
-        return sym ? k_vertex_jvpk<VM, ND_EM_DIFFUSION, ND_WRAP_SYMMETRIC, false, K>
-                   : k_vertex_jvpk<VM, ND_EM_DIFFUSION, ND_WRAP_ANTISYMMETRIC, false, K>;
+        return sym ? k_vertex_jvp<ND_EM_DIFFUSION, ND_WRAP_SYMMETRIC, false, K>
+                   : k_vertex_jvp<ND_EM_DIFFUSION, ND_WRAP_ANTISYMMETRIC, false, K>;
     case ND_EM_DIFFUSION_WEIGHTED:
-        return sym ? k_vertex_jvpk<VM, ND_EM_DIFFUSION_WEIGHTED, ND_WRAP_SYMMETRIC, false, K>
-                   : k_vertex_jvpk<VM, ND_EM_DIFFUSION_WEIGHTED, ND_WRAP_ANTISYMMETRIC, false, K>;
+        return sym ? k_vertex_jvp<ND_EM_DIFFUSION_WEIGHTED, ND_WRAP_SYMMETRIC, false, K>
+                   : k_vertex_jvp<ND_EM_DIFFUSION_WEIGHTED, ND_WRAP_ANTISYMMETRIC, false, K>;
     case ND_EM_DIFFUSION_FIDUCIAL:
-        return k_vertex_jvpk<VM, ND_EM_DIFFUSION_FIDUCIAL, ND_WRAP_ANTISYMMETRIC, false, K>;
+        return k_vertex_jvp<ND_EM_DIFFUSION_FIDUCIAL, ND_WRAP_ANTISYMMETRIC, false, K>;
     case ND_EM_ODE_SIN_DIFFUSION:
     case ND_EM_ODE_SIN_DIFFUSION_FAST:
     case ND_EM_ODE_LINEAR:
     case ND_EM_ODE_LAG:
     case ND_EM_EXT_DRIVEN:
-        return wrap == ND_WRAP_ANTISYMMETRIC ? k_vertex_jvpk<VM, ND_EM_ODE_LINEAR, ND_WRAP_ANTISYMMETRIC, false, K>
-                                             : k_vertex_jvpk<VM, ND_EM_ODE_LINEAR, ND_WRAP_FIDUCIAL, false, K>;
+        return wrap == ND_WRAP_ANTISYMMETRIC ? k_vertex_jvp<ND_EM_ODE_LINEAR, ND_WRAP_ANTISYMMETRIC, false, K>
+                                             : k_vertex_jvp<ND_EM_ODE_LINEAR, ND_WRAP_FIDUCIAL, false, K>;
     default:
-        return k_vertex_jvpk<VM, ND_EM_NOOP, ND_WRAP_NONE, false, K>;
+        return k_vertex_jvp<ND_EM_NOOP, ND_WRAP_NONE, false, K>;
     }
 }
 
-// the K-tangent vertex kernel of a batch, or null where the batch takes the generic or
-// vector-output kernels (those have single-tangent forms only)
-template <int K>
-JvpKKernel pick_jvpk_kernel(int vm, int em, int wrap, bool multi) {
-    switch (vm) {
-    case ND_VM_DIFFUSION: return pick_jvpk_edge<ND_VM_DIFFUSION, K>(em, wrap, multi);
-    case ND_VM_KURAMOTO: return pick_jvpk_edge<ND_VM_KURAMOTO, K>(em, wrap, multi);
-    case ND_VM_SWING: return pick_jvpk_edge<ND_VM_SWING, K>(em, wrap, multi);
-    case ND_VM_SWING_UNIT_DAMPING: return pick_jvpk_edge<ND_VM_SWING_UNIT_DAMPING, K>(em, wrap, multi);
-    case ND_VM_LOAD: return pick_jvpk_edge<ND_VM_LOAD, K>(em, wrap, multi);
-    case ND_VM_NOOP: return k_vertex_jvpk<ND_VM_NOOP, ND_EM_NOOP, ND_WRAP_NONE, false, K>;
-    default: return nullptr;
-    }
+// the vertex models of k_vertex_jvp with K tangents
+bool vertex_jvpk_known(int vm) {
+    return vm == ND_VM_DIFFUSION || vm == ND_VM_KURAMOTO || vm == ND_VM_SWING || vm == ND_VM_SWING_UNIT_DAMPING ||
+           vm == ND_VM_LOAD || vm == ND_VM_NOOP;
 }
 
 using EdgeOdeJvpKKernel = void (*)(EDesc, JvpKArgs, int);
@@ -1849,8 +1868,10 @@ struct nd_plan {
     std::vector<EDesc> edesc;
     std::vector<VertexKernel> vkern, vkern_stage;
     GroupKernel gkern = nullptr, gkern_stage = nullptr;   // several fused-set batches per launch
-    std::vector<JvpKernel> vkern_jvp;
-    std::vector<JvpKKernel> vkern_jvpk4, vkern_jvpk8;   // null: no K-tangent form for the batch
+    std::vector<JvpKernel> vkern_jvp;                    // the batches of the generic kernels; null for the fused ones
+    VertexJvpKernel vjvp1 = nullptr, vjvp4 = nullptr, vjvp8 = nullptr;
+    std::vector<int32_t> jvp_hub_first;                  // per batch: its long rows in d_jvp_hubs
+    int32_t* d_jvp_hubs = nullptr;
     double* d_dvoutk = nullptr;                          // 8 tangent columns of the vertex outputs
     double* d_dvout = nullptr;     // compact tangent outputs (Jacobian-vector products)
     double* rk_work = nullptr;
@@ -2552,13 +2573,24 @@ int nd_plan_create(const nd_network* h, nd_plan** out) {
         vd.extdim = k.extdim;
         vd.outkind = k.ff == ND_FF_NOFEEDFORWARD ? 1 : k.ff == ND_FF_PUREFEEDFORWARD ? 2 : 0;
         pl->vdesc.push_back(vd);
-        pl->vkern_jvp.push_back(vd.depth > 1 ? k_vertex_vec_jvp : vd.generic ? pick_gen_jvp(k.model)
-                                           : pick_jvp_kernel(k.model, n.eb.empty() ? ND_EM_NOOP : em0, wrap0, pl->multi));
-        const bool kform = vd.depth <= 1 && !vd.generic;
-        pl->vkern_jvpk4.push_back(kform ? pick_jvpk_kernel<4>(k.model, n.eb.empty() ? ND_EM_NOOP : em0, wrap0, pl->multi)
-                                        : nullptr);
-        pl->vkern_jvpk8.push_back(kform ? pick_jvpk_kernel<8>(k.model, n.eb.empty() ? ND_EM_NOOP : em0, wrap0, pl->multi)
-                                        : nullptr);
+        pl->vkern_jvp.push_back(vd.depth > 1 ? k_vertex_vec_jvp : vd.generic ? pick_gen_jvp(k.model) : nullptr);
+    }
+    pl->vjvp1 = pick_vertex_jvp<1>(em0, wrap0, pl->multi);
+    pl->vjvp4 = pick_vertex_jvp<4>(em0, wrap0, pl->multi);
+    pl->vjvp8 = pick_vertex_jvp<8>(em0, wrap0, pl->multi);
+    {
+        std::vector<int32_t> hubs;
+        for (const VDesc& vd : pl->vdesc) {
+            pl->jvp_hub_first.push_back(static_cast<int32_t>(hubs.size()));
+            if (vd.model == ND_VM_NOOP) continue;
+            for (int32_t q = 0; q < vd.count; ++q)
+                if (pl->rowptr_host[vd.row0 + q + 1] - pl->rowptr_host[vd.row0 + q] > kJvpRow) hubs.push_back(q);
+        }
+        pl->jvp_hub_first.push_back(static_cast<int32_t>(hubs.size()));
+        if (!hubs.empty()) {
+            rc = upload(pl, hubs, &pl->d_jvp_hubs);
+            if (rc) { delete pl; return rc; }
+        }
     }
     // loopback: each injector's input is its hub's output (gen_loopback_map, post_utils.jl:205-217)
     pl->computed_out = computed_out;
@@ -2684,6 +2716,28 @@ int nd_rhs(nd_plan* pl, double* du, const double* u, const double* p, double t, 
     return hip_check(hipGetLastError(), "nd_rhs launch");
 }
 
+// the fused vertex batches of a Jacobian-vector product with a.k tangents
+static void launch_vertex_jvp(nd_plan* pl, const JvpKArgs& a, hipStream_t s) {
+    const VertexJvpKernel kern = a.k == 1 ? pl->vjvp1 : a.k <= 4 ? pl->vjvp4 : pl->vjvp8;
+    JvpGroup g{};
+    auto flush = [&]() {
+        if (g.n)
+            hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(g.first[g.n])), dim3(256), 0, s, g, pl->d_rowptr, pl->d_slots,
+                               pl->d_slot_eb, pl->d_edesc, a);
+        g.n = 0;
+    };
+    for (size_t b = 0; b < pl->vdesc.size(); ++b) {
+        const VDesc& vd = pl->vdesc[b];
+        if (vd.count == 0 || pl->vkern_jvp[b]) continue;
+        g.vd[g.n] = vd;
+        g.hubs[g.n] = pl->d_jvp_hubs + pl->jvp_hub_first[b];
+        g.nhub[g.n] = pl->jvp_hub_first[b + 1] - pl->jvp_hub_first[b];
+        g.first[g.n + 1] = g.first[g.n] + g.nhub[g.n] + static_cast<int32_t>(blocks_for(vd.count, 256 / kJvpLanes));
+        if (++g.n == kGroupMax) flush();
+    }
+    flush();
+}
+
 int nd_rhs_jvp(nd_plan* pl, double* du, double* jv, const double* u, const double* v, const double* p, double t,
                int64_t len_du, int64_t len_u, int64_t len_p, void* stream) {
     if (!pl) return nd::set_error(ND_ERR_ARGUMENT, "plan is NULL");
@@ -2720,9 +2774,21 @@ int nd_rhs_jvp(nd_plan* pl, double* du, double* jv, const double* u, const doubl
         vo = pl->d_vout;
         dvo = pl->d_dvout;
     }
+    JvpKArgs a{};
+    a.u = u;
+    a.v = v;
+    a.vo = vo;
+    a.dvo = dvo;
+    a.p = p;
+    a.du = du;
+    a.jv = jv;
+    a.ldu = pl->dim;
+    a.ldo = pl->use_vout ? pl->vout_len : pl->dim;
+    a.k = 1;
+    launch_vertex_jvp(pl, a, s);
     for (size_t b = 0; b < pl->vdesc.size(); ++b) {
         VDesc vd = pl->vdesc[b];
-        if (vd.count == 0) continue;
+        if (vd.count == 0 || !pl->vkern_jvp[b]) continue;
         vd.t = t;
         hipLaunchKernelGGL(pl->vkern_jvp[b], dim3(blocks_for(vd.count, 256)), dim3(256), 0, s, vd, pl->d_rowptr,
                            pl->d_slots, pl->d_slot_eb, pl->d_edesc, u, v, vo, dvo, p, du, jv);
@@ -2748,7 +2814,7 @@ int nd_rhs_jvp_multi(nd_plan* pl, double* du, double* jv, const double* u, const
     if (pl->pdim > 0 && !p) return nd::set_error(ND_ERR_ARGUMENT, "NULL parameter pointer");
     if (pl->ff_out) return nd::set_error(ND_ERR_UNSUPPORTED, "feed-forward vertex outputs: one tangent per nd_rhs_jvp");
     for (size_t b = 0; b < pl->vdesc.size(); ++b)
-        if (pl->vdesc[b].count && !pl->vkern_jvpk8[b])
+        if (pl->vdesc[b].count && (pl->vkern_jvp[b] || !vertex_jvpk_known(pl->vdesc[b].model)))
             return nd::set_error(ND_ERR_UNSUPPORTED, "vertex batch %zu takes the generic kernels: one tangent per "
                                  "nd_rhs_jvp", b);
     int rc = check_device(pl);
@@ -2785,14 +2851,7 @@ int nd_rhs_jvp_multi(nd_plan* pl, double* du, double* jv, const double* u, const
         a.dvo = pl->d_dvoutk;
         a.ldo = pl->vout_len;
     }
-    for (size_t b = 0; b < pl->vdesc.size(); ++b) {
-        VDesc vd = pl->vdesc[b];
-        if (vd.count == 0) continue;
-        vd.t = t;
-        JvpKKernel kern = k <= 4 ? pl->vkern_jvpk4[b] : pl->vkern_jvpk8[b];
-        hipLaunchKernelGGL(kern, dim3(blocks_for(vd.count, 256)), dim3(256), 0, s, vd, pl->d_rowptr, pl->d_slots,
-                           pl->d_slot_eb, pl->d_edesc, a);
-    }
+    launch_vertex_jvp(pl, a, s);
     for (const EDesc& e : pl->edesc) {
         if (!e.ode || e.count == 0) continue;
         EdgeOdeJvpKKernel kern = k <= 4 ? pick_edge_ode_jvpk<4>(e.model) : pick_edge_ode_jvpk<8>(e.model);
