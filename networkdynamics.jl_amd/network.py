@@ -73,17 +73,25 @@ def _edge_outsym_flat(m):
     return [None] * m.outdim_src + list(m.outsym or [])
 
 
-def _tensor_ptr(x, n, what, torch):
+def _tensor_ptr(x, what, torch):
+    # one test for the tensors that are right: the calls on small networks last no longer on the
+    # device than these checks on the host (an RHS of 1000 vertices: 9.0 us a call with a test and
+    # a device object per property and torch.cuda.current_stream, 5.5 with this and _stream)
+    if isinstance(x, torch.Tensor) and x.dtype is torch.float64 and x.is_cuda and x.dim() == 1 and x.is_contiguous():
+        return x.data_ptr(), x.numel()
     if not isinstance(x, torch.Tensor):
         raise A.ArgumentError(f"{what} must be a torch tensor on the HIP device")
     if x.dtype != torch.float64:
         # network_structure.jl:146-151: caches are Float64
         raise A.ArgumentError(f"Network caches are initialized with Float64 but is used for {x.dtype} data!")
-    if x.device.type != "cuda":
+    if not x.is_cuda:
         raise A.ArgumentError(f"{what} must live on the HIP device, got {x.device}")
-    if x.dim() != 1 or not x.is_contiguous():
-        raise A.ArgumentError(f"{what} must be a contiguous vector")
-    return x.data_ptr(), x.numel()
+    raise A.ArgumentError(f"{what} must be a contiguous vector")
+
+
+def _stream(x, torch):
+    """The current stream of the device of x (a device tensor), as the C ABI takes it."""
+    return torch._C._cuda_getCurrentRawStream(x.get_device())
 
 
 class Network:
@@ -284,12 +292,12 @@ class Network:
     def collect_externals(self, extbuf, u, o):
         """collect_externals!(map, extbuf, u, o) (external_inputs.jl:49-77) on the device."""
         import torch
-        eptr, n = _tensor_ptr(extbuf, self.info.lastidx_extbuf, "extbuf", torch)
-        uptr, _ = _tensor_ptr(u, self.dim, "u", torch)
-        optr, _ = _tensor_ptr(o, self.info.lastidx_out, "o", torch)
+        eptr, n = _tensor_ptr(extbuf, "extbuf", torch)
+        uptr, _ = _tensor_ptr(u, "u", torch)
+        optr, _ = _tensor_ptr(o, "o", torch)
         if n != self.info.lastidx_extbuf or u.numel() != self.dim or o.numel() != self.info.lastidx_out:
             raise A.ArgumentError("extbuf / u / o sizes do not match the network")
-        stream = torch.cuda.current_stream(u.device).cuda_stream
+        stream = _stream(u, torch)
         A.check(A.lib().nd_collect_externals(self.plan, eptr, uptr, optr, stream))
 
     # ---- mass matrix (construction.jl:409-453) ----------------------------------------------
@@ -406,13 +414,13 @@ class Network:
         if perturb is not None:
             self.perturbed_jvp(du, None, u, None, p, t, perturb, None, perturb_maps)
             return None
-        dptr, ndu = _tensor_ptr(du, self.dim, "du", torch)
-        uptr, nu = _tensor_ptr(u, self.dim, "u", torch)
+        dptr, ndu = _tensor_ptr(du, "du", torch)
+        uptr, nu = _tensor_ptr(u, "u", torch)
         if self.pdim > 0:
-            pptr, np_ = _tensor_ptr(p, self.pdim, "p", torch)
+            pptr, np_ = _tensor_ptr(p, "p", torch)
         else:
             pptr, np_ = (p.data_ptr(), p.numel()) if isinstance(p, torch.Tensor) else (None, 0)
-        stream = torch.cuda.current_stream(du.device).cuda_stream
+        stream = _stream(du, torch)
         A.check(A.lib().nd_rhs(self.plan, dptr, uptr, pptr, float(t), ndu, nu, np_, stream))
         return None
 
@@ -421,17 +429,17 @@ class Network:
         Jacobian-vector product ForwardDiff forms in linearize_network
         (linear_analysis.jl:74-85).  Stream-ordered on torch's current stream."""
         import torch
-        dptr, ndu = _tensor_ptr(du, self.dim, "du", torch)
-        jptr, njv = _tensor_ptr(jv, self.dim, "jv", torch)
-        uptr, nu = _tensor_ptr(u, self.dim, "u", torch)
-        vptr, nv = _tensor_ptr(v, self.dim, "v", torch)
+        dptr, ndu = _tensor_ptr(du, "du", torch)
+        jptr, njv = _tensor_ptr(jv, "jv", torch)
+        uptr, nu = _tensor_ptr(u, "u", torch)
+        vptr, nv = _tensor_ptr(v, "v", torch)
         if njv != ndu or nv != nu:      # the tangent vectors have the state's layout
             raise A.ArgumentError(f"v and jv must have the length of u and du ({self.dim})")
         if self.pdim > 0:
-            pptr, np_ = _tensor_ptr(p, self.pdim, "p", torch)
+            pptr, np_ = _tensor_ptr(p, "p", torch)
         else:
             pptr, np_ = (p.data_ptr(), p.numel()) if isinstance(p, torch.Tensor) else (None, 0)
-        stream = torch.cuda.current_stream(du.device).cuda_stream
+        stream = _stream(du, torch)
         A.check(A.lib().nd_rhs_jvp(self.plan, dptr, jptr, uptr, vptr, pptr, float(t), ndu, nu, np_, stream))
 
     def jvp_multi(self, du, jv, u, v, p, t=0.0):
@@ -441,8 +449,8 @@ class Network:
         device tensors, C-contiguous.  Raises UnsupportedError for networks whose vertex
         batches take the generic kernels (jvp serves them one tangent at a time)."""
         import torch
-        dptr, ndu = _tensor_ptr(du, self.dim, "du", torch)
-        uptr, nu = _tensor_ptr(u, self.dim, "u", torch)
+        dptr, ndu = _tensor_ptr(du, "du", torch)
+        uptr, nu = _tensor_ptr(u, "u", torch)
         for name, x in (("v", v), ("jv", jv)):
             if not isinstance(x, torch.Tensor) or x.dtype != torch.float64 or x.device.type != "cuda" or \
                     x.dim() != 2 or x.shape[1] != self.dim or not x.is_contiguous():
@@ -451,10 +459,10 @@ class Network:
         if jv.shape[0] != k or not 1 <= k <= 8:
             raise A.ArgumentError(f"v and jv need the same number of rows k, 1 <= k <= 8 (got {k}, {jv.shape[0]})")
         if self.pdim > 0:
-            pptr, np_ = _tensor_ptr(p, self.pdim, "p", torch)
+            pptr, np_ = _tensor_ptr(p, "p", torch)
         else:
             pptr, np_ = (p.data_ptr(), p.numel()) if isinstance(p, torch.Tensor) else (None, 0)
-        stream = torch.cuda.current_stream(du.device).cuda_stream
+        stream = _stream(du, torch)
         A.check(A.lib().nd_rhs_jvp_multi(self.plan, dptr, jv.data_ptr(), uptr, v.data_ptr(), int(k), pptr, float(t),
                                          ndu, nu, np_, stream))
 
@@ -490,17 +498,17 @@ class Network:
         OrdinaryDiffEq methods do."""
         import torch
         self._require_identity_mass("rk4")
-        uptr, nu = _tensor_ptr(u, self.dim, "u", torch)
+        uptr, nu = _tensor_ptr(u, "u", torch)
         if self.pdim > 0:
-            pptr, np_ = _tensor_ptr(p, self.pdim, "p", torch)
+            pptr, np_ = _tensor_ptr(p, "p", torch)
         else:
             pptr, np_ = None, 0
         wptr = None
         if work is not None:
-            wptr, nw_ = _tensor_ptr(work, 3 * self.dim, "work", torch)
+            wptr, nw_ = _tensor_ptr(work, "work", torch)
             if nw_ < 3 * self.dim:
                 raise A.ArgumentError("work needs 3*dim entries")
-        stream = torch.cuda.current_stream(u.device).cuda_stream
+        stream = _stream(u, torch)
         A.check(A.lib().nd_rk4(self.plan, uptr, pptr, float(t0), float(dt), int(nsteps), wptr, nu, np_, stream))
 
     def tsit5(self, u, p, tspan, reltol=1e-8, abstol=1e-8, dt0=0.0, maxiters=10 ** 6):
@@ -516,13 +524,13 @@ class Network:
         import torch
         from .ensemble import STAT_DTYPE, tsit5_per_instance
         self._require_identity_mass("tsit5")
-        uptr, nu = _tensor_ptr(u, self.dim, "u", torch)
+        uptr, nu = _tensor_ptr(u, "u", torch)
         if self.pdim > 0:
-            pptr, np_ = _tensor_ptr(p, self.pdim, "p", torch)
+            pptr, np_ = _tensor_ptr(p, "p", torch)
         else:
             pptr, np_ = None, 0
         stats = torch.zeros(STAT_DTYPE.itemsize // 8, dtype=torch.float64, device=u.device)
-        stream = torch.cuda.current_stream(u.device).cuda_stream
+        stream = _stream(u, torch)
         rc = A.lib().nd_tsit5(self.plan, uptr, pptr, float(tspan[0]), float(tspan[1]), float(reltol), float(abstol),
                               float(dt0), int(maxiters), stats.data_ptr(), nu, np_, stream)
         if rc == A.ND_ERR_UNSUPPORTED:
@@ -537,11 +545,11 @@ class Network:
     def get_buffers(self, u, p, t=0.0):
         """get_buffers(nw, u, p, t; initbufs=true): (o, aggbuf) device tensors, coreloop.jl:103-109."""
         import torch
-        uptr, _ = _tensor_ptr(u, self.dim, "u", torch)
+        uptr, _ = _tensor_ptr(u, "u", torch)
         pptr = p.data_ptr() if isinstance(p, torch.Tensor) and p.numel() else None
         o = torch.empty(self.info.lastidx_out, dtype=torch.float64, device=u.device)
         agg = torch.empty(self.info.lastidx_aggr, dtype=torch.float64, device=u.device)
-        stream = torch.cuda.current_stream(u.device).cuda_stream
+        stream = _stream(u, torch)
         A.check(A.lib().nd_get_buffers(self.plan, o.data_ptr(), agg.data_ptr() if agg.numel() else None,
                                        uptr, pptr, float(t), stream))
         return o, agg
@@ -566,10 +574,10 @@ class Network:
         ddelta: None for zero tangents.  With buffers=True returns (o, do, aggbuf, dagg),
         the perturbed buffers and their tangents."""
         import torch
-        dptr, _ = _tensor_ptr(du, self.dim, "du", torch)
-        uptr, _ = _tensor_ptr(u, self.dim, "u", torch)
-        jptr = _tensor_ptr(jv, self.dim, "jv", torch)[0] if jv is not None else None
-        vptr = _tensor_ptr(v, self.dim, "v", torch)[0] if v is not None else None
+        dptr, _ = _tensor_ptr(du, "du", torch)
+        uptr, _ = _tensor_ptr(u, "u", torch)
+        jptr = _tensor_ptr(jv, "jv", torch)[0] if jv is not None else None
+        vptr = _tensor_ptr(v, "v", torch)[0] if v is not None else None
         delta = torch.as_tensor(np.asarray(delta, np.float64) if not isinstance(delta, torch.Tensor) else delta,
                                 dtype=torch.float64, device=u.device).contiguous()
         self._set_perturbation(delta.numel(), perturb_maps or {})
@@ -579,16 +587,16 @@ class Network:
             if ddelta.numel() != delta.numel():
                 raise A.ArgumentError("ddelta must have the length of delta")
         if self.pdim > 0:
-            pptr, _ = _tensor_ptr(p, self.pdim, "p", torch)
+            pptr, _ = _tensor_ptr(p, "p", torch)
         else:
             pptr = p.data_ptr() if isinstance(p, torch.Tensor) and p.numel() else None
-        dpptr = _tensor_ptr(dp, self.pdim, "dp", torch)[0] if dp is not None else None
+        dpptr = _tensor_ptr(dp, "dp", torch)[0] if dp is not None else None
         bufs = None
         if buffers:
             bufs = [torch.empty(n, dtype=torch.float64, device=u.device) for n in
                     (self.info.lastidx_out, self.info.lastidx_out, self.info.lastidx_aggr, self.info.lastidx_aggr)]
         bp = [b.data_ptr() if b is not None and b.numel() else None for b in (bufs or [None] * 4)]
-        stream = torch.cuda.current_stream(u.device).cuda_stream
+        stream = _stream(u, torch)
         A.check(A.lib().nd_rhs_perturbed_jvp(self.plan, dptr, jptr, uptr, vptr, pptr, dpptr, float(t),
                                              delta.data_ptr() if delta.numel() else None,
                                              ddelta.data_ptr() if ddelta is not None and ddelta.numel() else None,
