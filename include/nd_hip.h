@@ -378,6 +378,12 @@ int nd_rhs_jvp(nd_plan* plan, double* du, double* jv, const double* u, const dou
  * feed-forward vertex outputs -> ND_ERR_UNSUPPORTED (nd_rhs_jvp per tangent serves them). */
 int nd_rhs_jvp_multi(nd_plan* plan, double* du, double* jv, const double* u, const double* v, int32_t k,
                      const double* p, double t, int64_t len_du, int64_t len_u, int64_t len_p, void* stream);
+/* The same with scratch memory: work, 8*dim device doubles (16-byte aligned; NULL or shorter: not
+ * used) that the call may overwrite.  Large networks gather the tangents of more than four
+ * columns from a copy in it with one row per state.  The results are the same bits. */
+int nd_rhs_jvp_multi_work(nd_plan* plan, double* du, double* jv, const double* u, const double* v, int32_t k,
+                          const double* p, double t, double* work, int64_t len_work, int64_t len_du, int64_t len_u,
+                          int64_t len_p, void* stream);
 
 /* collect_externals!(map, extbuf, u, o), external_inputs.jl:49-77:
  * extbuf[k] = u[i] for StateBufIdx(i), o[i] for OutBufIdx(i).  extbuf: lastidx_extbuf

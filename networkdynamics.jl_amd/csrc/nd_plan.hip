@@ -731,7 +731,9 @@ struct JvpKArgs {
     double* jv;                   // k columns, stride ldu
     int64_t ldu, ldo;
     int32_t k;
+    const double* dvt;            // the tangents of what the slots address, kJvpWide a row, or null
 };
+constexpr int kJvpWide = 8;
 
 // x and the K tangents of the state (OUT: of the vertex outputs) at i.  The columns past k repeat the
 // last one: every load is unconditional, and their results are not stored.
@@ -747,15 +749,15 @@ __device__ __forceinline__ DualK<K> jvp_load(const JvpKArgs& a, int64_t i) {
     return r;
 }
 
+// nbr: the neighbour's output (or, for ODE edges, the edge state)
 template <int EM, int WRAP, int K>
-__device__ __forceinline__ DualK<K> slot_value_k(int2 s, const DualK<K>& own, const JvpKArgs& a) {
+__device__ __forceinline__ DualK<K> slot_value_k(int2 s, const DualK<K>& own, const DualK<K>& nbr, const JvpKArgs& a) {
     if constexpr (EM == ND_EM_NOOP) {
         return nan_of<DualK<K>>();
     } else if constexpr (is_ode_model(EM)) {
-        return ode_side_k<K>(WRAP, jvp_load<K, false>(a, s.x), s.y & 1);
+        return ode_side_k<K>(WRAP, nbr, s.y & 1);
     } else {
         // one evaluation for either direction: a wave holds entries of both
-        const DualK<K> nbr = jvp_load<K, true>(a, s.x);
         const bool is_src = s.y & 1;
         DualK<K> from, to;
         from.v = is_src ? own.v : nbr.v;
@@ -793,6 +795,32 @@ __device__ __forceinline__ void wave_order() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+// Entry E of every 8 lanes (its neighbour in lane E's nbr): lane j fetches tangent j
+template <int E>
+__device__ __forceinline__ void jvp_rows(int32_t nbr, int t, const double* __restrict__ dvt, double* buf) {
+    if constexpr (E < kJvpWide) {
+        const int32_t r = __builtin_amdgcn_ds_swizzle(nbr, 0x18 | (E << 5));
+        const double d = dvt[static_cast<int64_t>(r) * kJvpWide + t % kJvpWide];
+        jvp_rows<E + 1>(nbr, t, dvt, buf);
+        buf[(t - t % kJvpWide + E) * (kJvpWide + 1) + 1 + t % kJvpWide] = d;
+    }
+}
+// Tangents row by row: o[i * kJvpWide + j] = output i's tangent along column j of v (columns past k
+// repeat the last), of every batch's vertices
+__global__ void __launch_bounds__(256) k_jvp_tangents(VGroup g, const double* __restrict__ v, int64_t ldv, int32_t k,
+                                                      double* __restrict__ o) {
+    const int i = group_of_block(g, static_cast<int32_t>(blockIdx.x));
+    const VDesc& vd = g.vd[i];
+    const int64_t q = static_cast<int64_t>(static_cast<int32_t>(blockIdx.x) - g.first[i]) * 256 + threadIdx.x;
+    if (q >= vd.count || vd.depth < 1) return;
+    const double* x = v + vd.state0 + q * vd.dim + vd.mask[0];
+    double d[kJvpWide];
+#pragma unroll
+    for (int j = 0; j < kJvpWide; ++j) d[j] = vd.outkind == 1 ? 0.0 : x[(j < k ? j : k - 1) * ldv];
+    double2* to = reinterpret_cast<double2*>(o + (vd.out0 + q) * kJvpWide);
+#pragma unroll
+    for (int j = 0; j < kJvpWide / 2; ++j) to[j] = make_double2(d[2 * j], d[2 * j + 1]);
 }
 // Up to kGroupMax vertex batches in one launch: batch i owns the blocks first[i] ..
 // first[i + 1] - 1, first one per row of more than kJvpRow entries (positions hubs[i]), then one
@@ -835,7 +863,8 @@ __device__ __forceinline__ void jvp_vertex(const VDesc& vd, int32_t q, int col, 
 // of more than kJvpRow entries.  A lane evaluates one entry on all K tangents at once (the sine and
 // cosine once per entry, 2 + K independent loads), the results pass through LDS, and lane j sums
 // the value and tangent j in the order of the row.
-// Bound by the neighbours' loads, K + 1 cache lines an entry.  Eight tangents of 1e5 vertices on
+// Bound by the neighbours' loads, K + 1 cache lines an entry; with the tangents row by row
+// (dvt), two: 34 us instead of 48, 8 of them the pass that lays them out.  Eight tangents of 1e5 vertices on
 // a geometric graph (two batches, 4 entries a row): 48 us, one tangent 15; a thread per vertex,
 // one launch per batch, took 75 and 52 (its few waves wait on one entry at a time, and evaluate
 // both directions of an edge where a wave holds both).  Preferential attachment, 100 003
@@ -863,11 +892,24 @@ __global__ void __launch_bounds__(256) k_vertex_jvp(JvpGroup g, const int32_t* _
         const DualK<K> own = jvp_load<K, false>(a, static_cast<int64_t>(vd.state0) + static_cast<int64_t>(q) * vd.dim + vd.mask[0]);
         for (int32_t s0 = beg; s0 < end; s0 += width) {
             const int32_t s = s0 + lane, count = end - s0 < width ? end - s0 : width;
+            const int2 sl = slots[lane < count ? s : end - 1];
+            double* to = buf + t * (K + 1);
+            DualK<K> nbr;
+            if (K == kJvpWide && !MULTI && !is_ode_model(EM) && a.dvt) {
+                // the 8 lanes of a group read one entry's row of tangents at a time, and turn them in LDS
+                wave_order();
+                jvp_rows<0>(sl.x, t, a.dvt, buf);
+                wave_order();
+                nbr.v = a.vo[sl.x];
+#pragma unroll
+                for (int j = 0; j < K; ++j) nbr.d[j] = to[1 + j];
+            } else if constexpr (!MULTI) {
+                nbr = jvp_load<K, !is_ode_model(EM)>(a, sl.x);
+            }
             if (lane < count) {
                 DualK<K> y;
-                if constexpr (MULTI) y = slot_value_k_rt<K>(ed[slot_eb[s]], slots[s], own, a);
-                else y = slot_value_k<EM, WRAP, K>(slots[s], own, a);
-                double* to = buf + t * (K + 1);
+                if constexpr (MULTI) y = slot_value_k_rt<K>(ed[slot_eb[s]], sl, own, a);
+                else y = slot_value_k<EM, WRAP, K>(sl, own, nbr, a);
                 to[0] = y.v;
 #pragma unroll
                 for (int j = 0; j < K; ++j) to[1 + j] = y.d[j];
@@ -2716,9 +2758,30 @@ int nd_rhs(nd_plan* pl, double* du, const double* u, const double* p, double t, 
     return hip_check(hipGetLastError(), "nd_rhs launch");
 }
 
+// whether k_vertex_jvp gathers tangents row by row (JvpKArgs::dvt)
+static bool jvp_rows_ok(const nd_plan* pl) {
+    return !pl->multi && !pl->edesc.empty() && !pl->edesc[0].ode && pl->edesc[0].model != ND_EM_NOOP;
+}
+static void launch_jvp_tangents(const std::vector<VDesc>& vds, const double* v, int64_t ldv, int32_t k, double* o,
+                                hipStream_t s) {
+    VGroup g{};
+    auto flush = [&]() {
+        if (g.n)
+            hipLaunchKernelGGL(k_jvp_tangents, dim3(static_cast<unsigned>(g.first[g.n])), dim3(256), 0, s, g, v, ldv, k, o);
+        g.n = 0;
+    };
+    for (const VDesc& vd : vds) {
+        if (!vd.count) continue;
+        g.vd[g.n] = vd;
+        g.first[g.n + 1] = g.first[g.n] + static_cast<int32_t>(blocks_for(vd.count, 256));
+        if (++g.n == kGroupMax) flush();
+    }
+    flush();
+}
+
 // the fused vertex batches of a Jacobian-vector product with a.k tangents
 static void launch_vertex_jvp(nd_plan* pl, const JvpKArgs& a, hipStream_t s) {
-    const VertexJvpKernel kern = a.k == 1 ? pl->vjvp1 : a.k <= 4 ? pl->vjvp4 : pl->vjvp8;
+    const VertexJvpKernel kern = a.k == 1 ? pl->vjvp1 : a.k <= 4 && !a.dvt ? pl->vjvp4 : pl->vjvp8;
     JvpGroup g{};
     auto flush = [&]() {
         if (g.n)
@@ -2803,6 +2866,12 @@ int nd_rhs_jvp(nd_plan* pl, double* du, double* jv, const double* u, const doubl
 
 int nd_rhs_jvp_multi(nd_plan* pl, double* du, double* jv, const double* u, const double* v, int32_t k,
                      const double* p, double t, int64_t len_du, int64_t len_u, int64_t len_p, void* stream) {
+    return nd_rhs_jvp_multi_work(pl, du, jv, u, v, k, p, t, nullptr, 0, len_du, len_u, len_p, stream);
+}
+
+int nd_rhs_jvp_multi_work(nd_plan* pl, double* du, double* jv, const double* u, const double* v, int32_t k,
+                          const double* p, double t, double* work, int64_t len_work, int64_t len_du, int64_t len_u,
+                          int64_t len_p, void* stream) {
     if (!pl) return nd::set_error(ND_ERR_ARGUMENT, "plan is NULL");
     if (k < 1 || k > 8) return nd::set_error(ND_ERR_ARGUMENT, "k = %d tangents: need 1 <= k <= 8", k);
     if (k == 1) return nd_rhs_jvp(pl, du, jv, u, v, p, t, len_du, len_u, len_p, stream);
@@ -2839,17 +2908,31 @@ int nd_rhs_jvp_multi(nd_plan* pl, double* du, double* jv, const double* u, const
             pl->allocations.push_back(w);
             pl->d_dvoutk = static_cast<double*>(w);
         }
+        // one launch for all columns instead of one per column: 300 001 vertices (preferential
+        // attachment), four columns: 107 us column by column, 84 row by row; two: 77 us and about 82
+        const bool rows = k > 2 && jvp_rows_ok(pl);
         for (const VDesc& vd : pl->vdesc) {
             if (!vd.count) continue;
             const unsigned vb = blocks_for(vd.count, 256);
             hipLaunchKernelGGL(k_vertex_out, dim3(vb), dim3(256), 0, s, vd, u, pl->d_vout, no_sync(vb), p, 0);
-            for (int j = 0; j < k; ++j)
+            for (int j = 0; j < k && !rows; ++j)
                 hipLaunchKernelGGL(k_vertex_out, dim3(vb), dim3(256), 0, s, vd, v + static_cast<int64_t>(j) * pl->dim,
                                    pl->d_dvoutk + static_cast<int64_t>(j) * pl->vout_len, no_sync(vb), p, 1);
         }
         a.vo = pl->d_vout;
         a.dvo = pl->d_dvoutk;
         a.ldo = pl->vout_len;
+        if (rows) {
+            a.dvt = pl->d_dvoutk;
+            launch_jvp_tangents(pl->vdesc, v, pl->dim, k, pl->d_dvoutk, s);
+        }
+    } else if (k > 4 && work && len_work >= kJvpWide * pl->dim && (reinterpret_cast<uintptr_t>(work) & 15) == 0 &&
+               jvp_rows_ok(pl)) {
+        VDesc all{};                  // the slots address the state: one vertex per entry of it
+        all.dim = all.depth = 1;
+        all.count = static_cast<int32_t>(pl->dim);
+        a.dvt = work;
+        launch_jvp_tangents({all}, v, pl->dim, k, work, s);
     }
     launch_vertex_jvp(pl, a, s);
     for (const EDesc& e : pl->edesc) {

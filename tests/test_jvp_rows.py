@@ -58,3 +58,12 @@ def test_rows_of_every_length(ND, dev, kind, gather):
         duk, jvk = nan(nw.dim), nan(8, nw.dim)
         nw.jvp_multi(duk, jvk[:k], ud, Vd[:k], pd, 0.0)
         assert torch.equal(duk, du) and torch.equal(jvk[:k], jv[:k]) and bool(jvk[k:].isnan().all())
+        # with scratch memory: the tangents of more than four columns row by row; a scratch too short
+        # or not 16-byte aligned is not used
+        work = nan(8 * nw.dim + 1)
+        for first, length in ((0, 8 * nw.dim), (1, 8 * nw.dim), (0, 8 * nw.dim - 1)):
+            duk, jvk = nan(nw.dim), nan(8, nw.dim)
+            ND._abi.check(ND._abi.lib().nd_rhs_jvp_multi_work(
+                nw.plan, duk.data_ptr(), jvk.data_ptr(), ud.data_ptr(), Vd.data_ptr(), k, pd.data_ptr(), 0.0,
+                work.data_ptr() + 8 * first, length, nw.dim, nw.dim, nw.pdim, torch.cuda.current_stream(dev).cuda_stream))
+            assert torch.equal(duk, du) and torch.equal(jvk[:k], jv[:k]) and bool(jvk[k:].isnan().all())
