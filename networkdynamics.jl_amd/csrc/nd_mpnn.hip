@@ -450,14 +450,15 @@ __device__ __forceinline__ void product64(const float* Ws, const float* T, int l
 
 // Hout = relu((A H) W + H U + bias), W and U the halves of WU (64 x 128); with `out` also the
 // head out = Hout w_out + b_out.
-// At 773 293 nodes of 3.2 entries: 175 us, of which the matrix cores are busy for 81 (128 x 64
-// products at 153 TFLOP/s); reading and writing H alone takes 102.  Both overlap only in part:
+// At 773 293 nodes of 3.2 entries: 180 us, of which the matrix cores are busy for 81 (128 x 64
+// products at 153 TFLOP/s); reading and writing H alone takes 106.  Both overlap only in part:
 // the registers allow 16 waves a CU, and the neighbours' rows come from L2 with some 460 cycles
-// each.  What mattered, from 262 us: whole rows per access (64-byte pieces of 16 rows met lines
-// still on their way to L1, 262 -> 243 with the gather turned), all other loads likewise and
-// neighbouring tiles on different CUs (234 -> 191), stores past L2, which leave it to the
-// rows that are gathered, and one workgroup of 16 waves (191 -> 175).  Four entries of each node in flight
-// instead of two, wave priorities and skipping padded entries measured the same.
+// each.  What mattered, from 268 us: whole rows per access in the gather (64-byte pieces of 16
+// rows meet lines still on their way to L1; 247), the same for all other loads, and
+// neighbouring tiles on different CUs (239 -> 195), stores past L2, which leave it to the rows
+// that are gathered, and one workgroup of 16 waves (195 -> 180).  Four entries of each node in
+// flight instead of two, wave priorities and skipping padded entries measured the same; 20
+// waves of 96 registers 948 us a forward pass against 777.
 template <int NT, bool WIDE>
 __global__ void __launch_bounds__(NT, NT / 256) k_layer(int64_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ nbr,
                                                  const float* __restrict__ a, const float* __restrict__ H,
