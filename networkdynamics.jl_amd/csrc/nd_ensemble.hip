@@ -15,7 +15,7 @@
 // (first-order Kuramoto, RK4, 16 waves of one CU) takes 2.47 us per evaluation with the vector
 // units 67 % busy and the LDS 60 %; with an index list per row entry, a bound on every entry
 // and the longer sine it took 3.61 us.  1024 swing networks of 100 to 2000 vertices (Tsit5 to
-// t = 10, default classes) take 38.4 ms, against 69.0 ms; at four vertices per thread the
+// t = 10, default classes) take 39.7 ms, against 66.7 ms; at four vertices per thread the
 // vector units are 60 % busy with two waves per SIMD.
 //
 // Methods: Tsit5 (Tsitouras 2011) with the PI step-size controller of
