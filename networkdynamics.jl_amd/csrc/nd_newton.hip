@@ -79,10 +79,34 @@ using namespace nd;
 
 // a / b from y = 1.0 / b, both correctly rounded: one correction of the rounded product
 // a * y by its remainder gives the rounded quotient (Markstein 1990), with three operations
-// in place of a division's dozen
+// in place of a division's dozen.  The same bits as a division where a, b, y and the quotient
+// are normal numbers and the remainder does not underflow (|a| > 2^-960); not finite where y
+// or the quotient overflows or b is infinite (the caller divides there).
 __device__ __forceinline__ double quotient(double a, double b, double y) {
     const double q = a * y;
     return __builtin_fma(__builtin_fma(-q, b, a), y, q);
+}
+
+// z = r / dg, returns the thread's part of r . z.  A z that is not finite makes that sum not
+// finite, so one test finds every quotient to be divided out.
+template <int V>
+__device__ __forceinline__ double precondition(const double (&r)[V], const double (&dg)[V], const double (&dgi)[V],
+                                               double (&z)[V]) {
+    double rz = 0.0;
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+        z[k] = quotient(r[k], dg[k], dgi[k]);
+        rz += r[k] * z[k];
+    }
+    if (__builtin_expect(!(fabs(rz) <= 0x1.fffffffffffffp+1023), 0)) {
+        rz = 0.0;
+#pragma unroll
+        for (int k = 0; k < V; ++k) {
+            z[k] = r[k] / dg[k];
+            rz += r[k] * z[k];
+        }
+    }
+    return rz;
 }
 
 template <int V>
@@ -217,7 +241,7 @@ __global__ void __launch_bounds__(kThreads) k_newton(NewtonArgs a) {
         }
         __syncthreads();
         // CG for L_w d = F, d mean-zero (F sums to zero when P is balanced)
-        double rz = 0.0, rr0 = 0.0;
+        double rz = 0.0, rr0 = 0.0, z[V];
 #pragma unroll
         for (int k = 0; k < V; ++k) {
             const int v = t + k * T;
@@ -225,11 +249,12 @@ __global__ void __launch_bounds__(kThreads) k_newton(NewtonArgs a) {
             r[k] = v < n ? r[k] - fmean : 0.0;
             dg[k] = v < n ? rowv[v] : 1.0;
             dgi[k] = 1.0 / dg[k];
-            const double z = quotient(r[k], dg[k], dgi[k]);
-            if (v < n) buf[v] = z;
-            rz += r[k] * z;
             rr0 += r[k] * r[k];
         }
+        rz = precondition(r, dg, dgi, z);
+#pragma unroll
+        for (int k = 0; k < V; ++k)
+            if (t + k * T < n) buf[t + k * T] = z[k];
         red.sum2(rz, rr0);
         const double eta = a.inexact ? fmax(a.cg_rtol, fmin(a.eta_max, res)) : a.cg_rtol;
         const double stop2 = eta * eta * rr0;
@@ -287,10 +312,9 @@ __global__ void __launch_bounds__(kThreads) k_newton(NewtonArgs a) {
             for (int k = 0; k < V; ++k) {
                 d[k] += alpha * pi[k];
                 r[k] -= alpha * q[k];
-                q[k] = quotient(r[k], dg[k], dgi[k]);
-                rzn += r[k] * q[k];
                 rrn += r[k] * r[k];
             }
+            rzn = precondition(r, dg, dgi, q);
             red.sum2(rzn, rrn);
             rr = rrn;
             const double beta = rzn / rz;
