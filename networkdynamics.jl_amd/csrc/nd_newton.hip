@@ -177,12 +177,14 @@ __global__ void __launch_bounds__(kThreads) k_newton(NewtonArgs a) {
         for (int j = 0; j < nc; ++j) {
             const int jn = j1;
             const double kv = k1;
+            // padding adds 0 whatever the row's own angle is: a vertex without lines has no equation
+            const bool pad = e1 < 0;
             if (j + 1 < nc) {
                 e1 = se[(c0 + j + 1) * kWave];
                 j1 = nb[(c0 + j + 1) * kWave];
                 k1 = e1 >= 0 ? a.K[e1] : 0.0;
             }
-            term(c0 + j, kv, at(jn) - own);
+            term(c0 + j, kv, pad ? 0.0 : at(jn) - own);
         }
     };
 

@@ -25,3 +25,22 @@ def test_weights_that_sum_past_the_largest_double(ND, dev, n):
     assert st["retcode"][0] == 0 and st["newton_iters"][0] == 1
     assert np.isfinite(th).all()
     np.testing.assert_allclose(th[1:3] - th[0], [1e-208, -1e-208], rtol=1e-12)
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+@pytest.mark.parametrize("n", [70, 2100])
+def test_angle_of_a_vertex_without_lines(ND, dev, n, bad):
+    # the last vertex has no lines, so its angle enters no equation: a path of the others is solved
+    # as it is without that vertex, whatever the angle is
+    g = ND.SimpleGraph(n, np.arange(1, n - 1), np.arange(2, n))
+    rng = np.random.default_rng(3)
+    P = np.r_[rng.normal(0.0, 0.01, n - 1), 0.0]
+    P[:-1] -= P[:-1].mean()
+    K = rng.uniform(5.0, 10.0, n - 2)
+    theta = np.zeros(n)
+    ref, st0 = _solve(ND, dev, [g], P, K, theta)
+    assert st0["retcode"][0] == 0
+    theta[-1] = bad
+    th, st = _solve(ND, dev, [g], P, K, theta)
+    assert st["retcode"][0] == 0 and st["newton_iters"][0] == st0["newton_iters"][0]
+    assert np.array_equal(th[:-1], ref[:-1])
