@@ -868,7 +868,7 @@ __global__ void __launch_bounds__(256) k_jvp_tangents(VGroup g, const double* __
 }
 // Up to kGroupMax vertex batches in one launch: batch i owns the blocks first[i] ..
 // first[i + 1] - 1, first one per row of more than kJvpRow entries (positions hubs[i]), then one
-// per 32 vertices.
+// per 32 vertices (256 with a thread per vertex).
 constexpr int kJvpRow = 64, kJvpLanes = 8;
 struct JvpGroup {
     VDesc vd[kGroupMax];
@@ -903,19 +903,88 @@ __device__ __forceinline__ void jvp_vertex(const VDesc& vd, int32_t q, int col, 
     }
 }
 
+// du and the k columns of jv of vertex q from its states (two at most) and its aggregate
+template <int VM, int K>
+__device__ __forceinline__ void jvp_columns(const VDesc& vd, int32_t q, const DualK<K> (&x)[2], const DualK<K>& acc,
+                                            const JvpKArgs& a) {
+    constexpr int DIMC = VModel<VM>::dim;
+    const int dim = DIMC > 0 ? DIMC : vd.dim;
+    const int64_t x0 = static_cast<int64_t>(vd.state0) + static_cast<int64_t>(q) * dim;
+    if constexpr (VM == ND_VM_NOOP) {
+        for (int j = 0; j < dim; ++j) dk_store<K>(a.du, a.jv, a.ldu, a.k, x0 + j, zero_of<DualK<K>>());
+    } else {
+        static_assert(DIMC <= 2, "one or two states");
+        DualK<K> dx[DIMC];
+        vertex_f<VM, DualK<K>>(dx, x, acc, a.p + vd.param0 + static_cast<int64_t>(q) * vd.pdim, DIMC);
+#pragma unroll
+        for (int j = 0; j < DIMC; ++j) dk_store<K>(a.du, a.jv, a.ldu, a.k, x0 + j, dx[j]);
+    }
+}
+
+// The thread of a vertex: its row two entries at a time, in order, and the slots of the next two
+// with them
+template <int EM, int WRAP, bool MULTI, int K>
+__device__ __forceinline__ void jvp_near(const VDesc& vd, int32_t q, const int32_t* __restrict__ rowptr,
+                                         const int2* __restrict__ slots, const uint8_t* __restrict__ slot_eb,
+                                         const EDesc* __restrict__ ed, const JvpKArgs& a) {
+    if (q >= vd.count) return;
+    DualK<K> x[2], acc = zero_of<DualK<K>>();
+    if (vd.model != ND_VM_NOOP) {
+        const int32_t beg = rowptr[vd.row0 + q], end = rowptr[vd.row0 + q + 1];
+        if (end - beg > kJvpRow) return;
+        // all states at once, before the entries push their lines out of L1
+        const int64_t x0 = static_cast<int64_t>(vd.state0) + static_cast<int64_t>(q) * vd.dim;
+        x[0] = dk_load<K>(a.u, a.v, a.ldu, a.k, x0);
+        x[1] = vd.dim == 2 ? dk_load<K>(a.u, a.v, a.ldu, a.k, x0 + 1) : x[0];
+        const DualK<K> own = vd.mask[0] == 0 ? x[0] : x[1];
+        const int32_t last = end - 1;
+        int2 s0 = make_int2(0, 0), s1 = s0;
+        if (beg < end) {
+            s0 = slots[beg];
+            s1 = slots[min(beg + 1, last)];
+        }
+        for (int32_t s = beg; s < end; s += 2) {
+            const int2 c0 = s0, c1 = s1;
+            if constexpr (MULTI) {
+                acc = acc + slot_value_k_rt<K>(ed[slot_eb[s]], c0, own, a);
+                if (s + 1 < end) acc = acc + slot_value_k_rt<K>(ed[slot_eb[s + 1]], c1, own, a);
+                s0 = slots[min(s + 2, last)];
+                s1 = slots[min(s + 3, last)];
+            } else {
+                constexpr bool OUT = !is_ode_model(EM);
+                const DualK<K> n0 = dk_load<K>(OUT ? a.vo : a.u, OUT ? a.dvo : a.v, OUT ? a.ldo : a.ldu, a.k, c0.x);
+                const DualK<K> n1 = dk_load<K>(OUT ? a.vo : a.u, OUT ? a.dvo : a.v, OUT ? a.ldo : a.ldu, a.k, c1.x);
+                s0 = slots[min(s + 2, last)];
+                s1 = slots[min(s + 3, last)];
+                acc = acc + slot_value_k<EM, WRAP, K>(c0, own, n0, a);
+                if (s + 1 < end) acc = acc + slot_value_k<EM, WRAP, K>(c1, own, n1, a);
+            }
+        }
+    }
+    switch (vd.model) {
+    case ND_VM_DIFFUSION: return jvp_columns<ND_VM_DIFFUSION, K>(vd, q, x, acc, a);
+    case ND_VM_KURAMOTO: return jvp_columns<ND_VM_KURAMOTO, K>(vd, q, x, acc, a);
+    case ND_VM_SWING: return jvp_columns<ND_VM_SWING, K>(vd, q, x, acc, a);
+    case ND_VM_SWING_UNIT_DAMPING: return jvp_columns<ND_VM_SWING_UNIT_DAMPING, K>(vd, q, x, acc, a);
+    case ND_VM_LOAD: return jvp_columns<ND_VM_LOAD, K>(vd, q, x, acc, a);
+    default: return jvp_columns<ND_VM_NOOP, K>(vd, q, x, acc, a);
+    }
+}
+
 // The fused vertex batches, k <= K tangents: 8 lanes per vertex, or a whole workgroup for a row
-// of more than kJvpRow entries.  A lane evaluates one entry on all K tangents at once (the sine and
-// cosine once per entry, 2 + K independent loads), the results pass through LDS, and lane j sums
-// the value and tangent j in the order of the row.
-// Bound by the neighbours' loads, K + 1 cache lines an entry; with the tangents row by row
-// (dvt), two: 34 us instead of 48, 8 of them the pass that lays them out.  Eight tangents of 1e5 vertices on
-// a geometric graph (two batches, 4 entries a row): 48 us, one tangent 15; a thread per vertex,
-// one launch per batch, took 75 and 52 (its few waves wait on one entry at a time, and evaluate
-// both directions of an edge where a wave holds both).  Preferential attachment, 100 003
+// of more than kJvpRow entries.  NEAR: a thread per vertex in place of the 8 lanes, for networks
+// whose numbering puts neighbours together (jvp_near_columns has the times of both).
+// A lane evaluates one entry on all K tangents at once (the sine and cosine once per entry,
+// 2 + K independent loads), the results pass through LDS, and lane j sums the value and tangent j
+// in the order of the row.
+// Bound by the neighbours' loads, K + 1 cache lines an entry; with the tangents row by row (dvt),
+// two: 34 us instead of 48, 8 of them the pass that lays them out.  Eight tangents of 1e5 vertices
+// on a geometric graph in random order (two batches, 4 entries a row): 48 us, one tangent 15; a
+// thread per vertex, one launch per batch, took 75 and 52.  Preferential attachment, 100 003
 // vertices and rows up to about 900: 56 and 33 against 1037 and 652, one thread per row.
 // 2 / 4 / 8 lanes per vertex: 54 / 50 / 48 us for eight tangents, 15.3 / 14.0 / 14.6 for one;
 // lanes that share a vertex's entries and split its tangents, 57 to 60.
-template <int EM, int WRAP, bool MULTI, int K>
+template <int EM, int WRAP, bool MULTI, int K, bool NEAR>
 __global__ void __launch_bounds__(256) k_vertex_jvp(JvpGroup g, const int32_t* __restrict__ rowptr,
                                                     const int2* __restrict__ slots, const uint8_t* __restrict__ slot_eb,
                                                     const EDesc* __restrict__ ed, JvpKArgs a) {
@@ -925,6 +994,11 @@ __global__ void __launch_bounds__(256) k_vertex_jvp(JvpGroup g, const int32_t* _
     const VDesc& vd = g.vd[i];
     const int32_t b = static_cast<int32_t>(blockIdx.x) - g.first[i];
     const bool hub = b < g.nhub[i];
+    if constexpr (NEAR)
+        if (!hub) {
+            jvp_near<EM, WRAP, MULTI, K>(vd, (b - g.nhub[i]) * 256 + static_cast<int32_t>(threadIdx.x), rowptr, slots, slot_eb, ed, a);
+            return;
+        }
     const int t = threadIdx.x, lane = hub ? t : t % kJvpLanes, width = hub ? 256 : kJvpLanes, base = t - lane;
     const int32_t q = hub ? g.hubs[i][b] : (b - g.nhub[i]) * (256 / kJvpLanes) + t / kJvpLanes;
     if (q >= vd.count) return;
@@ -1828,34 +1902,34 @@ EdgeOdeJvpKernel pick_edge_ode_jvp(int em) {
 
 using VertexJvpKernel = void (*)(JvpGroup, const int32_t*, const int2*, const uint8_t*, const EDesc*, JvpKArgs);
 
-template <int K>
+template <int K, bool NEAR>
 VertexJvpKernel pick_vertex_jvp(int em, int wrap, bool multi) {
-    if (multi) return k_vertex_jvp<ND_EM_NOOP, ND_WRAP_NONE, true, K>;
+    if (multi) return k_vertex_jvp<ND_EM_NOOP, ND_WRAP_NONE, true, K, NEAR>;
     const bool sym = wrap == ND_WRAP_SYMMETRIC;
     switch (em) {
     case ND_EM_KURAMOTO:
-        return sym ? k_vertex_jvp<ND_EM_KURAMOTO, ND_WRAP_SYMMETRIC, false, K>
-                   : k_vertex_jvp<ND_EM_KURAMOTO, ND_WRAP_ANTISYMMETRIC, false, K>;
+        return sym ? k_vertex_jvp<ND_EM_KURAMOTO, ND_WRAP_SYMMETRIC, false, K, NEAR>
+                   : k_vertex_jvp<ND_EM_KURAMOTO, ND_WRAP_ANTISYMMETRIC, false, K, NEAR>;
     case ND_EM_STATIC_LINE:
-        return sym ? k_vertex_jvp<ND_EM_STATIC_LINE, ND_WRAP_SYMMETRIC, false, K>
-                   : k_vertex_jvp<ND_EM_STATIC_LINE, ND_WRAP_ANTISYMMETRIC, false, K>;
+        return sym ? k_vertex_jvp<ND_EM_STATIC_LINE, ND_WRAP_SYMMETRIC, false, K, NEAR>
+                   : k_vertex_jvp<ND_EM_STATIC_LINE, ND_WRAP_ANTISYMMETRIC, false, K, NEAR>;
     case ND_EM_DIFFUSION:
-        return sym ? k_vertex_jvp<ND_EM_DIFFUSION, ND_WRAP_SYMMETRIC, false, K>
-                   : k_vertex_jvp<ND_EM_DIFFUSION, ND_WRAP_ANTISYMMETRIC, false, K>;
+        return sym ? k_vertex_jvp<ND_EM_DIFFUSION, ND_WRAP_SYMMETRIC, false, K, NEAR>
+                   : k_vertex_jvp<ND_EM_DIFFUSION, ND_WRAP_ANTISYMMETRIC, false, K, NEAR>;
     case ND_EM_DIFFUSION_WEIGHTED:
-        return sym ? k_vertex_jvp<ND_EM_DIFFUSION_WEIGHTED, ND_WRAP_SYMMETRIC, false, K>
-                   : k_vertex_jvp<ND_EM_DIFFUSION_WEIGHTED, ND_WRAP_ANTISYMMETRIC, false, K>;
+        return sym ? k_vertex_jvp<ND_EM_DIFFUSION_WEIGHTED, ND_WRAP_SYMMETRIC, false, K, NEAR>
+                   : k_vertex_jvp<ND_EM_DIFFUSION_WEIGHTED, ND_WRAP_ANTISYMMETRIC, false, K, NEAR>;
     case ND_EM_DIFFUSION_FIDUCIAL:
-        return k_vertex_jvp<ND_EM_DIFFUSION_FIDUCIAL, ND_WRAP_ANTISYMMETRIC, false, K>;
+        return k_vertex_jvp<ND_EM_DIFFUSION_FIDUCIAL, ND_WRAP_ANTISYMMETRIC, false, K, NEAR>;
     case ND_EM_ODE_SIN_DIFFUSION:
     case ND_EM_ODE_SIN_DIFFUSION_FAST:
     case ND_EM_ODE_LINEAR:
     case ND_EM_ODE_LAG:
     case ND_EM_EXT_DRIVEN:
-        return wrap == ND_WRAP_ANTISYMMETRIC ? k_vertex_jvp<ND_EM_ODE_LINEAR, ND_WRAP_ANTISYMMETRIC, false, K>
-                                             : k_vertex_jvp<ND_EM_ODE_LINEAR, ND_WRAP_FIDUCIAL, false, K>;
+        return wrap == ND_WRAP_ANTISYMMETRIC ? k_vertex_jvp<ND_EM_ODE_LINEAR, ND_WRAP_ANTISYMMETRIC, false, K, NEAR>
+                                             : k_vertex_jvp<ND_EM_ODE_LINEAR, ND_WRAP_FIDUCIAL, false, K, NEAR>;
     default:
-        return k_vertex_jvp<ND_EM_NOOP, ND_WRAP_NONE, false, K>;
+        return k_vertex_jvp<ND_EM_NOOP, ND_WRAP_NONE, false, K, NEAR>;
     }
 }
 
@@ -1955,7 +2029,8 @@ struct nd_plan {
     std::vector<VertexKernel> vkern, vkern_stage;
     GroupKernel gkern = nullptr, gkern_stage = nullptr;   // several fused-set batches per launch
     std::vector<JvpKernel> vkern_jvp;                    // the batches of the generic kernels; null for the fused ones
-    VertexJvpKernel vjvp1 = nullptr, vjvp4 = nullptr, vjvp8 = nullptr;
+    VertexJvpKernel vjvp[3] = {}, vjvp_near[3] = {};      // 1, 4 and 8 tangents
+    int32_t jvp_near_k = 0;                              // tangents up to which vjvp_near is used
     std::vector<int32_t> jvp_hub_first;                  // per batch: its long rows in d_jvp_hubs
     int32_t* d_jvp_hubs = nullptr;
     double* d_dvoutk = nullptr;                          // 8 tangent columns of the vertex outputs
@@ -2218,6 +2293,69 @@ int rebuild_hubs(nd_plan* pl) {
 // once the network is large enough that its states do not stay in L2; below that the
 // vertex kernel reads u directly and one RHS is one launch per vertex batch.
 constexpr int64_t kCompactMinVertices = 1 << 18;
+// Cache lines per entry of the loads of a thread per vertex: of 64 consecutive vertices' first,
+// second, ... eighth entries, in about 256 waves spread over the network.  1/16 for a path, 0.14 for
+// a square lattice of swing vertices, 0.25 for a ring of them with one line in ten redirected, 0.31
+// for a geometric graph numbered cell by cell, about 1 for random numbers.
+double jvp_lines(const nd_plan* pl) {
+    int64_t waves = 0, lines = 0, entries = 0, w = 0;
+    for (const VDesc& vd : pl->vdesc) waves += (vd.count + kWave - 1) / kWave;
+    const int64_t step = std::max<int64_t>(1, waves / 256);
+    std::vector<int32_t> at;
+    for (const VDesc& vd : pl->vdesc)
+        for (int32_t q0 = 0; q0 < vd.count; q0 += kWave, ++w) {
+            if (w % step || vd.model == ND_VM_NOOP) continue;
+            for (int32_t j = 0; j < 8; ++j) {
+                at.clear();
+                for (int32_t q = q0; q < std::min(q0 + kWave, vd.count); ++q) {
+                    const int32_t beg = pl->rowptr_host[vd.row0 + q], len = pl->rowptr_host[vd.row0 + q + 1] - beg;
+                    if (j < len && len <= kJvpRow) at.push_back(pl->slots_host[static_cast<size_t>(beg) + j].x / 16);
+                }
+                if (at.empty()) break;
+                entries += static_cast<int64_t>(at.size());
+                std::sort(at.begin(), at.end());
+                lines += std::unique(at.begin(), at.end()) - at.begin();
+            }
+        }
+    return entries ? static_cast<double>(lines) / static_cast<double>(entries) : 0.0;
+}
+
+// The largest number of tangents that a thread per vertex (NEAR of k_vertex_jvp) serves better than
+// eight lanes per vertex; 0 where it never does.  It issues a third of the loads, which counts where
+// a wave's load meets few cache lines, and it walks a row two entries at a time, which needs many
+// vertices and short rows to hide.  Device time in us, eight lanes / a thread per vertex, for 1, 4 and
+// 8 tangents (lines: jvp_lines):
+//   path, 2e5 vertices                 lines 0.08   14.5 / 5.4    21.0 / 8.4    30.6 / 13.3
+//   swing lattice, 100^2                     0.15    4.2 / 4.2     4.6 / 5.4     5.9 / 6.8
+//   swing lattice, 200^2                     0.14    5.9 / 4.5     7.2 / 5.9    11.1 / 8.3
+//   swing lattice, 450^2                     0.14   19.6 / 9.9    26.8 / 20.5   38.7 / 37.5
+//   ring, 10 % redirected, 2e5               0.19   16.9 / 11.0   22.1 / 16.8   31.1 / 26.7
+//   ring, 30 % redirected, 2e5               0.39   17.6 / 14.5   24.9 / 28.1   42.1 / 51.3
+//   swing ring, 10 % redirected, 3e4         0.25    5.2 / 5.4     6.2 / 7.2     8.1 / 10.0
+//   swing ring, 30 % redirected, 1e5         0.46   11.9 / 9.9    17.9 / 17.6   28.3 / 30.9
+//   geometric, numbered by cells, 1e5        0.31   12.9 / 11.5   17.4 / 16.7   23.5 / 25.1
+//   geometric, numbered by cells, 2e5        0.31   22.9 / 17.7   28.8 / 29.4   40.4 / 48.6
+//   the same, 5e5 (compact outputs)          0.22   56.6 / 38.3    120 / 62.6    126 / 99.1
+//   ring, 30 %, 5e5 (compact outputs)        0.39   48.7 / 45.3   99.4 / 93.9    102 / 161
+//   geometric, random numbers, 1e5           1.00   16.0 / 17.5   32.3 / 34.3   61.3 / 62.2
+//   ring with 40 lines a row, 1e5            0.08   30.9 / 41.6   35.6 / 53.0   46.3 / 68.1
+//   ODE edges on a ring, 2e5                 0.35   20.9 / 18.7   31.7 / 37.8   51.9 / 72.8
+int32_t jvp_near_columns(const nd_plan* pl, double share) {
+    int64_t count = 0, total = 0;
+    for (const VDesc& vd : pl->vdesc) {
+        if (vd.generic || vd.depth > 1) return 0;
+        count += vd.count;
+        total += pl->rowptr_host[vd.row0 + vd.count] - pl->rowptr_host[vd.row0];
+    }
+    // 8192 vertices for each entry of a mean row
+    if (8192.0 * static_cast<double>(total) > static_cast<double>(count) * static_cast<double>(count) || share > 0.5) return 0;
+    const bool ode = !pl->edesc.empty() && pl->edesc[0].ode;
+    if (share <= 0.2 && !ode) return 8;
+    // how many columns stay in the L2s
+    const double most = ode ? 1.1 : pl->use_vout ? 2.0 : count <= 131072 ? 2.5 : 1.85;
+    return std::min<int32_t>(8, static_cast<int32_t>(most / share) - 1);
+}
+
 int apply_gather_mode(nd_plan* pl) {
     int64_t nv = 0;
     for (const VDesc& vd : pl->vdesc) nv += vd.count;
@@ -2227,6 +2365,9 @@ int apply_gather_mode(nd_plan* pl) {
     pl->kcache = pl->kcache_ok && pl->use_vout;
     const std::vector<int32_t>& x = pl->use_vout ? pl->slot_oidx : pl->slot_uidx;
     for (size_t k = 0; k < pl->slots_host.size(); ++k) pl->slots_host[k].x = x[k];
+    const bool large = nv >= 8192;
+    const double share = large ? jvp_lines(pl) : 1.0;
+    pl->jvp_near_k = large ? jvp_near_columns(pl, share) : 0;
     release(pl, pl->d_slots);
     pl->d_slots = nullptr;
     int rc = upload(pl, pl->slots_host, &pl->d_slots);
@@ -2683,9 +2824,12 @@ int nd_plan_create(const nd_network* h, nd_plan** out) {
         pl->vdesc.push_back(vd);
         pl->vkern_jvp.push_back(vd.depth > 1 ? k_vertex_vec_jvp : vd.generic ? pick_gen_jvp(k.model) : nullptr);
     }
-    pl->vjvp1 = pick_vertex_jvp<1>(em0, wrap0, pl->multi);
-    pl->vjvp4 = pick_vertex_jvp<4>(em0, wrap0, pl->multi);
-    pl->vjvp8 = pick_vertex_jvp<8>(em0, wrap0, pl->multi);
+    pl->vjvp[0] = pick_vertex_jvp<1, false>(em0, wrap0, pl->multi);
+    pl->vjvp[1] = pick_vertex_jvp<4, false>(em0, wrap0, pl->multi);
+    pl->vjvp[2] = pick_vertex_jvp<8, false>(em0, wrap0, pl->multi);
+    pl->vjvp_near[0] = pick_vertex_jvp<1, true>(em0, wrap0, pl->multi);
+    pl->vjvp_near[1] = pick_vertex_jvp<4, true>(em0, wrap0, pl->multi);
+    pl->vjvp_near[2] = pick_vertex_jvp<8, true>(em0, wrap0, pl->multi);
     {
         std::vector<int32_t> hubs;
         for (const VDesc& vd : pl->vdesc) {
@@ -2847,7 +2991,8 @@ static void launch_jvp_tangents(const std::vector<VDesc>& vds, const double* v, 
 
 // the fused vertex batches of a Jacobian-vector product with a.k tangents
 static void launch_vertex_jvp(nd_plan* pl, const JvpKArgs& a, hipStream_t s) {
-    const VertexJvpKernel kern = a.k == 1 ? pl->vjvp1 : a.k <= 4 && !a.dvt ? pl->vjvp4 : pl->vjvp8;
+    const bool near = a.k <= pl->jvp_near_k;
+    const VertexJvpKernel kern = (near ? pl->vjvp_near : pl->vjvp)[a.k == 1 ? 0 : a.k <= 4 && !a.dvt ? 1 : 2];
     JvpGroup g{};
     auto flush = [&]() {
         if (g.n)
@@ -2861,7 +3006,7 @@ static void launch_vertex_jvp(nd_plan* pl, const JvpKArgs& a, hipStream_t s) {
         g.vd[g.n] = vd;
         g.hubs[g.n] = pl->d_jvp_hubs + pl->jvp_hub_first[b];
         g.nhub[g.n] = pl->jvp_hub_first[b + 1] - pl->jvp_hub_first[b];
-        g.first[g.n + 1] = g.first[g.n] + g.nhub[g.n] + static_cast<int32_t>(blocks_for(vd.count, 256 / kJvpLanes));
+        g.first[g.n + 1] = g.first[g.n] + g.nhub[g.n] + static_cast<int32_t>(blocks_for(vd.count, near ? 256 : 256 / kJvpLanes));
         if (++g.n == kGroupMax) flush();
     }
     flush();
@@ -2976,7 +3121,7 @@ int nd_rhs_jvp_multi_work(nd_plan* pl, double* du, double* jv, const double* u, 
         }
         // one launch for all columns instead of one per column: 300 001 vertices (preferential
         // attachment), four columns: 107 us column by column, 84 row by row; two: 77 us and about 82
-        const bool rows = k > 2 && jvp_rows_ok(pl);
+        const bool rows = k > 2 && jvp_rows_ok(pl) && k > pl->jvp_near_k;
         for (const VDesc& vd : pl->vdesc) {
             if (!vd.count) continue;
             const unsigned vb = blocks_for(vd.count, 256);
@@ -2993,7 +3138,7 @@ int nd_rhs_jvp_multi_work(nd_plan* pl, double* du, double* jv, const double* u, 
             launch_jvp_tangents(pl->vdesc, v, pl->dim, k, pl->d_dvoutk, s);
         }
     } else if (k > 4 && work && len_work >= kJvpWide * pl->dim && (reinterpret_cast<uintptr_t>(work) & 15) == 0 &&
-               jvp_rows_ok(pl)) {
+               jvp_rows_ok(pl) && k > pl->jvp_near_k) {
         VDesc all{};                  // the slots address the state: one vertex per entry of it
         all.dim = all.depth = 1;
         all.count = static_cast<int32_t>(pl->dim);
