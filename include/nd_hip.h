@@ -379,8 +379,12 @@ int nd_rhs_jvp(nd_plan* plan, double* du, double* jv, const double* u, const dou
 int nd_rhs_jvp_multi(nd_plan* plan, double* du, double* jv, const double* u, const double* v, int32_t k,
                      const double* p, double t, int64_t len_du, int64_t len_u, int64_t len_p, void* stream);
 /* The same with scratch memory: work, 8*dim device doubles (16-byte aligned; NULL or shorter: not
- * used) that the call may overwrite.  Large networks gather the tangents of more than four
- * columns from a copy in it with one row per state.  The results are the same bits. */
+ * used) that the call may overwrite.  Networks of one feed-forward edge batch that gather from u
+ * directly and whose numbering scatters neighbours then take the tangents of more than four columns
+ * from a copy in it with one row per state; others do not use it.  The results are the same
+ * bits.  nd_rhs_jvp_multi_scratch: the doubles that make k tangents of this plan faster, 0 where
+ * the copy is not used or takes longer than it saves. */
+int64_t nd_rhs_jvp_multi_scratch(const nd_plan* plan, int32_t k);
 int nd_rhs_jvp_multi_work(nd_plan* plan, double* du, double* jv, const double* u, const double* v, int32_t k,
                           const double* p, double t, double* work, int64_t len_work, int64_t len_du, int64_t len_u,
                           int64_t len_p, void* stream);

@@ -2031,6 +2031,7 @@ struct nd_plan {
     std::vector<JvpKernel> vkern_jvp;                    // the batches of the generic kernels; null for the fused ones
     VertexJvpKernel vjvp[3] = {}, vjvp_near[3] = {};      // 1, 4 and 8 tangents
     int32_t jvp_near_k = 0;                              // tangents up to which vjvp_near is used
+    double jvp_share = 1.0;                              // jvp_lines
     std::vector<int32_t> jvp_hub_first;                  // per batch: its long rows in d_jvp_hubs
     int32_t* d_jvp_hubs = nullptr;
     double* d_dvoutk = nullptr;                          // 8 tangent columns of the vertex outputs
@@ -2366,8 +2367,8 @@ int apply_gather_mode(nd_plan* pl) {
     const std::vector<int32_t>& x = pl->use_vout ? pl->slot_oidx : pl->slot_uidx;
     for (size_t k = 0; k < pl->slots_host.size(); ++k) pl->slots_host[k].x = x[k];
     const bool large = nv >= 8192;
-    const double share = large ? jvp_lines(pl) : 1.0;
-    pl->jvp_near_k = large ? jvp_near_columns(pl, share) : 0;
+    pl->jvp_share = large ? jvp_lines(pl) : 1.0;
+    pl->jvp_near_k = large ? jvp_near_columns(pl, pl->jvp_share) : 0;
     release(pl, pl->d_slots);
     pl->d_slots = nullptr;
     int rc = upload(pl, pl->slots_host, &pl->d_slots);
@@ -3075,6 +3076,25 @@ int nd_rhs_jvp(nd_plan* pl, double* du, double* jv, const double* u, const doubl
     return hip_check(hipGetLastError(), "nd_rhs_jvp launch");
 }
 
+// The copy of the tangents row by row costs a pass over all columns and saves k - 1 cache lines an
+// entry, which counts where the entries' lines are scattered and the columns outgrow the L2s.
+// Device time in us without / with it:
+//   random numbers, geometric    6e4 vertices, 1.2e5 states   k = 6 25.7 / 27.3   k = 7 29.7 / 27.4   k = 8 33.7 / 27.5
+//                                1e5, 2e5                      k = 5 40.3 / 38.7   k = 6 47.2 / 38.2   k = 8 61.3 / 39.1
+//                                2e5, 4e5                      k = 5 87.1 / 65.2   k = 8  138 / 67.5
+//   preferential attachment      3e4, 6e4                      k = 8 23.6 / 27.0
+//                                1e5, 2e5                      k = 5 33.9 / 39.7   k = 6 39.0 / 39.1   k = 8 51.3 / 40.0
+//                                2.5e5, 5e5                    k = 5 97.1 / 80.6   k = 8  157 / 82.6
+//   ring, 60 % redirected        1e5, 2e5                      k = 6 32.7 / 35.3   k = 8 41.7 / 35.8
+//   ring, 30 % redirected        1e5, 2e5                      k = 8 28.3 / 35.8
+int64_t nd_rhs_jvp_multi_scratch(const nd_plan* pl, int32_t k) {
+    if (!pl || k <= 4 || k > kJvpWide || pl->use_vout || pl->ff_out || !jvp_rows_ok(pl)) return 0;
+    for (size_t b = 0; b < pl->vdesc.size(); ++b)
+        if (pl->vdesc[b].count && pl->vkern_jvp[b]) return 0;
+    if (k <= pl->jvp_near_k || pl->jvp_share <= 0.5 || (k - 4) * pl->dim < 300000) return 0;
+    return kJvpWide * pl->dim;
+}
+
 int nd_rhs_jvp_multi(nd_plan* pl, double* du, double* jv, const double* u, const double* v, int32_t k,
                      const double* p, double t, int64_t len_du, int64_t len_u, int64_t len_p, void* stream) {
     return nd_rhs_jvp_multi_work(pl, du, jv, u, v, k, p, t, nullptr, 0, len_du, len_u, len_p, stream);
@@ -3119,9 +3139,11 @@ int nd_rhs_jvp_multi_work(nd_plan* pl, double* du, double* jv, const double* u, 
             pl->allocations.push_back(w);
             pl->d_dvoutk = static_cast<double*>(w);
         }
-        // one launch for all columns instead of one per column: 300 001 vertices (preferential
-        // attachment), four columns: 107 us column by column, 84 row by row; two: 77 us and about 82
-        const bool rows = k > 2 && jvp_rows_ok(pl) && k > pl->jvp_near_k;
+        // One launch for all columns instead of one per column, and rows to gather from.  In us, column
+        // by column / row by row: preferential attachment, 3e5 vertices, two 67 / about 82, three 84 / 88,
+        // four 105 / 90, eight 204 / 94; ring, 30 % redirected, 5e5, four 89 / 99, five 108 / 100;
+        // geometric, numbered by cells, 5e5, three 79 / 118, four 83 / 120, eight 128 / 126.
+        const bool rows = k > (pl->jvp_share > 0.5 ? 2 : 4) && k > pl->jvp_near_k && jvp_rows_ok(pl);
         for (const VDesc& vd : pl->vdesc) {
             if (!vd.count) continue;
             const unsigned vb = blocks_for(vd.count, 256);

@@ -463,12 +463,11 @@ class Network:
         else:
             pptr, np_ = (p.data_ptr(), p.numel()) if isinstance(p, torch.Tensor) else (None, 0)
         stream = _stream(du, torch)
-        # scratch for the tangents row by row: worth its pass where the columns pass an L2 (4 MB) and
-        # nearly all of a row's eight are used.  8 columns of 83 200 / 130 000 / 200 006 states: 25.8 / 48.3 /
-        # 55.9 us without, 24.8 / 33.6 / 51.3 with; 5 columns of 200 006: 43.4 and 50.0
-        work = torch.empty(8 * nu, dtype=torch.float64, device=u.device) if k >= 7 and nu >= 100_000 else None
+        # scratch for the tangents row by row, where the plan says that it pays
+        need = A.lib().nd_rhs_jvp_multi_scratch(self.plan, int(k)) if k > 4 else 0
+        work = torch.empty(need, dtype=torch.float64, device=u.device) if need else None
         A.check(A.lib().nd_rhs_jvp_multi_work(self.plan, dptr, jv.data_ptr(), uptr, v.data_ptr(), int(k), pptr, float(t),
-                                              work.data_ptr() if work is not None else None, 8 * nu, ndu, nu, np_, stream))
+                                              work.data_ptr() if need else None, need, ndu, nu, np_, stream))
 
     def jacobian(self, u, p, t=0.0, colored=True):
         """Dense Jacobian d(du)/du at u (dim x dim, float64 device tensor): the matrix
