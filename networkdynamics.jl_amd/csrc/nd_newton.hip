@@ -14,7 +14,9 @@
 // Layout: the rows (a vertex's lines) are taken in order of decreasing length and stored in
 // slices of 64, column by column: entry j of the slice's 64 rows is one contiguous column of
 // 64, padded to the slice's longest row (a few per cent after the sort).  Every read of a
-// column is one contiguous access of its wave, and all columns' reads are independent.
+// column is one contiguous access of its wave, and all columns' reads are independent.  Rows that
+// would widen their slice for the other 63 (hubs; long_rows chooses) are stored apart, entries
+// 64 j .. 64 j + 63 in one column, and a whole wave evaluates them, adding in order.
 //
 // Who does what: thread t sums the rows at positions t, t + 512, ... of that order and hands
 // each result over through LDS to the thread that owns the vertex; vertices t, t + 512, ...
@@ -50,7 +52,8 @@ constexpr int kThreads = 512;
 constexpr int kColBytes = kWave * (sizeof(double) + sizeof(uint16_t));   // one column in LDS
 
 struct GridDesc {
-    int32_t n, ncol;     // vertices, columns of all slices
+    int32_t n, ncol;     // vertices, columns of all slices and long rows
+    int32_t nlong, pad_; // long rows
     int64_t voff;        // vertex offset (theta, P, scale, perm)
     int64_t coff;        // column offset
     int64_t soff;        // slice offset
@@ -58,8 +61,9 @@ struct GridDesc {
 
 struct NewtonArgs {
     const GridDesc* grid;
-    const int2* slice;       // per slice of 64 positions: {first column, columns}
-    const uint16_t* perm;    // vertex of each row position
+    const int2* slice;       // per slice of 64 positions: {first column, columns}; then per long row: {first
+                             // column, entries}
+    const uint16_t* perm;    // vertex of each row position, the long rows' last
     const uint16_t* nbr;     // per entry: 8 x the neighbour (padding: 8 x the row's own vertex)
     const int32_t* slot_edge;// global edge index per entry, -1 for padding
     double* w;               // weight per entry (columns that do not fit LDS)
@@ -109,14 +113,31 @@ __device__ __forceinline__ double precondition(const double (&r)[V], const doubl
     return rz;
 }
 
-template <int V>
+// acc + x of lane 0, + x of lane 1, ... of the first count lanes and of the others up to a multiple
+// of 8, where x is 0
+__device__ __forceinline__ double add_in_order(double acc, double x, int count) {
+    const long long b = __double_as_longlong(x);
+    const int lo = static_cast<int>(b), hi = static_cast<int>(b >> 32);
+    for (int i = 0; i < count; i += 8) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const unsigned l = static_cast<unsigned>(__builtin_amdgcn_readlane(lo, i + j));
+            const unsigned h = static_cast<unsigned>(__builtin_amdgcn_readlane(hi, i + j));
+            acc += __longlong_as_double((static_cast<long long>(h) << 32) | l);
+        }
+    }
+    return acc;
+}
+
+// LONG: some grid of the launch has long rows (their code costs the others 2 to 3 %)
+template <int V, bool LONG>
 __global__ void __launch_bounds__(kThreads) k_newton(NewtonArgs a) {
     constexpr int T = kThreads, WPB = kThreads / kWave;
     const int t = static_cast<int>(threadIdx.x), lane = t & (kWave - 1);
     const int wv = __builtin_amdgcn_readfirstlane(t / kWave);
     const int g = a.first + static_cast<int>(blockIdx.x);
     const GridDesc G = a.grid[g];
-    const int n = G.n;
+    const int n = G.n, nr = LONG ? n - G.nlong : n;   // nr: rows in slices
     extern __shared__ double sm[];
     double* buf = sm;                          // theta or the CG search vector
     double* rowv = buf + n;                    // row results: F, the Jacobi diagonal, L_w p
@@ -135,7 +156,7 @@ __global__ void __launch_bounds__(kThreads) k_newton(NewtonArgs a) {
     // slice k of this wave, kept on lane k: {first column, columns}, columns < 0 in memory
     static_assert(V <= kWave, "a slice per lane");
     int2 mine = make_int2(0, 0);
-    if (lane < V && lane * T + wv * kWave < n) mine = sl[lane * WPB + wv];
+    if (lane < V && lane * T + wv * kWave < nr) mine = sl[lane * WPB + wv];
     if (mine.x + mine.y > cols_lds) mine.y = -mine.y;
     auto slice_of = [&](int k) {
         return make_int2(__builtin_amdgcn_readlane(mine.x, k), __builtin_amdgcn_readlane(mine.y, k));
@@ -160,7 +181,7 @@ __global__ void __launch_bounds__(kThreads) k_newton(NewtonArgs a) {
 #pragma unroll
     for (int k = 0; k < V; ++k) {
         const int v = t + k * T;
-        row[k] = v < n ? a.perm[G.voff + v] : -1;
+        row[k] = v < nr ? a.perm[G.voff + v] : -1;
         if (v < n) buf[v] = th[v];
     }
     __syncthreads();
@@ -188,16 +209,45 @@ __global__ void __launch_bounds__(kThreads) k_newton(NewtonArgs a) {
         }
     };
 
+    // f(vertex, first column, entries) for the long rows of this wave, and the sum of a lane's
+    // f(column) over a row's entries in order
+    auto long_rows = [&](auto f) {
+        if constexpr (!LONG) return;
+        for (int j = wv; j < G.nlong; j += WPB) {
+            const int2 S = sl[(nr + kWave - 1) / kWave + j];
+            f(static_cast<int>(a.perm[G.voff + nr + j]), __builtin_amdgcn_readfirstlane(S.x), __builtin_amdgcn_readfirstlane(S.y));
+        }
+    };
+    auto long_sum = [&](int c0, int len, auto f) {
+        double acc = 0.0;
+        for (int e = 0; e < len; e += kWave) {
+            const double x = e + lane < len ? f(c0 + e / kWave) : 0.0;
+            acc = add_in_order(acc, x, min(len - e, kWave));
+        }
+        return acc;
+    };
+    auto in_lds = [&](int c0, int len) { return c0 + (len + kWave - 1) / kWave <= cols_lds; };
+
     // F(theta) of every vertex into rowv, from the theta in buf; returns max |F/scale| over the
     // grid.  The library sin and cos, called out of line: a handful of evaluations per solve,
     // whose registers the CG loop needs.
     auto residual = [&]() {
         double m = 0.0;
+        long_rows([&](int v, int c0, int len) {
+            const double own = buf[v];
+            const double acc = long_sum(c0, len, [&](int c) {
+                const double kv = a.K[se[c * kWave]], D = at(nb[c * kWave]) - own;
+                return a.linearized ? kv * D : kv * sin_far(D);
+            });
+            const double F = a.P[G.voff + v] + acc;
+            if (lane == 0) rowv[v] = F;
+            m = MaxNanOp{}(m, fabs(F / a.scale[G.voff + v]));
+        });
 #pragma unroll 1
         for (int k = 0; k < V; ++k) {
-            if (k * T + wv * kWave >= n) break;
+            if (k * T + wv * kWave >= nr) break;
             const int i = t + k * T;
-            if (i < n) {
+            if (i < nr) {
                 const int v = a.perm[G.voff + i];
                 double acc = 0.0;
                 if (a.linearized) row_terms(k, buf[v], [&](int, double kv, double D) { acc += kv * D; });
@@ -224,11 +274,23 @@ __global__ void __launch_bounds__(kThreads) k_newton(NewtonArgs a) {
         }
         fmean = red.sum(fmean) / n;                 // its barrier: rowv may be written again
         // weights and Jacobi diagonal at the current theta
+        long_rows([&](int v, int c0, int len) {
+            const double own = buf[v];
+            const bool lds = in_lds(c0, len);
+            const double dsum = long_sum(c0, len, [&](int c) {
+                const double kv = a.K[se[c * kWave]], D = at(nb[c * kWave]) - own;
+                const double ws = a.linearized ? kv : kv * cos_far(D);
+                if (lds) wl[c * kWave] = ws;
+                else wg[c * kWave] = ws;
+                return ws;
+            });
+            if (lane == 0) rowv[v] = dsum > 0.0 ? dsum : 1.0;
+        });
 #pragma unroll 1
         for (int k = 0; k < V; ++k) {
-            if (k * T + wv * kWave >= n) break;
+            if (k * T + wv * kWave >= nr) break;
             const int i = t + k * T;
-            if (i < n) {
+            if (i < nr) {
                 const int v = a.perm[G.voff + i];
                 double dsum = 0.0;
                 const bool mem = slice_of(k).y < 0;
@@ -267,9 +329,18 @@ __global__ void __launch_bounds__(kThreads) k_newton(NewtonArgs a) {
             // L_w p of the thread's rows, two rows and four columns of each at a time: eight
             // neighbours and weights are on their way together.  Columns past a row's last
             // repeat it and are not added.
+            long_rows([&](int v, int c0, int len) {
+                const double own = buf[v];
+                const bool lds = in_lds(c0, len);
+                const double sum = long_sum(c0, len, [&](int c) {
+                    const double ws = lds ? wl[c * kWave] : wg[c * kWave];
+                    return ws * (own - at(lds ? nl[c * kWave] : nb[c * kWave]));
+                });
+                if (lane == 0) rowv[v] = sum;
+            });
 #pragma unroll
             for (int k = 0; k < V; k += 2) {
-                if (k * T + wv * kWave < n) {       // whole waves without rows do nothing
+                if (k * T + wv * kWave < nr) {       // whole waves without rows do nothing
                     const int2 Sa = slice_of(k), Sb = slice_of(k + 1);    // empty beyond the last slice
                     const int na = abs(Sa.y), nb_ = abs(Sb.y), ca = Sa.x + na - 1, cb = Sb.x + nb_ - 1;
                     const double oa = buf[max(row[k], 0)], ob = buf[max(row[k + 1], 0)];
@@ -363,6 +434,30 @@ __global__ void __launch_bounds__(kThreads) k_newton(NewtonArgs a) {
     }
 }
 
+// How many of a grid's rows, given by decreasing length, are long rows.  Modelled cost of a product
+// in cycles: the wave with the widest slices, kColumn per column, and the long rows over 8 waves.
+// Solves of 64 stars of 1500 / 5000 vertices: 7.5 / 28 ms with every row in a slice, 0.54 / 1.6 so (4.6 /
+// 15.4 with a thread per row and nothing padded); 256 preferential attachment grids of 500 to 2000 / 2100
+// to 5000 vertices: 1.96 / 4.3 ms, 0.98 / 1.7 (2.5 / 4.9).  A wide first slice also left no room in
+// LDS for those after it.
+constexpr int kLongRow = 32;        // no shorter row is one
+int64_t long_row_count(const std::vector<int32_t>& len) {
+    constexpr int64_t kColumn = 100, kRow = 300, kEntry = 25;
+    const int64_t n = static_cast<int64_t>(len.size());
+    int64_t best = 0, cost = INT64_MAX, rows = 0;
+    for (int64_t m = 0; m <= n; ++m) {
+        int64_t c = rows / (kThreads / kWave);
+        for (int64_t i = m; i < n; i += kThreads) c += kColumn * len[static_cast<size_t>(i)];
+        if (c < cost) {
+            cost = c;
+            best = m;
+        }
+        if (m == n || len[static_cast<size_t>(m)] <= kLongRow) break;
+        rows += kRow + kEntry * len[static_cast<size_t>(m)];
+    }
+    return best;
+}
+
 int herr(hipError_t e, const char* w) {
     return e == hipSuccess ? ND_OK : nd::set_error(ND_ERR_DEVICE, "%s: %s", w, hipGetErrorString(e));
 }
@@ -382,6 +477,7 @@ struct nd_fixpoint {
     double* d_w = nullptr;
     int lds_max = 0;
     int32_t lds[2] = {0, 0};                // dynamic LDS of the two classes' launches
+    bool has_long[2] = {false, false};      // whether a grid of the class has long rows
     int64_t total_vertices = 0, total_edges = 0;
     // the two size classes run on their own streams, forked from and joined back to the
     // caller's stream with events, so the large grids start while small ones still run
@@ -461,25 +557,38 @@ int nd_fixpoint_create(int32_t ngrid, const int64_t* nv, const int64_t* ne, cons
             pos[v] = first[longest - (deg[v + 1] - deg[v])]++;
             perm[p0 + pos[v]] = static_cast<uint16_t>(v);
         }
+        // the longest rows that are better off apart go behind the others
+        std::vector<int32_t> len(static_cast<size_t>(n));
+        for (size_t i = 0; i < len.size(); ++i) len[i] = deg[perm[p0 + i] + 1] - deg[perm[p0 + i]];
+        const int32_t nlong = static_cast<int32_t>(long_row_count(len)), nr = static_cast<int32_t>(n) - nlong;
+        std::rotate(perm.begin() + p0, perm.begin() + p0 + nlong, perm.end());
+        for (int32_t i = 0; i < static_cast<int32_t>(n); ++i) pos[perm[p0 + i]] = i;
         int32_t col = 0;
         const size_t s0 = slices.size(), e0 = nb.size();
-        for (int32_t i = 0; i < static_cast<int32_t>(n); i += kWave) {
+        for (int32_t i = 0; i < nr; i += kWave) {
             const int32_t v = perm[p0 + i], width = deg[v + 1] - deg[v];
             slices.push_back(make_int2(col, width));
             col += width;
         }
+        const size_t l0 = slices.size();
+        for (int32_t i = nr; i < static_cast<int32_t>(n); ++i) {
+            const int32_t v = perm[p0 + i], entries = deg[v + 1] - deg[v];
+            slices.push_back(make_int2(col, entries));
+            col += (entries + kWave - 1) / kWave;
+        }
         nb.resize(e0 + static_cast<size_t>(col) * kWave);
         sedge.resize(nb.size(), -1);
-        for (size_t s = s0; s < slices.size(); ++s)
+        for (size_t s = s0; s < l0; ++s)
             for (int32_t l = 0; l < kWave; ++l) {
                 const size_t i = (s - s0) * kWave + l;
-                const uint16_t own = static_cast<uint16_t>(8 * (i < static_cast<size_t>(n) ? perm[p0 + i] : 0));
+                const uint16_t own = static_cast<uint16_t>(8 * (i < static_cast<size_t>(nr) ? perm[p0 + i] : 0));
                 for (int32_t j = 0; j < slices[s].y; ++j) nb[e0 + static_cast<size_t>(slices[s].x + j) * kWave + l] = own;
             }
         std::vector<int32_t> fill(static_cast<size_t>(n), 0);
         auto entry = [&](int64_t v, int64_t other, int64_t e) {
-            const int32_t i = pos[v], c = slices[s0 + i / kWave].x + fill[v]++;
-            const size_t k = e0 + static_cast<size_t>(c) * kWave + i % kWave;
+            const int32_t i = pos[v], f = fill[v]++;
+            const size_t k = i < nr ? e0 + static_cast<size_t>(slices[s0 + i / kWave].x + f) * kWave + i % kWave
+                                    : e0 + static_cast<size_t>(slices[l0 + i - nr].x) * kWave + f;
             nb[k] = static_cast<uint16_t>(8 * other);
             sedge[k] = static_cast<int32_t>(eoff + e);
         };
@@ -489,8 +598,10 @@ int nd_fixpoint_create(int32_t ngrid, const int64_t* nv, const int64_t* ne, cons
             entry(d, s, e);
         }
         G.ncol = col;
+        G.nlong = nlong;
         // the vectors, the reduction buffers and as many columns of weights as there is room for
         const int cls = n <= 4 * kThreads ? 0 : 1;
+        f->has_long[cls] = f->has_long[cls] || nlong > 0;
         f->lds[cls] = std::max(f->lds[cls], static_cast<int32_t>(std::min<int64_t>(lds_max, 8 * (2 * n + 64) + static_cast<int64_t>(kColBytes) * col)));
         f->grids.push_back(G);
         (n <= 4 * kThreads ? f->small : f->large).push_back(gi);
@@ -565,15 +676,17 @@ int nd_fixpoint_solve(nd_fixpoint* f, double* theta, const double* P, const doub
         if (!rc && !f->ev_join[c]) rc = herr(hipEventCreateWithFlags(&f->ev_join[c], hipEventDisableTiming), "hipEventCreate");
     }
     if (rc) return rc;
+    const auto small_kernel = f->has_long[0] ? k_newton<4, true> : k_newton<4, false>;
+    const auto large_kernel = f->has_long[1] ? k_newton<10, true> : k_newton<10, false>;
     size_t lds_s = 0, lds_l = 0;
     if (ns) {
         lds_s = static_cast<size_t>(f->lds[0]);
-        rc = herr(hipFuncSetAttribute(reinterpret_cast<const void*>(k_newton<4>), hipFuncAttributeMaxDynamicSharedMemorySize,
+        rc = herr(hipFuncSetAttribute(reinterpret_cast<const void*>(small_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                       static_cast<int>(lds_s)), "hipFuncSetAttribute");
     }
     if (!rc && nl) {
         lds_l = static_cast<size_t>(f->lds[1]);
-        rc = herr(hipFuncSetAttribute(reinterpret_cast<const void*>(k_newton<10>), hipFuncAttributeMaxDynamicSharedMemorySize,
+        rc = herr(hipFuncSetAttribute(reinterpret_cast<const void*>(large_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                       static_cast<int>(lds_l)), "hipFuncSetAttribute");
     }
     rc = rc ? rc : herr(hipEventRecord(f->ev_fork, s), "hipEventRecord");
@@ -585,7 +698,7 @@ int nd_fixpoint_solve(nd_fixpoint* f, double* theta, const double* P, const doub
         if (rc) return rc;
         a.first = static_cast<int32_t>(ns);
         a.lds = f->lds[1];
-        hipLaunchKernelGGL(k_newton<10>, dim3(static_cast<unsigned>(nl)), dim3(kThreads), lds_l, cs, a);
+        hipLaunchKernelGGL(large_kernel, dim3(static_cast<unsigned>(nl)), dim3(kThreads), lds_l, cs, a);
         rc = herr(hipGetLastError(), "newton launch");
         rc = rc ? rc : herr(hipEventRecord(f->ev_join[1], cs), "hipEventRecord");
         rc = rc ? rc : herr(hipStreamWaitEvent(s, f->ev_join[1], 0), "hipStreamWaitEvent");
@@ -597,7 +710,7 @@ int nd_fixpoint_solve(nd_fixpoint* f, double* theta, const double* P, const doub
         if (rc) return rc;
         a.first = 0;
         a.lds = f->lds[0];
-        hipLaunchKernelGGL(k_newton<4>, dim3(static_cast<unsigned>(ns)), dim3(kThreads), lds_s, cs, a);
+        hipLaunchKernelGGL(small_kernel, dim3(static_cast<unsigned>(ns)), dim3(kThreads), lds_s, cs, a);
         rc = herr(hipGetLastError(), "newton launch");
         rc = rc ? rc : herr(hipEventRecord(f->ev_join[0], cs), "hipEventRecord");
         rc = rc ? rc : herr(hipStreamWaitEvent(s, f->ev_join[0], 0), "hipStreamWaitEvent");
