@@ -91,17 +91,10 @@ __device__ __forceinline__ double quotient(double a, double b, double y) {
     return __builtin_fma(__builtin_fma(-q, b, a), y, q);
 }
 
-// z = r / dg, returns the thread's part of r . z.  A z that is not finite makes that sum not
-// finite, so one test finds every quotient to be divided out.
+// A quotient that is not finite makes the sum rz = r . z not finite, so one test finds every z to be
+// divided out
 template <int V>
-__device__ __forceinline__ double precondition(const double (&r)[V], const double (&dg)[V], const double (&dgi)[V],
-                                               double (&z)[V]) {
-    double rz = 0.0;
-#pragma unroll
-    for (int k = 0; k < V; ++k) {
-        z[k] = quotient(r[k], dg[k], dgi[k]);
-        rz += r[k] * z[k];
-    }
+__device__ __forceinline__ double divide_out(double rz, const double (&r)[V], const double (&dg)[V], double (&z)[V]) {
     if (__builtin_expect(!(fabs(rz) <= 0x1.fffffffffffffp+1023), 0)) {
         rz = 0.0;
 #pragma unroll
@@ -313,9 +306,11 @@ __global__ void __launch_bounds__(kThreads) k_newton(NewtonArgs a) {
             r[k] = v < n ? r[k] - fmean : 0.0;
             dg[k] = v < n ? rowv[v] : 1.0;
             dgi[k] = 1.0 / dg[k];
+            z[k] = quotient(r[k], dg[k], dgi[k]);
+            rz += r[k] * z[k];
             rr0 += r[k] * r[k];
         }
-        rz = precondition(r, dg, dgi, z);
+        rz = divide_out(rz, r, dg, z);
 #pragma unroll
         for (int k = 0; k < V; ++k)
             if (t + k * T < n) buf[t + k * T] = z[k];
@@ -385,9 +380,11 @@ __global__ void __launch_bounds__(kThreads) k_newton(NewtonArgs a) {
             for (int k = 0; k < V; ++k) {
                 d[k] += alpha * pi[k];
                 r[k] -= alpha * q[k];
+                q[k] = quotient(r[k], dg[k], dgi[k]);
+                rzn += r[k] * q[k];
                 rrn += r[k] * r[k];
             }
-            rzn = precondition(r, dg, dgi, q);
+            rzn = divide_out(rzn, r, dg, q);
             red.sum2(rzn, rrn);
             rr = rrn;
             const double beta = rzn / rz;
