@@ -278,6 +278,12 @@ __device__ __forceinline__ TileRange wave_tiles(int64_t ntiles, int waves, int w
 constexpr int kWS = 68;             // LDS stride of a weight or node row: 16-byte columns free of bank conflicts
 constexpr int kTile = 16;           // nodes per wave and step
 constexpr int kAhead = 2;           // entries of each of four nodes whose rows are in flight at once
+// Entries of a row that are summed beside those of the tile's other nodes; the others of a longer row
+// the wave takes 32 at a time (gather_long).  Forward passes with every row beside its tile's others /
+// so: a star of 20 000 lines 14.8 / 1.46 ms, one preferential attachment graph of 1e5 nodes 666 / 508
+// us, 100 of 2000 nodes 329 / 290 (cap 64: 274), 20 dense graphs of 30 to 90 lines a node 283 / 284
+// (cap 64: 293).  The check costs a small batch (5 grids of 1000 nodes, 74 us) 2 %.
+constexpr int kRowCap = 96;
 
 // lane J of each 16 lanes to all of them; the 16 lanes moved down by kAhead
 template <int J>
@@ -337,7 +343,52 @@ __device__ __forceinline__ void tile_entries(const int32_t* __restrict__ nbr, co
     t.nbr = nbr[s];
     t.a = a[s];
 }
-// z[p] = sum_s a[s] X[nbr[s], 4 li ..] over the entries of node 4 p + lk, in order
+// The entries of one row from position first on, added to the row's z: the wave takes 32 at a time,
+// eight on each of its four node lanes, and adds the four sums at the end.
+template <bool WIDE>
+__device__ __forceinline__ float4 gather_long(const int32_t* __restrict__ nbr, const float* __restrict__ a,
+                                              const Rows<WIDE>& X, int32_t first, int32_t end, int lane, int li, int lk) {
+    float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    auto entries = [&](int64_t base, uint32_t& at, float& w) {
+        const int64_t s = base + lane;
+        at = s < end ? X.at(nbr[s]) : X.kNone;
+        w = s < end ? a[s] : 0.0f;
+    };
+    uint32_t at;
+    float w;
+    entries(first, at, w);
+    for (int64_t base = first; base < end; base += kWave) {
+        const uint32_t at0 = at;
+        const float w0 = w;
+        entries(base + kWave, at, w);                     // the next 64 are on their way meanwhile
+#pragma unroll 1
+        for (int h = 0; h < kWave && base + h < end; h += 32) {
+            float4 x[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                x[i] = X.part(static_cast<uint32_t>(__shfl(static_cast<int>(at0), h + 4 * i + lk, kWave)), li);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float c = __shfl(w0, h + 4 * i + lk, kWave);
+                z.x = __builtin_fmaf(c, x[i].x, z.x);
+                z.y = __builtin_fmaf(c, x[i].y, z.y);
+                z.z = __builtin_fmaf(c, x[i].z, z.z);
+                z.w = __builtin_fmaf(c, x[i].w, z.w);
+            }
+        }
+    }
+#pragma unroll
+    for (int off = 16; off < kWave; off *= 2) {
+        z.x += __shfl_xor(z.x, off, kWave);
+        z.y += __shfl_xor(z.y, off, kWave);
+        z.z += __shfl_xor(z.z, off, kWave);
+        z.w += __shfl_xor(z.w, off, kWave);
+    }
+    return z;
+}
+// z[p] = sum_s a[s] X[nbr[s], 4 li ..] over the entries of node 4 p + lk: the first kRowCap in order
+// and side by side for all nodes, the others of a longer row by gather_long.  (The order depends on
+// the row alone, so a node's sum does not depend on its place in the batch.)
 template <bool WIDE>
 __device__ __forceinline__ void gather_tile(const int32_t* __restrict__ nbr, const float* __restrict__ a, const Rows<WIDE>& X,
                                             const TileEntries& t, int li, int lk, float4 (&z)[4]) {
@@ -349,10 +400,11 @@ __device__ __forceinline__ void gather_tile(const int32_t* __restrict__ nbr, con
     most = max(most, __builtin_amdgcn_update_dpp(0, most, 0x122, 0xf, 0xf, true));
     most = max(most, __builtin_amdgcn_update_dpp(0, most, 0x121, 0xf, 0xf, true));
     most = __builtin_amdgcn_readfirstlane(most);
+    const int32_t side = most < kRowCap ? most : kRowCap;
 #pragma unroll
     for (int p = 0; p < 4; ++p) z[p] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     uint32_t nb[4], av[4];                                // the next 16 entries of each node, one per lane
-    for (int32_t k = 0; k < most; k += kAhead) {
+    for (int32_t k = 0; k < side; k += kAhead) {
         if (k % 16 == 0) {
 #pragma unroll
             for (int p = 0; p < 4; ++p) {
@@ -395,6 +447,18 @@ __device__ __forceinline__ void gather_tile(const int32_t* __restrict__ nbr, con
                 z[p].z = __builtin_fmaf(c[i], x[p][i].z, z[p].z);
                 z[p].w = __builtin_fmaf(c[i], x[p][i].w, z[p].w);
             }
+        }
+    }
+    if (most > kRowCap) {
+        const int lane = 16 * lk + li;
+#pragma unroll 1
+        for (int j = 0; j < kTile; ++j) {
+            const int32_t start = __builtin_amdgcn_readlane(t.rows, j), end = __builtin_amdgcn_readlane(t.rows, j + 1);
+            if (end - start <= kRowCap) continue;
+            const float4 y = gather_long<WIDE>(nbr, a, X, start + kRowCap, end, lane, li, lk);
+#pragma unroll
+            for (int p = 0; p < 4; ++p)
+                if (j == 4 * p + lk) z[p] = make_float4(z[p].x + y.x, z[p].y + y.y, z[p].z + y.z, z[p].w + y.w);
         }
     }
 }
