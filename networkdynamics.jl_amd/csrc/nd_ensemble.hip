@@ -422,10 +422,10 @@ __device__ __forceinline__ double line_cond(const Lds& L, const double* th, cons
 }
 
 // sg[e] = sign8 of every edge's condition at the state y (two block barriers)
-template <int VM, int EM, int V>
+template <int VM, int EM, int V, bool FRESH>
 __device__ __forceinline__ void line_signs(const InstDesc& I, const Lds& L, const double* lim,
                                            const double (&y)[V][VModel<VM>::dim], int8_t* sg) {
-    const int T = static_cast<int>(blockDim.x), t = static_cast<int>(threadIdx.x);
+    const int T = static_cast<int>(blockDim.x), t = fresh<FRESH>(static_cast<int>(threadIdx.x));
 #pragma unroll
     for (int k = 0; k < V; ++k) {
         const int v = t + k * T;
@@ -605,8 +605,8 @@ __device__ __forceinline__ void ensemble_body(const SolveArgs& a, int inst, cons
         }
         tcur = a.t0 + static_cast<double>(done) * dt;
     } else {
-        // k3..k5 hold the dense-output coefficients d2..d4 once the last evaluation has begun
-        // (crossing location), k2 the error estimate's sum over the first six stages
+        // k3..k5 hold the dense-output coefficients d2..d4 over the first six stages once the last
+        // evaluation has begun (crossing location), k2 the error estimate's sum over the first six stages
         double k1[V][D], k2[V][D], k3[V][D], k4[V][D], k5[V][D], k6[V][D];
         auto &d2 = k3, &d3 = k4, &d4 = k5;
         ND_EACH { ys[q][j] = y[q][j]; k1[q][j] = k2[q][j] = k3[q][j] = k4[q][j] = k5[q][j] = k6[q][j] = 0.0; }
@@ -692,13 +692,6 @@ __device__ __forceinline__ void ensemble_body(const SolveArgs& a, int inst, cons
                 continue;
             }
             if (phase == 6) {
-                if constexpr (kLocate) {
-                    ND_EACH {
-                        d2[q][j] = d2[q][j] + ND_R(7, 2) * k[q][j];
-                        d3[q][j] = d3[q][j] + ND_R(7, 3) * k[q][j];
-                        d4[q][j] = d4[q][j] + ND_R(7, 4) * k[q][j];
-                    }
-                }
                 double s = 0.0;
 #pragma unroll
                 for (int q = 0; q < V; ++q)
@@ -726,6 +719,18 @@ __device__ __forceinline__ void ensemble_body(const SolveArgs& a, int inst, cons
                     bool located = false;
                     if constexpr (kLocate) {
                         if (lim) {
+                            const int t = fresh<kFresh<V, LB>>(static_cast<int>(threadIdx.x));
+                            // the dense output's coefficients with the last derivative, in arrays of their
+                            // own: updated in place, both values would be live around the loop over the
+                            // phases (210 spilled registers at four vertices per thread instead of 63, 67
+                            // instead of 6 at three; 512 networks of 1700 / 1900 vertices 32 / 39 ms instead
+                            // of 22 / 25)
+                            double e2[V][D], e3[V][D], e4[V][D];
+                            ND_EACH {
+                                e2[q][j] = d2[q][j] + ND_R(7, 2) * k[q][j];
+                                e3[q][j] = d3[q][j] + ND_R(7, 3) * k[q][j];
+                                e4[q][j] = d4[q][j] + ND_R(7, 4) * k[q][j];
+                            }
                             // the condition at the points s = m/9 of the step (m = 9: the accepted
                             // state), against its sign at the step start
                             double first = 10.0;
@@ -738,7 +743,7 @@ __device__ __forceinline__ void ensemble_body(const SolveArgs& a, int inst, cons
                                     const int v = t + q * T;
                                     if (v < I.n)
                                         th[v] = m == 9 ? ys[q][0]
-                                                       : dense_at(y[q][0], k1[q][0], d2[q][0], d3[q][0], d4[q][0], h, s);
+                                                       : dense_at(y[q][0], k1[q][0], e2[q][0], e3[q][0], e4[q][0], h, s);
                                 }
                                 __syncthreads();
                                 for (int e = t; e < I.ne; e += T) {
@@ -766,7 +771,7 @@ __device__ __forceinline__ void ensemble_body(const SolveArgs& a, int inst, cons
 #pragma unroll
                                     for (int q = 0; q < V; ++q) {
                                         const int v = t + q * T;
-                                        if (v < I.n) L.theta[v] = dense_at(y[q][0], k1[q][0], d2[q][0], d3[q][0], d4[q][0], h, s);
+                                        if (v < I.n) L.theta[v] = dense_at(y[q][0], k1[q][0], e2[q][0], e3[q][0], e4[q][0], h, s);
                                     }
                                     __syncthreads();
                                     double hit = 0.0;
@@ -787,7 +792,7 @@ __device__ __forceinline__ void ensemble_body(const SolveArgs& a, int inst, cons
                                     const int v = t + q * T;
                                     if (v < I.n)
                                         L.theta[v] = hi_end ? ys[q][0]
-                                                            : dense_at(y[q][0], k1[q][0], d2[q][0], d3[q][0], d4[q][0], h, shi);
+                                                            : dense_at(y[q][0], k1[q][0], e2[q][0], e3[q][0], e4[q][0], h, shi);
                                 }
                                 __syncthreads();
                                 constexpr int NPE1 = NPE > 0 ? NPE : 1;
@@ -805,7 +810,7 @@ __device__ __forceinline__ void ensemble_body(const SolveArgs& a, int inst, cons
                                 for (int q = 0; q < V; ++q)
 #pragma unroll
                                     for (int j = 0; j < D; ++j)
-                                        y[q][j] = dense_at(y[q][j], k1[q][j], d2[q][j], d3[q][j], d4[q][j], h, slo);
+                                        y[q][j] = dense_at(y[q][j], k1[q][j], e2[q][j], e3[q][j], e4[q][j], h, slo);
                                 tcur = lo;
                                 located = true;
                                 changed = 1;                            // the state moved: new derivative
@@ -851,7 +856,7 @@ __device__ __forceinline__ void ensemble_body(const SolveArgs& a, int inst, cons
             } else if (phase == 8) {
                 ND_EACH k1[q][j] = k[q][j];
                 if constexpr (kLocate)
-                    if (lim) line_signs<VM, EM, V>(I, L, lim, y, gsign);
+                    if (lim) line_signs<VM, EM, V, kFresh<V, LB>>(I, L, lim, y, gsign);
                 accepted = true;
             } else {
                 // the start: k1, then for an automatic initial step its probe (Hairer, Norsett &
@@ -877,7 +882,7 @@ __device__ __forceinline__ void ensemble_body(const SolveArgs& a, int inst, cons
                 dt = fmin(dt, a.dtmax);
                 begun = false;
                 if constexpr (kLocate)
-                    if (lim) line_signs<VM, EM, V>(I, L, lim, y, gsign);
+                    if (lim) line_signs<VM, EM, V, kFresh<V, LB>>(I, L, lim, y, gsign);
             }
             if (accepted && a.ss && at_steady_state<V, D>(a, I, L, y, k1)) {
                 retcode = 4;
