@@ -183,12 +183,12 @@ template <int V>
 constexpr bool kParamsInMemory = V >= 4;
 
 // fslot = the outputs of every edge at the state ys in row order, the src side negated
-// (AntiSymmetric).  Two block barriers: after the vertex outputs and after the edges.  The
-// first batch's table records and parameters do not depend on the state and are read before
-// the first barrier.
-template <int VM, int EM, int V, bool FRESH>
-__device__ __forceinline__ void edge_flows(const InstDesc& I, const Lds& L, const double (&ys)[V][VModel<VM>::dim]) {
-    constexpr int N = kEdgeBatch, NP = EModel<EM>::np;
+// (AntiSymmetric), N consecutive edges per thread at a time.  Two block barriers: after the vertex
+// outputs and after the edges.  The first batch's table records and parameters do not depend on
+// the state and are read before the first barrier.
+template <int VM, int EM, int V, bool FRESH, int N>
+__device__ __forceinline__ void edge_flows_n(const InstDesc& I, const Lds& L, const double (&ys)[V][VModel<VM>::dim]) {
+    constexpr int NP = EModel<EM>::np;
     const int T = static_cast<int>(blockDim.x);
     const int t = fresh<FRESH>(static_cast<int>(threadIdx.x));
     uint2 rec[N];
@@ -231,6 +231,17 @@ __device__ __forceinline__ void edge_flows(const InstDesc& I, const Lds& L, cons
     __syncthreads();
 }
 
+// SMALL: two at a time where there are no more than two per thread, so that fewer threads idle while
+// others have four.  1024 networks of 64 / 100 vertices, Tsit5 (128 threads): 673 / 731 us with four,
+// 605 / 687 with two.  In kernels of their own, for launches a quarter of whose instances are so small: the
+// second path costs the others up to 5 %.
+template <int VM, int EM, int V, bool FRESH, bool SMALL>
+__device__ __forceinline__ void edge_flows(const InstDesc& I, const Lds& L, const double (&ys)[V][VModel<VM>::dim]) {
+    const int T = static_cast<int>(blockDim.x);
+    if (SMALL && I.ne <= 2 * T) edge_flows_n<VM, EM, V, FRESH, 2>(I, L, ys);
+    else edge_flows_n<VM, EM, V, FRESH, kEdgeBatch>(I, L, ys);
+}
+
 // the entries of pairs first .. first + N - 1 of a row; pairs past its end are the zeros (an
 // address select in place of a bound on every entry)
 template <int N>
@@ -256,13 +267,13 @@ __device__ __forceinline__ void row_add(const double2 (&f)[N], double& part) {
 // summed by chunks spread over the block first, which takes a third barrier.  row: the
 // thread's row words; pv: the vertex parameters in registers, or pg: the instance's vertex
 // parameters in memory (kParamsInMemory)
-template <int VM, int EM, int V, bool FRESH>
+template <int VM, int EM, int V, bool FRESH, bool SMALL>
 __device__ __forceinline__ void rhs(const InstDesc& I, const Lds& L, const double (&ys)[V][VModel<VM>::dim],
                                     const double (&pv)[V][VPar<VM>::np > 0 ? VPar<VM>::np : 1],
                                     const double* __restrict__ pg, const uint32_t (&row_)[V],
                                     double (&out)[V][VModel<VM>::dim]) {
     const int T = static_cast<int>(blockDim.x);
-    edge_flows<VM, EM, V, FRESH>(I, L, ys);
+    edge_flows<VM, EM, V, FRESH, SMALL>(I, L, ys);
     const int t = fresh<FRESH>(static_cast<int>(threadIdx.x));
     uint32_t row[V];
 #pragma unroll
@@ -490,11 +501,12 @@ __device__ __forceinline__ double dense_at(double y0, double k1, double d2, doub
     return y0 + h * (s * (k1 + s * (d2 + s * (d3 + s * d4))));
 }
 
-template <int VM, int EM, int METHOD, int V, int LB>
+template <int VM, int EM, int METHOD, int V, int LB, bool FRESH>
 __device__ __forceinline__ void ensemble_body(const SolveArgs& a, int inst, const InstDesc& I, double2* smem) {
     constexpr int D = VModel<VM>::dim;
     constexpr int NPV = VPar<VM>::np > 0 ? VPar<VM>::np : 1;
     constexpr int NPE = EModel<EM>::np;
+    constexpr bool kSmall = LB <= 256 && V <= 2;
     const int T = static_cast<int>(blockDim.x), t = static_cast<int>(threadIdx.x);
     const int ne4 = pad_edges(I.ne);
     Lds L;
@@ -573,7 +585,7 @@ __device__ __forceinline__ void ensemble_body(const SolveArgs& a, int inst, cons
         ND_EACH { ys[q][j] = y[q][j]; acc[q][j] = 0.0; }
         int stage = 0;                              // 0..3, 4: the steady-state check's evaluation
         for (int64_t step = 0; step < nsteps;) {
-            rhs<VM, EM, V, kFresh<V, LB>>(I, L, ys, pv, pg, row, k);
+            rhs<VM, EM, V, FRESH, kSmall>(I, L, ys, pv, pg, row, k);
             ++nf;
             if (stage < 3) {
                 const double hs = stage == 2 ? dt : half;
@@ -587,7 +599,7 @@ __device__ __forceinline__ void ensemble_body(const SolveArgs& a, int inst, cons
                 ND_EACH { y[q][j] = y[q][j] + sixth * (acc[q][j] + k[q][j]); ys[q][j] = y[q][j]; }
                 ++naccept;
                 if (a.limit) {
-                    edge_flows<VM, EM, V, kFresh<V, LB>>(I, L, y);
+                    edge_flows<VM, EM, V, FRESH, kSmall>(I, L, y);
                     ntrip += trip_lines<VM, EM>(a, I, L);
                 }
                 if (ee >= 0 && step + 1 == static_cast<int64_t>(llround((te - a.t0) / dt))) ntrip += trip_edge<VM, EM>(a, I, L, ee);
@@ -643,7 +655,7 @@ __device__ __forceinline__ void ensemble_body(const SolveArgs& a, int inst, cons
         // 7 the initial step's probe, 8 the first derivative again after a trip
         int phase = 0;
         for (;;) {
-            rhs<VM, EM, V, kFresh<V, LB>>(I, L, ys, pv, pg, row, k);
+            rhs<VM, EM, V, FRESH, kSmall>(I, L, ys, pv, pg, row, k);
             ++nf;
             bool accepted = false, begun = true;
             if (phase >= 1 && phase <= 5) {
@@ -719,7 +731,7 @@ __device__ __forceinline__ void ensemble_body(const SolveArgs& a, int inst, cons
                     bool located = false;
                     if constexpr (kLocate) {
                         if (lim) {
-                            const int t = fresh<kFresh<V, LB>>(static_cast<int>(threadIdx.x));
+                            const int t = fresh<FRESH>(static_cast<int>(threadIdx.x));
                             // the dense output's coefficients with the last derivative, in arrays of their
                             // own: updated in place, both values would be live around the loop over the
                             // phases (210 spilled registers at four vertices per thread instead of 63, 67
@@ -856,7 +868,7 @@ __device__ __forceinline__ void ensemble_body(const SolveArgs& a, int inst, cons
             } else if (phase == 8) {
                 ND_EACH k1[q][j] = k[q][j];
                 if constexpr (kLocate)
-                    if (lim) line_signs<VM, EM, V, kFresh<V, LB>>(I, L, lim, y, gsign);
+                    if (lim) line_signs<VM, EM, V, FRESH>(I, L, lim, y, gsign);
                 accepted = true;
             } else {
                 // the start: k1, then for an automatic initial step its probe (Hairer, Norsett &
@@ -882,7 +894,7 @@ __device__ __forceinline__ void ensemble_body(const SolveArgs& a, int inst, cons
                 dt = fmin(dt, a.dtmax);
                 begun = false;
                 if constexpr (kLocate)
-                    if (lim) line_signs<VM, EM, V, kFresh<V, LB>>(I, L, lim, y, gsign);
+                    if (lim) line_signs<VM, EM, V, FRESH>(I, L, lim, y, gsign);
             }
             if (accepted && a.ss && at_steady_state<V, D>(a, I, L, y, k1)) {
                 retcode = 4;
@@ -919,61 +931,72 @@ __device__ __forceinline__ void ensemble_body(const SolveArgs& a, int inst, cons
     }
 }
 
+// Waves per SIMD that a kernel leaves registers for.  Three where a small workgroup's kernel comes
+// close to their 168 registers by itself (RK4, one state per vertex).
+template <int VM, int METHOD, int V, int LB>
+constexpr int kMinWaves = LB > 512 ? 4 : LB <= 256 && V <= 2 && (METHOD == 1 || (METHOD == 0 && VModel<VM>::dim == 1)) ? 3 : 2;
+
 template <int VM, int EM, int METHOD, int V, int LB>
-__global__ void __launch_bounds__(LB) k_ensemble(SolveArgs a) {
+__global__ void __launch_bounds__(LB, (kMinWaves<VM, METHOD, V, LB>)) k_ensemble(SolveArgs a) {
     extern __shared__ double2 smem[];
     const int inst = a.order[a.first + static_cast<int>(blockIdx.x)];
     const InstDesc I = a.inst[inst];
-    ensemble_body<VM, EM, METHOD, V, LB>(a, inst, I, smem);
+    ensemble_body<VM, EM, METHOD, V, LB, kFresh<V, LB>>(a, inst, I, smem);
 }
 
 // Several size classes of one thread count in one launch: each instance runs with its
 // class's vertices per thread.
-template <int VM, int EM, int METHOD>
-__global__ void __launch_bounds__(512) k_ensemble_mixed(SolveArgs a) {
+template <int VM, int EM, int METHOD, int LB>
+__global__ void __launch_bounds__(LB, 2) k_ensemble_mixed(SolveArgs a) {
     extern __shared__ double2 smem[];
     const int inst = a.order[a.first + static_cast<int>(blockIdx.x)];
     const InstDesc I = a.inst[inst];
     switch (__builtin_amdgcn_readfirstlane(I.vper)) {
-    case 1: ensemble_body<VM, EM, METHOD, 1, 512>(a, inst, I, smem); break;
-    case 2: ensemble_body<VM, EM, METHOD, 2, 512>(a, inst, I, smem); break;
-    case 3: ensemble_body<VM, EM, METHOD, 3, 512>(a, inst, I, smem); break;
-    default: ensemble_body<VM, EM, METHOD, 4, 512>(a, inst, I, smem); break;
+    case 1: ensemble_body<VM, EM, METHOD, 1, LB, kFresh<1, LB>>(a, inst, I, smem); break;
+    case 2: ensemble_body<VM, EM, METHOD, 2, LB, kFresh<2, LB>>(a, inst, I, smem); break;
+    case 3: ensemble_body<VM, EM, METHOD, 3, LB, kFresh<3, LB>>(a, inst, I, smem); break;
+    default: ensemble_body<VM, EM, METHOD, 4, LB, kFresh<4, LB>>(a, inst, I, smem); break;
     }
 }
 
 using EnsKernel = void (*)(SolveArgs);
 
-// Workgroups of up to 512 threads take any vper (0: by instance); 1024-thread workgroups
-// (16 waves, at most 128 VGPRs each) take one or two vertices per thread.
-template <int VM, int EM, int METHOD>
-EnsKernel pick_v(int vper, int threads) {
-    if (vper == 0) return k_ensemble_mixed<VM, EM, METHOD>;
-    if (threads > 512) return vper == 1 ? k_ensemble<VM, EM, METHOD, 1, 1024> : k_ensemble<VM, EM, METHOD, 2, 1024>;
+// vper 0: by instance
+template <int VM, int EM, int METHOD, int LB>
+EnsKernel pick_vper(int vper) {
     switch (vper) {
-    case 1: return k_ensemble<VM, EM, METHOD, 1, 512>;
-    case 3: return k_ensemble<VM, EM, METHOD, 3, 512>;
-    case 4: return k_ensemble<VM, EM, METHOD, 4, 512>;
-    default: return k_ensemble<VM, EM, METHOD, 2, 512>;
+    case 0: return k_ensemble_mixed<VM, EM, METHOD, LB>;
+    case 1: return k_ensemble<VM, EM, METHOD, 1, LB>;
+    case 3: return k_ensemble<VM, EM, METHOD, 3, LB>;
+    case 4: return k_ensemble<VM, EM, METHOD, 4, LB>;
+    default: return k_ensemble<VM, EM, METHOD, 2, LB>;
     }
+}
+// Workgroups of up to 512 threads take any vper; 1024-thread workgroups (16 waves, at most 128
+// VGPRs each) take one or two vertices per thread.  small: at most 256 threads, and few edges per
+// thread in a quarter of the instances or more
+template <int VM, int EM, int METHOD>
+EnsKernel pick_v(int vper, int threads, bool small) {
+    if (threads > 512) return vper == 1 ? k_ensemble<VM, EM, METHOD, 1, 1024> : k_ensemble<VM, EM, METHOD, 2, 1024>;
+    return small ? pick_vper<VM, EM, METHOD, 256>(vper) : pick_vper<VM, EM, METHOD, 512>(vper);
 }
 
 // kernel method: 0 Tsit5, 1 RK4, 2 Tsit5 with line crossings located on the dense output
 template <int VM, int EM>
-EnsKernel pick_m(int kmethod, int vper, int threads) {
+EnsKernel pick_m(int kmethod, int vper, int threads, bool small) {
     switch (kmethod) {
-    case 1: return pick_v<VM, EM, 1>(vper, threads);
-    case 2: return pick_v<VM, EM, 2>(vper, threads);
-    default: return pick_v<VM, EM, 0>(vper, threads);
+    case 1: return pick_v<VM, EM, 1>(vper, threads, small);
+    case 2: return pick_v<VM, EM, 2>(vper, threads, small);
+    default: return pick_v<VM, EM, 0>(vper, threads, small);
     }
 }
 
-EnsKernel pick_ensemble(int vm, int em, int kmethod, int vper, int threads) {
-    if (vm == ND_VM_SWING && em == ND_EM_KURAMOTO) return pick_m<ND_VM_SWING, ND_EM_KURAMOTO>(kmethod, vper, threads);
-    if (vm == ND_VM_SWING && em == ND_EM_STATIC_LINE) return pick_m<ND_VM_SWING, ND_EM_STATIC_LINE>(kmethod, vper, threads);
-    if (vm == ND_VM_KURAMOTO && em == ND_EM_KURAMOTO) return pick_m<ND_VM_KURAMOTO, ND_EM_KURAMOTO>(kmethod, vper, threads);
+EnsKernel pick_ensemble(int vm, int em, int kmethod, int vper, int threads, bool small) {
+    if (vm == ND_VM_SWING && em == ND_EM_KURAMOTO) return pick_m<ND_VM_SWING, ND_EM_KURAMOTO>(kmethod, vper, threads, small);
+    if (vm == ND_VM_SWING && em == ND_EM_STATIC_LINE) return pick_m<ND_VM_SWING, ND_EM_STATIC_LINE>(kmethod, vper, threads, small);
+    if (vm == ND_VM_KURAMOTO && em == ND_EM_KURAMOTO) return pick_m<ND_VM_KURAMOTO, ND_EM_KURAMOTO>(kmethod, vper, threads, small);
     if (vm == ND_VM_KURAMOTO && em == ND_EM_STATIC_LINE)
-        return pick_m<ND_VM_KURAMOTO, ND_EM_STATIC_LINE>(kmethod, vper, threads);
+        return pick_m<ND_VM_KURAMOTO, ND_EM_STATIC_LINE>(kmethod, vper, threads, small);
     return nullptr;
 }
 
@@ -1167,12 +1190,13 @@ int32_t class_limit(const nd_ensemble* en, int c, int kmethod) {
 }
 
 // The launches of a solve, largest instances first.  Neighbouring classes of one thread
-// count share a launch: at 512 threads a CU holds one workgroup whatever its vertices per
-// thread, and one list of instances by decreasing size ends more evenly than several
+// count share a launch: at 512 threads a CU holds one workgroup of most kernels whatever its
+// vertices per thread, and one list of instances by decreasing size ends more evenly than several
 // launches side by side.  (1024 networks of 100 to 2000 vertices, default classes, three
-// ensembles solved in turn: 46.9 ms each with a launch and a stream per class, since streams
-// beyond the four hardware queues of a process share one and their classes run one after the
-// other; 40.2 ms so.)
+// ensembles solved in turn, swing Tsit5: 46.9 ms each with a launch and a stream per class, since
+// streams beyond the four hardware queues of a process share one and their classes run one after
+// the other; 40.2 ms so.  Where the separate kernels would leave room for a second workgroup, RK4,
+// the two are even: 4.56 ms and 4.49 for swing, 4.27 and 4.36 for first-order vertices.)
 struct Launch {
     EnsKernel kernel;
     int32_t first, count, threads, lds;
@@ -1192,7 +1216,10 @@ int launches(const nd_ensemble* en, int kmethod, Launch* out) {
             l.count = en->cls_first[c] - l.first;
         }
         l.lds = lds;
-        l.kernel = pick_ensemble(en->vk.model, en->ek.model, kmethod, vper, threads);
+        int32_t few = 0;
+        for (int32_t q = l.first; q < l.first + l.count; ++q) few += en->inst[en->order[q]].ne <= 2 * threads;
+        const bool small = threads <= 256 && 4 * few > l.count;
+        l.kernel = pick_ensemble(en->vk.model, en->ek.model, kmethod, vper, threads, small);
         out[n++] = l;
     }
     return n;
