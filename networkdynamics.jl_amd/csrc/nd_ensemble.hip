@@ -932,16 +932,16 @@ __device__ __forceinline__ void ensemble_body(const SolveArgs& a, int inst, cons
 }
 
 // Waves per SIMD that a kernel leaves registers for.  Three where a small workgroup's kernel comes
-// close to their 168 registers by itself (RK4, one state per vertex).
-template <int VM, int METHOD, int V, int LB>
-constexpr int kMinWaves = LB > 512 ? 4 : LB <= 256 && V <= 2 && (METHOD == 1 || (METHOD == 0 && VModel<VM>::dim == 1)) ? 3 : 2;
+// close to their 168 registers by itself (RK4, one state per vertex).  DENSE: four
+template <int VM, int METHOD, int V, int LB, bool DENSE>
+constexpr int kMinWaves = DENSE || LB > 512 ? 4 : LB <= 256 && V <= 2 && (METHOD == 1 || (METHOD == 0 && VModel<VM>::dim == 1)) ? 3 : 2;
 
-template <int VM, int EM, int METHOD, int V, int LB>
-__global__ void __launch_bounds__(LB, (kMinWaves<VM, METHOD, V, LB>)) k_ensemble(SolveArgs a) {
+template <int VM, int EM, int METHOD, int V, int LB, bool DENSE = false>
+__global__ void __launch_bounds__(LB, (kMinWaves<VM, METHOD, V, LB, DENSE>)) k_ensemble(SolveArgs a) {
     extern __shared__ double2 smem[];
     const int inst = a.order[a.first + static_cast<int>(blockIdx.x)];
     const InstDesc I = a.inst[inst];
-    ensemble_body<VM, EM, METHOD, V, LB, kFresh<V, LB>>(a, inst, I, smem);
+    ensemble_body<VM, EM, METHOD, V, LB, kFresh<V, LB> || DENSE>(a, inst, I, smem);
 }
 
 // Several size classes of one thread count in one launch: each instance runs with its
@@ -963,7 +963,11 @@ using EnsKernel = void (*)(SolveArgs);
 
 // vper 0: by instance
 template <int VM, int EM, int METHOD, int LB>
-EnsKernel pick_vper(int vper) {
+EnsKernel pick_vper(int vper, bool dense) {
+    if constexpr (METHOD == 1) {
+        if (dense && vper == 1) return k_ensemble<VM, EM, METHOD, 1, LB, true>;
+        if (dense && vper == 2) return k_ensemble<VM, EM, METHOD, 2, LB, true>;
+    }
     switch (vper) {
     case 0: return k_ensemble_mixed<VM, EM, METHOD, LB>;
     case 1: return k_ensemble<VM, EM, METHOD, 1, LB>;
@@ -976,27 +980,27 @@ EnsKernel pick_vper(int vper) {
 // VGPRs each) take one or two vertices per thread.  small: at most 256 threads, and few edges per
 // thread in a quarter of the instances or more
 template <int VM, int EM, int METHOD>
-EnsKernel pick_v(int vper, int threads, bool small) {
+EnsKernel pick_v(int vper, int threads, bool small, bool dense) {
     if (threads > 512) return vper == 1 ? k_ensemble<VM, EM, METHOD, 1, 1024> : k_ensemble<VM, EM, METHOD, 2, 1024>;
-    return small ? pick_vper<VM, EM, METHOD, 256>(vper) : pick_vper<VM, EM, METHOD, 512>(vper);
+    return small ? pick_vper<VM, EM, METHOD, 256>(vper, dense) : pick_vper<VM, EM, METHOD, 512>(vper, dense);
 }
 
 // kernel method: 0 Tsit5, 1 RK4, 2 Tsit5 with line crossings located on the dense output
 template <int VM, int EM>
-EnsKernel pick_m(int kmethod, int vper, int threads, bool small) {
+EnsKernel pick_m(int kmethod, int vper, int threads, bool small, bool dense) {
     switch (kmethod) {
-    case 1: return pick_v<VM, EM, 1>(vper, threads, small);
-    case 2: return pick_v<VM, EM, 2>(vper, threads, small);
-    default: return pick_v<VM, EM, 0>(vper, threads, small);
+    case 1: return pick_v<VM, EM, 1>(vper, threads, small, dense);
+    case 2: return pick_v<VM, EM, 2>(vper, threads, small, dense);
+    default: return pick_v<VM, EM, 0>(vper, threads, small, dense);
     }
 }
 
-EnsKernel pick_ensemble(int vm, int em, int kmethod, int vper, int threads, bool small) {
-    if (vm == ND_VM_SWING && em == ND_EM_KURAMOTO) return pick_m<ND_VM_SWING, ND_EM_KURAMOTO>(kmethod, vper, threads, small);
-    if (vm == ND_VM_SWING && em == ND_EM_STATIC_LINE) return pick_m<ND_VM_SWING, ND_EM_STATIC_LINE>(kmethod, vper, threads, small);
-    if (vm == ND_VM_KURAMOTO && em == ND_EM_KURAMOTO) return pick_m<ND_VM_KURAMOTO, ND_EM_KURAMOTO>(kmethod, vper, threads, small);
+EnsKernel pick_ensemble(int vm, int em, int kmethod, int vper, int threads, bool small, bool dense) {
+    if (vm == ND_VM_SWING && em == ND_EM_KURAMOTO) return pick_m<ND_VM_SWING, ND_EM_KURAMOTO>(kmethod, vper, threads, small, dense);
+    if (vm == ND_VM_SWING && em == ND_EM_STATIC_LINE) return pick_m<ND_VM_SWING, ND_EM_STATIC_LINE>(kmethod, vper, threads, small, dense);
+    if (vm == ND_VM_KURAMOTO && em == ND_EM_KURAMOTO) return pick_m<ND_VM_KURAMOTO, ND_EM_KURAMOTO>(kmethod, vper, threads, small, dense);
     if (vm == ND_VM_KURAMOTO && em == ND_EM_STATIC_LINE)
-        return pick_m<ND_VM_KURAMOTO, ND_EM_STATIC_LINE>(kmethod, vper, threads, small);
+        return pick_m<ND_VM_KURAMOTO, ND_EM_STATIC_LINE>(kmethod, vper, threads, small, dense);
     return nullptr;
 }
 
@@ -1026,6 +1030,7 @@ int hip_err(hipError_t e, const char* what) {
 struct nd_ensemble {
     int device = 0;
     int lds_max = 0;                                // dynamic LDS a workgroup may take
+    int cus = 0;                                    // of the device
     int32_t ninst = 0;
     nd_kind vk{}, ek{};
     int32_t dim = 0;
@@ -1189,6 +1194,13 @@ int32_t class_limit(const nd_ensemble* en, int c, int kmethod) {
     return lim;
 }
 
+// RK4 at one and two vertices per thread comes within 128 registers with its addresses recomputed,
+// which costs 5 % where the instances are on the chip at once (168 registers, twelve waves a CU)
+// and gains where they are not.  us for 1024 swing networks, 168 / 128 registers: 128 vertices (128
+// threads) 704 / 741, 300 (256 threads) 1493 / 1219, 700 (512 threads) 3447 / 2490; 4096 of 20 to 250
+// vertices 2134 / 2014; one of 1000 792 / 850.
+constexpr int kSparseWaves = 12;
+
 // The launches of a solve, largest instances first.  Neighbouring classes of one thread
 // count share a launch: at 512 threads a CU holds one workgroup of most kernels whatever its
 // vertices per thread, and one list of instances by decreasing size ends more evenly than several
@@ -1219,7 +1231,8 @@ int launches(const nd_ensemble* en, int kmethod, Launch* out) {
         int32_t few = 0;
         for (int32_t q = l.first; q < l.first + l.count; ++q) few += en->inst[en->order[q]].ne <= 2 * threads;
         const bool small = threads <= 256 && 4 * few > l.count;
-        l.kernel = pick_ensemble(en->vk.model, en->ek.model, kmethod, vper, threads, small);
+        l.kernel = pick_ensemble(en->vk.model, en->ek.model, kmethod, vper, threads, small,
+                                 l.count > en->cus * std::max(1, kSparseWaves * kWave / threads));
         out[n++] = l;
     }
     return n;
@@ -1307,6 +1320,8 @@ int nd_ensemble_create(int32_t ninst, const int64_t* nv, const int64_t* ne, cons
     if (hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, en->device) != hipSuccess || lds_max <= 0)
         lds_max = 64 * 1024;
     en->lds_max = lds_max;
+    if (hipDeviceGetAttribute(&en->cus, hipDeviceAttributeMultiprocessorCount, en->device) != hipSuccess || en->cus <= 0)
+        en->cus = 256;
     en->ninst = ninst;
     en->vk = *vkind;
     en->ek = *ekind;
