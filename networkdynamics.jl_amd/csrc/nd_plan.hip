@@ -17,8 +17,9 @@
 // Segments longer than hub_degree ("hubs") are reduced by one 64-lane wave:
 // lane-strided partial sums, then a fixed xor-butterfly, so results are
 // reproducible run to run (a deterministic tree order instead of the
-// sequential one).  Edges with their own state (ODE edges) get a separate
-// per-edge kernel for du_e.
+// sequential one).  Edges with their own state (ODE edges) get their du_e in the
+// vertices' launch where the network has one batch of them, in a per-edge kernel
+// otherwise.
 //
 // Generic device primitives mirror the reference's internal dispatch points
 // for any output depth: gather! (gbufs.jl:25), aggregate! (aggregators.jl:140)
@@ -716,7 +717,8 @@ __device__ __forceinline__ Dual slot_value_dual_rt(const EDesc& e, int2 s, Dual 
     return g_dst_rt<Dual>(e.model, nbr, own, pe);
 }
 
-// batches whose f does nothing in networks of the generic kernels
+// batches of the generic kernels whose model has no f there (truss nodes declared with one
+// output component, which the right-hand side leaves at zero as well)
 __global__ void __launch_bounds__(256) k_vertex_noop_jvp(VDesc vd, const int32_t* __restrict__, const int2* __restrict__,
                                                          const uint8_t* __restrict__, const EDesc* __restrict__,
                                                          const double* __restrict__, const double* __restrict__,
@@ -860,12 +862,6 @@ __device__ __forceinline__ DualK<K> slot_value_k_rt(const EDesc& e, int2 s, cons
     return g_dst_rt<DualK<K>>(e.model, nbr, own, pe);
 }
 
-// order between LDS writes and reads of lanes of one wave
-__device__ __forceinline__ void wave_order() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 // Entry E of every 8 lanes (its neighbour in lane E's nbr): lane j fetches tangent j
 template <int E>
 __device__ __forceinline__ void jvp_rows(int32_t nbr, int t, const double* __restrict__ dvt, double* buf) {
@@ -1041,9 +1037,9 @@ __global__ void __launch_bounds__(256) k_vertex_jvp(JvpGroup g, const int32_t* _
             DualK<K> nbr;
             if (K == kJvpWide && !MULTI && !is_ode_model(EM) && a.dvt) {
                 // the 8 lanes of a group read one entry's row of tangents at a time, and turn them in LDS
-                wave_order();
+                wave_sync();
                 jvp_rows<0>(sl.x, t, a.dvt, buf);
-                wave_order();
+                wave_sync();
                 nbr.v = a.vo[sl.x];
 #pragma unroll
                 for (int j = 0; j < K; ++j) nbr.d[j] = to[1 + j];
@@ -1059,7 +1055,7 @@ __global__ void __launch_bounds__(256) k_vertex_jvp(JvpGroup g, const int32_t* _
                 for (int j = 0; j < K; ++j) to[1 + j] = y.d[j];
             }
             if (hub) __syncthreads();
-            else wave_order();
+            else wave_sync();
             if (lane < K) {
                 const double* from = buf + base * (K + 1);
                 for (int e0 = 0; e0 < count; e0 += 8) {
@@ -1075,7 +1071,7 @@ __global__ void __launch_bounds__(256) k_vertex_jvp(JvpGroup g, const int32_t* _
                 }
             }
             if (hub) __syncthreads();
-            else wave_order();
+            else wave_sync();
         }
     }
     if (lane >= a.k) return;
