@@ -992,10 +992,11 @@ extern "C" {
 int64_t nd_mp_param_count(int32_t nfeat) { return offsets(nfeat).total; }
 
 int64_t nd_mp_workspace_floats(int64_t nnodes) {
-    // per node: activations H0..H4 (5*64), the column sums' partials (128), two gradients in
-    // turn and A^T g (3*64 of 4*64 + 1); then the partial sums
+    // per node: activations H0..H4 (5*64), two gradients in turn and A^T g (3*64); then the
+    // column sums' partials (64 per workgroup) and the other partial sums (at most 128 * 64 for
+    // every 64 nodes).  Every array starts at a multiple of 64 floats.
     const int64_t nb = std::min<int64_t>(kMaxPartBlocks, (nnodes + 63) / 64);
-    return nnodes * (5 * kH + 2 * kH + kH + 2 * kH + kH + 1) + (nb + 2) * (kH * 2 * kH) + nnodes / 4 + 8;
+    return nnodes * (8 * kH) + kWgradBlocks * kH + (nb + 2) * (kH * 2 * kH);
 }
 
 int nd_mp_forward(int64_t n, const int32_t* rowptr, const int32_t* nbr, const float* a_fwd, const float* X, int32_t nfeat,
@@ -1037,11 +1038,11 @@ int nd_mp_backward(int64_t n, const int32_t* rowptr, const int32_t* nbr, const f
     hipStream_t s = static_cast<hipStream_t>(stream);
     const Offsets o = offsets(nfeat);
     float* H = work;
-    float* G = work + 5 * n * kH + n * 2 * kH;   // gradients at the layers' sums, in turn: n x 64 each
+    float* G = work + 5 * n * kH;                 // gradients at the layers' sums, in turn: n x 64 each
     float* G2 = G + n * kH;
     float* Z = G2 + n * kH;                       // A^T g: n x 64
-    float* part = G + n * (kH + 2 * kH + kH + 1); // partials
-    float* bpart = work + 5 * n * kH;             // column-sum partials
+    float* bpart = Z + n * kH;                    // column-sum partials
+    float* part = bpart + kWgradBlocks * kH;      // partials
     const LayerShape sh = layer_shape(n);
     const auto layer_bwd = sh.wide ? k_layer_bwd<1024, true> : sh.threads == 1024 ? k_layer_bwd<1024, false>
                                                            : sh.threads == 512    ? k_layer_bwd<512, false> : k_layer_bwd<256, false>;
