@@ -2161,7 +2161,11 @@ void release(nd_plan* pl, void* ptr) {
 }
 
 // Entries per wave of the low path: one window of 4*64, fewer where that would leave the
-// network with less than kLowWaves waves (two per SIMD)
+// network with less than kLowWaves waves (two per SIMD).  us per RK4 stage with 512 / 1024 /
+// 2048 / 4096 / 8192: Barabasi-Albert, 4 lines a vertex, 10000 vertices 5.8 / 5.3 / 5.3 / 5.3 /
+// 5.3, 30000 6.6 / 6.1 / 5.5 / 5.5 / 5.5, 60000 7.4 / 7.5 / 7.1 / 6.9 / 6.9, 100000 8.9 / 8.9 /
+// 9.0 / 9.4 / 10.5, 200000 17.6 with all but 17.3 with 8192; Watts-Strogatz, 4 a vertex, 100000
+// 5.6 / 5.6 / 5.6 / 6.4 / 7.5.  Geometric graphs lie between.
 constexpr int64_t kLowWaves = 2048;
 int32_t wave_entries(int64_t nlow) {
     const int64_t c = (nlow / kLowWaves + kWave - 1) / kWave * kWave;
