@@ -15,7 +15,7 @@
 // (first-order Kuramoto, RK4, 16 waves of one CU) takes 2.47 us per evaluation with the vector
 // units 67 % busy and the LDS 60 %; with an index list per row entry, a bound on every entry
 // and the longer sine it took 3.61 us.  1024 swing networks of 100 to 2000 vertices (Tsit5 to
-// t = 10, default classes) take 39.7 ms, against 66.7 ms; at four vertices per thread the
+// t = 10, default classes) take 39.1 ms, against 66.7 ms; at four vertices per thread the
 // vector units are 60 % busy with two waves per SIMD.
 //
 // Methods: Tsit5 (Tsitouras 2011) with the PI step-size controller of
@@ -569,9 +569,9 @@ __device__ __forceinline__ void ensemble_body(const SolveArgs& a, int inst, cons
     const double inv_len = 1.0 / (static_cast<double>(I.n) * D);
 
     // The right-hand side appears once in each method below, inside one loop over the
-    // evaluations: with a copy per stage the Tsit5 loop's code exceeded the instruction cache
-    // and its constants the scalar registers.  (A kernel of 9 copies: about 100 KB of code and
-    // 230 spilled scalar registers, reloaded lane by lane inside the edge loops.)
+    // evaluations: with a copy per stage the Tsit5 loop's code, about 100 KB of nine copies,
+    // exceeded the instruction cache.  (It saves no scalar registers: the Tsit5 kernels spill 147
+    // to 199 of them, 67 to 104 with the copies.)
 #define ND_EACH                                        \
     _Pragma("unroll") for (int q = 0; q < V; ++q)      \
         _Pragma("unroll") for (int j = 0; j < D; ++j)

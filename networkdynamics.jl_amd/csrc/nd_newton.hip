@@ -15,7 +15,7 @@
 // slices of 64, column by column: entry j of the slice's 64 rows is one contiguous column of
 // 64, padded to the slice's longest row (a few per cent after the sort).  Every read of a
 // column is one contiguous access of its wave, and all columns' reads are independent.  Rows that
-// would widen their slice for the other 63 (hubs; long_rows chooses) are stored apart, entries
+// would widen their slice for the other 63 (hubs; long_row_count chooses) are stored apart, entries
 // 64 j .. 64 j + 63 in one column, and a whole wave evaluates them, adding in order.
 //
 // Who does what: thread t sums the rows at positions t, t + 512, ... of that order and hands
