@@ -216,7 +216,7 @@ end
 
 # Chunked duals, N = 2..8 partials (ForwardDiff's chunk, the size the reference gives its
 # DiffCache buffers, src/construction.jl:205-208): the value and the N partial columns go
-# to nd_rhs_jvp_multi in one launch.  Networks on the library's generic kernels have no
+# to nd_rhs_jvp_multi_work in one call.  Networks on the library's generic kernels have no
 # K-partial form there (ND_ERR_UNSUPPORTED): they take one nd_rhs_jvp per partial.
 function (nw::Network{<:HIPExecution})(du::ROCVector{Dual{T,Float64,N}}, u::ROCVector{Dual{T,Float64,N}},
                                        p::ROCVector{Float64}, t) where {T,N}
@@ -228,11 +228,14 @@ function (nw::Network{<:HIPExecution})(du::ROCVector{Dual{T,Float64,N}}, u::ROCV
     uval = um[1, :]
     upart = permutedims(um[2:end, :])                  # n x N: partial j contiguous, column j
     dval, dpart = similar(uval), similar(upart)
-    rc = ccall((:nd_rhs_jvp_multi, libnd), Cint,
+    # scratch where the plan gathers the partials faster from a copy in it (0: none)
+    nwork = ccall((:nd_rhs_jvp_multi_scratch, libnd), Int64, (Ptr{Cvoid}, Int32), a.plan, Int32(N))
+    work = ROCVector{Float64}(undef, max(nwork, 0))
+    rc = GC.@preserve work ccall((:nd_rhs_jvp_multi_work, libnd), Cint,
                (Ptr{Cvoid}, Ptr{Float64}, Ptr{Float64}, Ptr{Float64}, Ptr{Float64}, Int32, Ptr{Float64}, Float64,
-                Int64, Int64, Int64, Ptr{Cvoid}),
+                Ptr{Float64}, Int64, Int64, Int64, Int64, Ptr{Cvoid}),
                a.plan, pointer(dval), pointer(dpart), pointer(uval), pointer(upart), Int32(N), pointer(p), Float64(t),
-               n, n, length(p), AMDGPU.stream().stream)
+               nwork > 0 ? pointer(work) : Ptr{Float64}(C_NULL), length(work), n, n, length(p), AMDGPU.stream().stream)
     if rc == 2                                          # ND_ERR_UNSUPPORTED
         for j in 1:N
             off = (j - 1) * n + 1
